@@ -10,6 +10,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "mdgfx950.h"
 #include "runtime.h"
@@ -20,7 +21,8 @@ namespace {
 
 constexpr int BLOCK     = 256;
 constexpr int MAXTYPES2 = 64;  // ntypes <= 8
-constexpr int FAST_LPA  = 4;   // lanes per atom in the fast force kernels
+constexpr int FUSE_GHOSTS_EAM = 300000;  // EAM systems up to this size move ghosts in the force call
+constexpr int FAST_LPA  = 4;   // lanes per atom in the fast force kernels of large systems
 
 struct Grid {
     double off[3];     // pad * binsize + 1e-9 (coord2bin, neighbor.c:386-400)
@@ -75,6 +77,10 @@ struct State {
     size_t cap_gcnt = 0, cap_goff = 0;
     int* d_pbc = nullptr;
     size_t cap_pbc = 0;
+    // locals and ghosts of the last setupPbcGFX950, which d_gcnt, d_goff and d_pbc describe
+    // (-1: none)
+    int gmap_nlocal = -1, gmap_nghost = -1;
+    bool ghosts_current = false;  // the last fused force call also wrote the ghosts' positions
     // neighbour list capacity (elements)
     size_t cap_nb = 0, cap_numneigh = 0;
     // EAM
@@ -425,25 +431,64 @@ __global__ void __launch_bounds__(BLOCK) k_build_neighbor(int nlocal, const doub
 // an atom's total force also applies finalIntegrate (integrate.c:61-86) and the next step's
 // initialIntegrate (integrate.c:29-59) with it, the same FP64 operations in the same order as
 // k_final_integrate then k_initial_integrate, and writes the new position to xn.
-struct Fuse {
+// With gcnt set (the ghosts of setupPbcGFX950: atom i's images are goff[i] .. goff[i] + gcnt[i])
+// the atom's lanes also write its images' new positions, as k_update_pbc does afterwards: a step
+// is then one launch instead of two (the ghost update is 3.8 us of a 256-atom step and 5.2 us of
+// a 1M-atom one, nearly all of it the launch).
+struct Fuse0 {
     double* v;
     double* xn;
     double dt, dtforce;
 };
+struct Fuse : Fuse0 {
+    const int* gcnt;
+    const int* goff;
+    const int* pbc;
+    double prd[3];
+};
+
+template <bool GH>
+using FuseOf = std::conditional_t<GH, Fuse, Fuse0>;
 
 // v0 (loaded at the kernel's start, so its latency hides behind the neighbour loop) and x0 are
-// the atom's velocity and position.
-__device__ inline void fused_integrate(const Fuse& fu, int i, const double* v0, const double* x0,
-    double fx, double fy, double fz)
+// the atom's velocity and position, fx, fy, fz its total force: the same in all of its LPA lanes.
+template <int LPA, bool GH>
+__device__ inline void fused_integrate(const FuseOf<GH>& fu, int nlocal, int i, int lane,
+    const double* v0, const double* x0, int ng, int g0, double fx, double fy, double fz)
 {
     const double fr[3] = { fx, fy, fz };
+    double xn[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        double vv         = v0[d] + fu.dtforce * fr[d];
-        vv                = vv + fu.dtforce * fr[d];
-        fu.v[3 * i + d]   = vv;
-        fu.xn[3 * i + d]  = x0[d] + fu.dt * vv;
+        double vv = v0[d] + fu.dtforce * fr[d];
+        vv        = vv + fu.dtforce * fr[d];
+        xn[d]     = x0[d] + fu.dt * vv;
+        if (lane == 0) {
+            fu.v[3 * i + d]  = vv;
+            fu.xn[3 * i + d] = xn[d];
+        }
     }
+    if constexpr (GH)
+        for (int k = lane; k < ng; k += LPA) {
+            const int g = g0 + k;
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+                fu.xn[3 * (nlocal + g) + d] = xn[d] + fu.pbc[3 * g + d] * fu.prd[d];
+        }
+}
+
+// What fused_integrate needs of atom i, loaded ahead of the neighbour loop.
+template <bool GH>
+__device__ inline void fused_load(const FuseOf<GH>& fu, int i, double* v0, int* ng, int* g0)
+{
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+        v0[d] = fu.v[3 * i + d];
+    if constexpr (GH)
+        if (fu.gcnt) {
+            *ng = fu.gcnt[i];
+            *g0 = fu.goff[i];
+        }
 }
 
 // ---------------------------------------------------------------- LJ (force_lj.c:17-206)
@@ -456,30 +501,31 @@ __global__ void __launch_bounds__(BLOCK) k_force_lj(int nlocal, const double* __
 {
     __shared__ double s_tab[3][MAXTYPES2];
     __shared__ double s_red[16];
-    const int nt2 = ntypes * ntypes;
-    for (int k = threadIdx.x; k < nt2; k += blockDim.x) {
-        s_tab[0][k] = tab.eps[k];
-        s_tab[1][k] = tab.sig6[k];
-        s_tab[2][k] = tab.cutf[k];
+    if (!uniform) {
+        const int nt2 = ntypes * ntypes;
+        for (int k = threadIdx.x; k < nt2; k += blockDim.x) {
+            s_tab[0][k] = tab.eps[k];
+            s_tab[1][k] = tab.sig6[k];
+            s_tab[2][k] = tab.cutf[k];
+        }
+        __syncthreads();
     }
-    __syncthreads();
     const int gid  = blockIdx.x * blockDim.x + threadIdx.x;
     const int i    = gid / LPA;
     const int lane = gid % LPA;
     const bool act = i < nlocal;
     double fix = 0, fiy = 0, fiz = 0, e = 0, w = 0;
     double v0[3] = {}, x0[3] = {};
-    if (!HALF && fu.v && act && lane == 0)
-        for (int d = 0; d < 3; d++)
-            v0[d] = fu.v[3 * i + d];
+    int ng = 0, g0 = 0;
+    if (!HALF && fu.v && act && (lane == 0 || fu.gcnt)) fused_load<true>(fu, i, v0, &ng, &g0);
     if (act) {
         const double xt = x[3 * i], yt = x[3 * i + 1], zt = x[3 * i + 2];
         x0[0] = xt;
         x0[1] = yt;
         x0[2] = zt;
-        const int ti    = type[i];
+        const int ti    = uniform ? 0 : type[i];
         const int nn    = numneigh[i];
-        double eps0 = s_tab[0][0], sig0 = s_tab[1][0], cut0 = s_tab[2][0];
+        const double eps0 = tab.eps[0], sig0 = tab.sig6[0], cut0 = tab.cutf[0];
         for (int k = lane; k < nn; k += LPA) {
             const int j = neighbors[(size_t)k * nlocal + i];
             double dx   = xt - x[3 * j];
@@ -535,9 +581,10 @@ __global__ void __launch_bounds__(BLOCK) k_force_lj(int nlocal, const double* __
             f[3 * i]     = fix;
             f[3 * i + 1] = fiy;
             f[3 * i + 2] = fiz;
-            if (fu.v) fused_integrate(fu, i, v0, x0, fix, fiy, fiz);
         }
     }
+    if (!HALF && fu.v && act && (lane == 0 || fu.gcnt))
+        fused_integrate<LPA, true>(fu, nlocal, i, lane, v0, x0, ng, g0, fix, fiy, fiz);
     if (EV) {
         double be = block_sum(e, s_red);
         double bw = block_sum(w, s_red);
@@ -653,9 +700,8 @@ __global__ void __launch_bounds__(BLOCK) k_eam_force(int nlocal, const double* _
     const bool act = i < nlocal;
     double fix = 0, fiy = 0, fiz = 0, e = 0, w = 0;
     double v0[3] = {}, x0[3] = {};
-    if (fu.v && act && lane == 0)
-        for (int d = 0; d < 3; d++)
-            v0[d] = fu.v[3 * i + d];
+    int ng = 0, g0 = 0;
+    if (fu.v && act && (lane == 0 || fu.gcnt)) fused_load<true>(fu, i, v0, &ng, &g0);
     if (act) {
         const double xt = x[3 * i], yt = x[3 * i + 1], zt = x[3 * i + 2];
         x0[0] = xt;
@@ -702,8 +748,9 @@ __global__ void __launch_bounds__(BLOCK) k_eam_force(int nlocal, const double* _
         f[3 * i + 1] = fiy;
         f[3 * i + 2] = fiz;
         if (EV && eatom) eatom[i] += ea;
-        if (fu.v) fused_integrate(fu, i, v0, x0, fix, fiy, fiz);
     }
+    if (fu.v && act && (lane == 0 || fu.gcnt))
+        fused_integrate<LPA, true>(fu, nlocal, i, lane, v0, x0, ng, g0, fix, fiy, fiz);
     if (EV) {
         double be = block_sum(e, s_red);
         double bw = block_sum(w, s_red);
@@ -773,12 +820,14 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_density_tab(int nlocal, int p
     }
 }
 
-template <int LPA, bool STRICT>
+// GH: with the ghosts' positions (a variant of its own: in one kernel with the other, the large
+// systems' passes, which do not write them, ran 1 % slower).
+template <int LPA, bool STRICT, bool GH>
 __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per_block,
     const double* __restrict__ x, const int* __restrict__ neighbors,
     const int* __restrict__ numneigh, double cutforcesq, const double* __restrict__ rs,
     const double* __restrict__ zs, int nr, double rdr, const double* __restrict__ fp,
-    double* __restrict__ f, Fuse fu)
+    double* __restrict__ f, FuseOf<GH> fu)
 {
     __shared__ double s_t[TAB_NR * 10];  // per row: rho c0..c2, then z2r c0..c6
     for (int k = threadIdx.x; k < nr * 10; k += TAB_BLOCK) {
@@ -796,9 +845,8 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per
         const bool act = i < end;
         double fix = 0, fiy = 0, fiz = 0;
         double v0[3] = {}, x0[3] = {};
-        if (fu.v && act && lane == 0)
-            for (int d = 0; d < 3; d++)
-                v0[d] = fu.v[3 * i + d];
+        int ng = 0, g0 = 0;
+        if (fu.v && act && (lane == 0 || GH)) fused_load<GH>(fu, i, v0, &ng, &g0);
         if (act) {
             const double xt = x[3 * i], yt = x[3 * i + 1], zt = x[3 * i + 2];
             x0[0]            = xt;
@@ -839,8 +887,9 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per
             f[3 * i]     = fix;
             f[3 * i + 1] = fiy;
             f[3 * i + 2] = fiz;
-            if (fu.v) fused_integrate(fu, i, v0, x0, fix, fiy, fiz);
         }
+        if (fu.v && act && (lane == 0 || GH))
+            fused_integrate<LPA, GH>(fu, nlocal, i, lane, v0, x0, ng, g0, fix, fiy, fiz);
     }
 }
 
@@ -965,6 +1014,7 @@ void initDeviceGFX950(Parameter* param, Atom* atom, Neighbor* neighbor)
     grow_n(&dn->numneigh, &S.cap_numneigh, (size_t)atom->Nlocal, 0);
     S.binned = false;
     S.ready  = true;
+    S.gmap_nlocal = -1;
     copyDataToGFX950Device(param, atom);
 }
 
@@ -1042,6 +1092,7 @@ void copyDataToGFX950Device(Parameter* param, Atom* atom)
 {
     (void)param;
     if (failed() || !S.ready) return;
+    S.ghosts_current = false;
     size_t nall = (size_t)atom->Nlocal + atom->Nghost;
     DeviceAtom* d = &atom->d_atom;
     MDG_HIP(hipMemcpyAsync(d->x, atom->x, 3 * nall * sizeof(double), hipMemcpyHostToDevice, stream()));
@@ -1191,6 +1242,8 @@ void sortAtomGFX950(Atom* atom)
     if (failed() || !S.ready) return;
     const int n  = atom->Nlocal;
     atom->Nghost = 0;
+    S.gmap_nlocal    = -1;
+    S.ghosts_current = false;
     if (n <= 0) return;
     fill_i32(S.d_status, 0, 2);
     binatomsGFX950(atom);
@@ -1257,6 +1310,8 @@ void setupPbcGFX950(Atom* atom, Parameter* param)
     if (failed() || !S.ready) return;
     TimedRegion tr(F_PBC);
     const int nlocal = atom->Nlocal;
+    S.gmap_nlocal    = -1;
+    S.ghosts_current = false;
     Prd prd{ { param->xprd, param->yprd, param->zprd } };
     grow_n(&S.d_gcnt, &S.cap_gcnt, (size_t)nlocal + 1, 0);
     grow_n(&S.d_goff, &S.cap_goff, (size_t)nlocal + 1, 0);
@@ -1291,7 +1346,9 @@ void setupPbcGFX950(Atom* atom, Parameter* param)
     k_ghost_fill<<<blocks_for(nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x, prd,
         param->cutneigh, S.d_goff, atom->d_atom.border_map, S.d_pbc, atom->d_atom.type);
     MDG_LAUNCH_CHECK("ghost_fill");
-    atom->Nghost = nghost;
+    atom->Nghost  = nghost;
+    S.gmap_nlocal = nlocal;
+    S.gmap_nghost = nghost;
 }
 
 void updatePbcGFX950(Atom* atom, Parameter* param, bool doReneighbor)
@@ -1309,10 +1366,33 @@ void updateAtomsPbcGFX950(Atom* atom, Parameter* param, bool doReneighbor)
 {
     (void)doReneighbor;
     if (failed() || !S.ready) return;
+    S.ghosts_current = false;
     TimedRegion tr(F_PBC);
     k_wrap<<<blocks_for(3LL * atom->Nlocal, BLOCK), BLOCK, 0, stream()>>>(3 * atom->Nlocal,
         atom->d_atom.x, param->xprd, param->yprd, param->zprd);
     MDG_LAUNCH_CHECK("wrap");
+}
+
+// Lanes per atom of the fast full-list LJ kernel without energies.  A small system leaves the chip
+// idle and waits on the chain of loads along each lane's share of the list, so its lists go to more
+// lanes; a large one fills the chip with 4, and more lanes only make the list rows' loads narrower.
+// us per step (force, integration and ghosts in one launch, 76 listed neighbours) with
+//     atoms     4     8    16    32    64 lanes
+//       256  13.2   8.9   6.2   5.3   4.7
+//      2048  14.4   8.6   6.3   5.3   5.3
+//      6912  13.8   8.7   7.0   7.2   8.5
+//     16384  14.3  10.2   8.9  10.9  17.2
+//     32000  16.9  11.8  14.4  19.4  29.0
+//     55296  19.5  16.3  22.8  30.0  45.7
+//    131072  28.5  35.1  49.1  67.2 102.7
+// (before: 4 lanes and a ghost update of 3.8 us a step at every size).
+static int lanes_per_atom(int nlocal)
+{
+    return nlocal <= 1500    ? 64
+           : nlocal <= 5000  ? 32
+           : nlocal <= 24000 ? 16
+           : nlocal <= 80000 ? 8
+                             : FAST_LPA;
 }
 
 static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu)
@@ -1323,8 +1403,6 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
     const int nlocal = atom->Nlocal;
     const int nall   = nlocal + atom->Nghost;
     const bool strict = strict_mode();
-    const int lpa    = strict ? 1 : FAST_LPA;
-    unsigned grid    = blocks_for((long long)nlocal * lpa, BLOCK);
     hipStream_t s    = stream();
     if (S.ev_on) fill_f64(S.d_ev, 0.0, 2);
     const int half = neighbor->half_neigh;
@@ -1332,7 +1410,7 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
     {
         TimedRegion tr(F_FORCE_LJ);
 #define MDG_LJ(L, ST, H, E)                                                                      \
-    k_force_lj<L, ST, H, E><<<grid, BLOCK, 0, s>>>(nlocal, atom->d_atom.x, atom->d_atom.type,    \
+    k_force_lj<L, ST, H, E><<<blocks_for((long long)nlocal * L, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x, atom->d_atom.type,    \
         S.ntypes, S.tab, S.uniform ? 1 : 0, neighbor->d_neighbor.neighbors,                      \
         neighbor->d_neighbor.numneigh, atom->d_atom.fx, S.d_ev, fu)
         if (strict) {
@@ -1347,8 +1425,14 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
             if (half) {
                 if (S.ev_on) MDG_LJ(FAST_LPA, false, true, true);
                 else MDG_LJ(FAST_LPA, false, true, false);
+            } else if (S.ev_on) {
+                MDG_LJ(FAST_LPA, false, false, true);
             } else {
-                if (S.ev_on) MDG_LJ(FAST_LPA, false, false, true);
+                const int lanes = lanes_per_atom(nlocal);
+                if (lanes == 64) MDG_LJ(64, false, false, false);
+                else if (lanes == 32) MDG_LJ(32, false, false, false);
+                else if (lanes == 16) MDG_LJ(16, false, false, false);
+                else if (lanes == 8) MDG_LJ(8, false, false, false);
                 else MDG_LJ(FAST_LPA, false, false, false);
             }
         }
@@ -1361,7 +1445,7 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
 double computeForceLJGFX950(Parameter* param, Atom* atom, Neighbor* neighbor, Stats* stats)
 {
     (void)stats;
-    return force_lj(param, atom, neighbor, Fuse{ nullptr, nullptr, 0.0, 0.0 });
+    return force_lj(param, atom, neighbor, Fuse{});
 }
 
 void setEamTablesGFX950(int nr, int nrho, double rdr, double rdrho, const double* rhor_spline,
@@ -1422,6 +1506,10 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
             S.d_z2r, S.nr, S.rdr, S.d_fp, atom->d_atom.fx, S.d_ev, eatom, fu);                   \
     } while (0)
     // without the energy and for tables of up to TAB_NR rows: the LDS-table passes
+#define MDG_EAM_FT(L, ST, G)                                                                     \
+    k_eam_force_tab<L, ST, G><<<gf, TAB_BLOCK, 0, s>>>(nlocal, pf, atom->d_atom.x,               \
+        neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, cutf, S.d_rhor, S.d_z2r,  \
+        S.nr, S.rdr, S.d_fp, atom->d_atom.fx, fu)
 #define MDG_EAM_TAB(L, ST)                                                                       \
     do {                                                                                         \
         const unsigned gd = 2u * (unsigned)S.ncu, gf = (unsigned)S.ncu;                          \
@@ -1430,9 +1518,8 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
             neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, cutf, S.d_rhor,       \
             S.d_frho, S.nr, S.nrho, S.rdr, S.rdrho, S.d_fp);                                     \
         launch_ghost_copy(S.d_fp, atom);                                                         \
-        k_eam_force_tab<L, ST><<<gf, TAB_BLOCK, 0, s>>>(nlocal, pf, atom->d_atom.x,              \
-            neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, cutf, S.d_rhor,       \
-            S.d_z2r, S.nr, S.rdr, S.d_fp, atom->d_atom.fx, fu);                                  \
+        if (fu.gcnt) MDG_EAM_FT(L, ST, true);                                                    \
+        else MDG_EAM_FT(L, ST, false);                                                           \
     } while (0)
     const bool tab = !ev && S.nr <= TAB_NR && S.ncu > 0 && nlocal > 0;
     if (strict) {
@@ -1445,6 +1532,7 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
         else MDG_EAM(FAST_LPA, false, false);
     }
 #undef MDG_EAM_TAB
+#undef MDG_EAM_FT
 #undef MDG_EAM
     MDG_LAUNCH_CHECK("force_eam");
     return wtime() - t0;
@@ -1453,7 +1541,7 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
 double computeForceEamGFX950(Parameter* param, Atom* atom, Neighbor* neighbor, Stats* stats)
 {
     (void)stats;
-    return force_eam(param, atom, neighbor, Fuse{ nullptr, nullptr, 0.0, 0.0 });
+    return force_eam(param, atom, neighbor, Fuse{});
 }
 
 double computeForceFinalInitialGFX950(Parameter* param, Atom* atom, Neighbor* neighbor,
@@ -1471,13 +1559,30 @@ double computeForceFinalInitialGFX950(Parameter* param, Atom* atom, Neighbor* ne
     }
     grow_n(&S.d_xn, &S.cap_xn, 3 * S.cap_all, 0);
     if (failed()) return 0.0;
-    const Fuse fu{ atom->d_atom.vx, S.d_xn, param->dt, param->dtforce };
+    Fuse fu{ { atom->d_atom.vx, S.d_xn, param->dt, param->dtforce } };
+    // (not for large EAM systems: the images' writes in the border atoms' tails hold up their
+    // persistent blocks by 15 us a step at 1M atoms, more than the 5 us of the ghost update)
+    const bool ghosts = S.gmap_nlocal == atom->Nlocal && S.gmap_nghost == atom->Nghost &&
+                        !(eam && atom->Nlocal > FUSE_GHOSTS_EAM);
+    if (ghosts) {
+        fu.gcnt   = S.d_gcnt;
+        fu.goff   = S.d_goff;
+        fu.pbc    = S.d_pbc;
+        fu.prd[0] = param->xprd;
+        fu.prd[1] = param->yprd;
+        fu.prd[2] = param->zprd;
+    }
     const double t = eam ? force_eam(param, atom, neighbor, fu) : force_lj(param, atom, neighbor, fu);
-    // the new local positions become the current ones; ghost positions follow at updatePbc
+    // the new local positions become the current ones; ghost positions written too if their map
+    // is known, else they follow at updatePbc
     std::swap(atom->d_atom.x, S.d_xn);
-    S.cap_xn = 3 * S.cap_all;
+    S.cap_xn         = 3 * S.cap_all;
+    S.ghosts_current = ghosts && !failed();
     return t;
 }
+
+// For the run loop: the last call was a fused force call that also moved the ghosts.
+int mdg_vl_ghosts_current(void) { return S.ghosts_current; }
 
 void requestEamAtomEnergyGFX950(int on)
 {
@@ -1501,6 +1606,7 @@ void initialIntegrateGFX950(bool reneigh, Parameter* param, Atom* atom)
 {
     (void)reneigh;
     if (failed() || !S.ready) return;
+    S.ghosts_current = false;
     TimedRegion tr(F_INTEGRATE);
     int n3 = 3 * atom->Nlocal;
     k_initial_integrate<<<blocks_for(n3, BLOCK), BLOCK, 0, stream()>>>(n3, atom->d_atom.x,

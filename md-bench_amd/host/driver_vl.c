@@ -256,7 +256,8 @@ int mdbVLRun(mdb_vl* s, int nsteps, double* ksum)
             setupPbcGFX950(a, p);
             updatePbcGFX950(a, p, true);
             buildNeighborGFX950(a, nb);
-        } else {
+        } else if (!(integrated && mdg_vl_ghosts_current())) {
+            /* (the fused force call wrote the ghosts' positions with the atoms') */
             updatePbcGFX950(a, p, false);
         }
         /* plain LJ/EAM steps carry the next step's initialIntegrate in the force call, unless
