@@ -77,15 +77,15 @@ void updateSingleAtomsGFX950(Parameter* param, Atom* atom);
    computeForceLJ4xn{Full,Half}Neigh (src/clusterpair/force_lj.c): full or half list by
    neighbor->half_neigh, precision by setClusterPrecisionGFX950 */
 double computeForceLJClusterGFX950(Parameter* param, Atom* atom, Neighbor* neighbor, Stats* stats);
-/* computeForce then finalIntegrate (main.c:349-350) in one call: the FP32 full-list kernel
-   applies the final velocity kick to each atom whose total force it has just written (one pass
+/* computeForce then finalIntegrate (main.c:349-350) in one call: the full-list kernels (FP32, and
+   FP64 with i-clusters of four) and the FP32 tiled half-list one apply the final velocity kick to each atom whose total force it has just written (one pass
    fewer over v and f); other configurations run the two calls in order (no reference
    counterpart: a fused form of the two reference calls) */
 double computeForceFinalClusterGFX950(Parameter* param, Atom* atom, Neighbor* neighbor,
     Stats* stats);
 /* computeForce, finalIntegrate and the NEXT step's initialIntegrate (main.c:349-350, 326) in one
-   call: the FP32 full-list kernel kicks each atom twice with the force it has just written and
-   drifts it into a second position buffer, which then becomes the current one; the same FP64
+   call: the same kernels kick each atom twice with the force they have just written and
+   drift it into a second position buffer, which then becomes the current one; the same FP64
    operations in the same order as the three calls, so the trajectory is bit-identical.  The
    velocities it leaves are the next half step's: callers that read full-step velocities after a
    step (thermo, the last step) use computeForceFinalClusterGFX950 there.  Ghost slots keep

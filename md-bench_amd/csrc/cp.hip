@@ -7,9 +7,12 @@
 // per i-cluster, ordered compaction with ballots, masked entries first).
 //
 // Force kernels:
-//   k_cp_force_f64          one thread per i-slot, the reference kernel's arithmetic
-//                           (computeForceLJRef, src/clusterpair/force_lj.c:22-189); full lists
-//                           are bit-identical to it.
+//   k_cp_force_f64_full     FP64, full lists of i-clusters of four: one wavefront per i-cluster,
+//                           16 list entries side by side, the reference kernel's arithmetic and
+//                           order of sums (computeForceLJRef, src/clusterpair/force_lj.c:22-189),
+//                           bit-identical to it; the run loop's kicks and drift fused in.
+//   k_cp_force_f64          the same arithmetic, one thread per i-slot: half lists and 1x2
+//                           clusters.
 //   k_cp_force_f32_full     FP32-mixed, full lists: one wavefront per four i-clusters, one
 //                           j-atom per lane against the group's four i-atoms, j-atoms read as
 //                           16-byte FP32 records (offset in a power-of-two grid cell, cell bytes
@@ -117,6 +120,7 @@ struct CPState {
     double* d_sxn   = nullptr;
     size_t cap_sxn  = 0;
     bool sxn_valid  = false;  // padding, dummy and ghost slots of d_sxn match d_sx
+    bool sxn_recs   = false;  // and those of d_srn match d_sr (FP32 kernels)
     // FP32 j-records of d_sx and d_sxn (make_rec), for the FP32 full-list kernel
     float4 *d_sr = nullptr, *d_srn = nullptr;
     size_t cap_sr = 0, cap_srn = 0;
@@ -1403,6 +1407,128 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64(int nci, int ncj, int nt
         }
     }
     if (EV) ev_store(e, w, ev);
+}
+
+// Full lists of i-clusters of four, the same arithmetic and the same order of sums, bit for bit:
+// per i-atom and list entry the N pair forces in order, then the entries in list order.  One
+// wavefront per i-cluster: lane (e, a) takes i-atom a and entry e of a round of 16, so the pairs
+// of a round run side by side; their sums go to LDS and 12 lanes (atom and axis) add them in list
+// order.  The tail kicks and drifts like k_cp_final and k_cp_initial (v set, xn set), each on the
+// lane that holds the total.
+// One thread per i-slot walking its whole list (k_cp_force_f64, still the half lists' and the
+// 1x2 clusters' kernel) took 148 us for 34,960 atoms of the Kob-Andersen mixture, 547 wavefronts
+// waiting on their lists; this takes 24.6 us, kicks and drift included (9.9 us in launches of
+// their own before).  Bound now: FP64 instructions (the exact division of the pairs inside the
+// cutoff above all).
+template <int N, bool EV, bool UNIFORM>
+__global__ void __launch_bounds__(BLOCK) k_cp_force_f64_full(int nci, int ntypes, Tab64 tab,
+    const double* __restrict__ sx, const int* __restrict__ st, const int* __restrict__ nb,
+    const int* __restrict__ numneigh, const int* __restrict__ ci_natoms, int maxneighs,
+    double* __restrict__ f, double* __restrict__ ev, double* __restrict__ v, double dtforce,
+    double* __restrict__ xn, double dt)
+{
+    constexpr int ROW = 13;  // doubles per entry: 12 sums, one apart so that entries spread
+    __shared__ double s_sum[BLOCK / 64][16 * ROW];
+    __shared__ double s_tab[3][MAXT2];
+    if (!UNIFORM) {
+        for (int k = threadIdx.x; k < ntypes * ntypes; k += BLOCK) {
+            s_tab[0][k] = tab.eps[k];
+            s_tab[1][k] = tab.sig6[k];
+            s_tab[2][k] = tab.cutf[k];
+        }
+        __syncthreads();
+    }
+    // i-clusters of one XCD adjacent (the grid is a multiple of 8 blocks)
+    const int per = gridDim.x >> 3;
+    const int lb  = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    const int w   = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int ci  = __builtin_amdgcn_readfirstlane(lb * (BLOCK / 64) + w);
+    if (ci >= nci) return;
+    const int a = lane & 3, e = lane >> 2, si = ci * 4 + a;
+    const double xt = sx[3 * si], yt = sx[3 * si + 1], zt = sx[3 * si + 2];
+    const int ti   = UNIFORM ? 0 : st[si] * ntypes;
+    const int* lst = nb + (size_t)ci * maxneighs;
+    const int nn   = numneigh[ci];
+    double* sum    = s_sum[w];
+    // the tail's inputs, loaded ahead of the loop
+    const int ta = lane / 3, t3 = 3 * (ci * 4) + lane;
+    const bool tail = lane < 12;
+    double v0 = 0.0, x0 = 0.0;
+    int nat = 0;
+    if (v && tail) {
+        v0  = v[t3];
+        nat = ci_natoms[ci];
+        if (xn) x0 = sx[t3];
+    }
+    double tot = 0.0, ee = 0.0, ww = 0.0;
+    int cj = e < nn ? lst[e] : -1;
+    for (int k0 = 0; k0 < nn; k0 += 16) {
+        const int kn  = k0 + 16 + e;
+        const int cjn = kn < nn ? lst[kn] : -1;
+        double fix = 0.0, fiy = 0.0, fiz = 0.0;
+        if (cj >= 0) {
+            double xj[N][3];
+            int tj[N];
+#pragma unroll
+            for (int b = 0; b < N; b++) {
+                const int sj = cj * N + b;
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+                    xj[b][d] = sx[3 * (size_t)sj + d];
+                tj[b] = UNIFORM ? 0 : st[sj];
+            }
+#pragma unroll
+            for (int b = 0; b < N; b++) {
+                const double dx  = xt - xj[b][0];
+                const double dy  = yt - xj[b][1];
+                const double dz  = zt - xj[b][2];
+                const double rsq = dx * dx + dy * dy + dz * dz;
+                const int tij    = ti + tj[b];
+                const double cut = UNIFORM ? tab.cutf[0] : s_tab[2][tij];
+                if (cj * N + b != si && rsq < cut) {
+                    const double eps   = UNIFORM ? tab.eps[0] : s_tab[0][tij];
+                    const double sig6  = UNIFORM ? tab.sig6[0] : s_tab[1][tij];
+                    const double sr2   = 1.0 / rsq;
+                    const double sr6   = sr2 * sr2 * sr2 * sig6;
+                    const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
+                    fix += dx * force;
+                    fiy += dy * force;
+                    fiz += dz * force;
+                    if (EV) {
+                        ee += 0.5 * 4.0 * eps * sr6 * (sr6 - 1.0);
+                        ww += 0.5 * rsq * force;
+                    }
+                }
+            }
+        }
+        sum[e * ROW + 3 * a]     = fix;
+        sum[e * ROW + 3 * a + 1] = fiy;
+        sum[e * ROW + 3 * a + 2] = fiz;
+        // one wavefront: its LDS operations complete in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (tail)
+#pragma unroll
+            for (int q = 0; q < 16; q++)
+                tot += sum[q * ROW + lane];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        cj = cjn;
+    }
+    if (tail) {
+        f[t3] = tot;
+        if (v && ta < nat) {
+            double vv = v0 + dtforce * tot;
+            if (xn) {
+                vv     = vv + dtforce * tot;
+                xn[t3] = x0 + dt * vv;
+            }
+            v[t3] = vv;
+        }
+    }
+    if (EV) ev_store(ee, ww, ev);
 }
 
 // ---------------------------------------------------------------- FP32-mixed force kernel
@@ -3439,6 +3565,8 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
     const bool tiled = C.precision == 0 && half && !C.comp && C.tiles_ok;
     // the FP32 full-list and tiled half-list kernels read records
     const bool recs = C.precision == 0 && (!half || tiled);
+    // FP64, full lists of i-clusters of four: the wavefront-per-cluster kernel
+    const bool full64 = C.precision == 1 && !half && C.M == 4;
     if (recs) ensure_records();
     if (failed()) return 0;
     // the next step's positions and their records go to the second buffers, whose padding,
@@ -3446,21 +3574,23 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
     // upload)
     double* xn = nullptr;
     float4* rn = nullptr;
-    if (fuse_initial && fuse_final && recs) {
+    if (fuse_initial && fuse_final && (recs || full64)) {
         const size_t nsl = nslots_all(), n3 = 3 * nsl, cap0 = C.cap_sxn, capr0 = C.cap_srn;
         grow_n(&C.d_sxn, &C.cap_sxn, n3, 0);
-        grow_n(&C.d_srn, &C.cap_srn, nsl, 0);
+        if (recs) grow_n(&C.d_srn, &C.cap_srn, nsl, 0);
         if (failed()) return 0;
-        if (C.cap_sxn != cap0 || C.cap_srn != capr0) C.sxn_valid = false;
+        if (C.cap_sxn != cap0 || C.cap_srn != capr0 || C.sxn_recs != recs) C.sxn_valid = false;
         if (!C.sxn_valid) {
             MDG_HIP(hipMemcpyAsync(C.d_sxn, C.d_sx, n3 * sizeof(double),
                 hipMemcpyDeviceToDevice, s));
-            MDG_HIP(hipMemcpyAsync(C.d_srn, C.d_sr, nsl * sizeof(float4),
-                hipMemcpyDeviceToDevice, s));
+            if (recs)
+                MDG_HIP(hipMemcpyAsync(C.d_srn, C.d_sr, nsl * sizeof(float4),
+                    hipMemcpyDeviceToDevice, s));
             C.sxn_valid = true;
+            C.sxn_recs  = recs;
         }
         xn = C.d_sxn;
-        rn = C.d_srn;
+        rn = recs ? C.d_srn : nullptr;
     }
     TimedRegion tr(F_FORCE_CP);
     if (C.precision == 0 &&
@@ -3483,26 +3613,44 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
         grow_n(&C.d_sf64, &C.cap_sf64, 3 * nslots_all(), 0);
         if (failed()) return 0;
         if (half) fill_f64(C.d_sf64, 0.0, 3 * nslots_all());
-        unsigned grid = blocks_for((long long)nloc, BLOCK);
-        double* evp   = ev_parts((size_t)grid * (BLOCK / 64));
+        const unsigned grid = full64 ? (blocks_for(nci, BLOCK / 64) + 7) & ~7u
+                                     : blocks_for((long long)nloc, BLOCK);
+        double* evp = ev_parts((size_t)grid * (BLOCK / 64));
         if (failed()) return 0;
         const int uni = C.uniform ? 1 : 0;
+        if (full64 && fuse_final) fused = FUSED_FINAL | (xn ? FUSED_INITIAL : 0);
+#define MDG_F64C(NN, E, U)                                                                       \
+    k_cp_force_f64_full<NN, E, U><<<grid, BLOCK, 0, s>>>(nci, C.ntypes, C.t64, C.d_sx, C.d_st,    \
+        C.d_nb, C.d_numneigh, C.d_ci_natoms, C.maxneighs, C.d_sf64, evp,                          \
+        fused ? C.d_sv : nullptr, param->dtforce, xn, param->dt)
+#define MDG_F64C_N(NN)                                                                           \
+    do {                                                                                         \
+        if (C.ev_on) {                                                                           \
+            if (C.uniform) MDG_F64C(NN, true, true);                                             \
+            else MDG_F64C(NN, true, false);                                                      \
+        } else {                                                                                 \
+            if (C.uniform) MDG_F64C(NN, false, true);                                            \
+            else MDG_F64C(NN, false, false);                                                     \
+        }                                                                                        \
+    } while (0)
 #define MDG_F64(MM, NN, H, E)                                                                    \
     k_cp_force_f64<MM, NN, H, E><<<grid, BLOCK, 0, s>>>(nci, C.ncj, C.ntypes, uni, C.t64, C.d_sx, \
         C.d_st, C.d_nb, C.d_numneigh, C.maxneighs, C.d_sf64, evp)
 #define MDG_F64_SHAPE(MM, NN)                                                                    \
     do {                                                                                         \
-        if (half) {                                                                              \
-            if (C.ev_on) MDG_F64(MM, NN, true, true);                                            \
-            else MDG_F64(MM, NN, true, false);                                                   \
-        } else {                                                                                 \
-            if (C.ev_on) MDG_F64(MM, NN, false, true);                                           \
-            else MDG_F64(MM, NN, false, false);                                                  \
-        }                                                                                        \
+        if (C.ev_on) MDG_F64(MM, NN, true, true);                                                \
+        else MDG_F64(MM, NN, true, false);                                                       \
     } while (0)
-        if (C.M == 4 && C.N == 4) MDG_F64_SHAPE(4, 4);
+        if (full64) {
+            if (C.N == 4) MDG_F64C_N(4);
+            else MDG_F64C_N(8);
+        } else if (C.M == 4 && C.N == 4) MDG_F64_SHAPE(4, 4);
         else if (C.M == 4 && C.N == 8) MDG_F64_SHAPE(4, 8);
-        else MDG_F64_SHAPE(1, 2);
+        else if (half) MDG_F64_SHAPE(1, 2);
+        else if (C.ev_on) MDG_F64(1, 2, false, true);
+        else MDG_F64(1, 2, false, false);
+#undef MDG_F64C_N
+#undef MDG_F64C
 #undef MDG_F64_SHAPE
 #undef MDG_F64
         C.forces_are_f32 = false;
@@ -3591,8 +3739,12 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
     if (fused & FUSED_INITIAL) {
         std::swap(C.d_sx, C.d_sxn);
         std::swap(C.cap_sx, C.cap_sxn);
-        std::swap(C.d_sr, C.d_srn);
-        std::swap(C.cap_sr, C.cap_srn);
+        if (recs) {
+            std::swap(C.d_sr, C.d_srn);
+            std::swap(C.cap_sr, C.cap_srn);
+        } else {
+            C.rec_valid = false;
+        }
     }
     *secs = wtime() - t0;
     return fused;
