@@ -49,6 +49,9 @@ struct State {
     // local positions there (its other lanes still read the current ones) and the two swap
     double* d_xn  = nullptr;
     size_t cap_xn = 0;
+    // fast half lists: force accumulators of the local atoms, zero between calls
+    double* d_acc  = nullptr;
+    size_t cap_acc = 0;
     // atom sort: the bin-ordered copies of x, v and f (9 doubles per atom) and of the types
     double* d_sort    = nullptr;
     size_t cap_sort   = 0;
@@ -595,6 +598,149 @@ __global__ void __launch_bounds__(BLOCK) k_force_lj(int nlocal, const double* __
     }
 }
 
+// Half lists, fast: a block takes HALF_T / LPA consecutive atoms (of one region of the box, in the
+// lattice's or the bin sort's order) and adds the forces on their listed neighbours in LDS, those
+// of its own atoms in place, those of other atoms in a hash table keyed by the atom, and only then
+// adds each touched atom to memory once.  One FP64 atomic per pair and axis to memory instead took
+// 121 us a call for 35,700 atoms (1.4M pairs), nearly all of it the atomics; this takes
+// 18.5 us and 5.3 for the gather of the accumulators (with the integration).
+// LDS atomics and the latency of the list's loads bound it.  A pair that finds no slot within HALF_PROBE tries adds to memory directly.  acc: zero on entry.
+constexpr int HALF_T = 1024, HALF_PROBE = 8;
+
+template <int LPA, bool EV>
+__global__ void __launch_bounds__(HALF_T) k_force_lj_half(int nlocal, const double* __restrict__ x,
+    const int* __restrict__ type, int ntypes, Tables tab, int uniform,
+    const int* __restrict__ neighbors, const int* __restrict__ numneigh, double* __restrict__ acc,
+    double* __restrict__ ev)
+{
+    constexpr int A = HALF_T / LPA, LOG = LPA <= 8 ? 11 : 10, SLOTS = 1 << LOG;
+    __shared__ double s_tab[3][MAXTYPES2];
+    __shared__ double s_red[16];
+    __shared__ int s_key[SLOTS];
+    __shared__ double s_f[3 * SLOTS];
+    __shared__ double s_own[3 * A];
+    if (!uniform)
+        for (int k = threadIdx.x; k < ntypes * ntypes; k += HALF_T) {
+            s_tab[0][k] = tab.eps[k];
+            s_tab[1][k] = tab.sig6[k];
+            s_tab[2][k] = tab.cutf[k];
+        }
+    for (int k = threadIdx.x; k < SLOTS; k += HALF_T)
+        s_key[k] = -1;
+    for (int k = threadIdx.x; k < 3 * SLOTS; k += HALF_T)
+        s_f[k] = 0.0;
+    for (int k = threadIdx.x; k < 3 * A; k += HALF_T)
+        s_own[k] = 0.0;
+    __syncthreads();
+    const int i0   = blockIdx.x * A;
+    const int i    = i0 + threadIdx.x / LPA;
+    const int lane = threadIdx.x % LPA;
+    double fix = 0, fiy = 0, fiz = 0, e = 0, w = 0;
+    if (i < nlocal) {
+        const double xt = x[3 * i], yt = x[3 * i + 1], zt = x[3 * i + 2];
+        const int ti    = uniform ? 0 : type[i];
+        const int nn    = numneigh[i];
+        const double eps0 = tab.eps[0], sig0 = tab.sig6[0], cut0 = tab.cutf[0];
+        for (int k = lane; k < nn; k += LPA) {
+            const int j      = neighbors[(size_t)k * nlocal + i];
+            const double dx  = xt - x[3 * j];
+            const double dy  = yt - x[3 * j + 1];
+            const double dz  = zt - x[3 * j + 2];
+            const double rsq = fma(dx, dx, fma(dy, dy, dz * dz));
+            double eps = eps0, sig6 = sig0, cutf = cut0;
+            if (!uniform) {
+                const int tij = ti * ntypes + type[j];
+                eps           = s_tab[0][tij];
+                sig6          = s_tab[1][tij];
+                cutf          = s_tab[2][tij];
+            }
+            if (!(rsq < cutf)) continue;
+            const double sr2   = 1.0 / rsq;
+            const double sr6   = sr2 * sr2 * sr2 * sig6;
+            const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
+            fix = fma(dx, force, fix);
+            fiy = fma(dy, force, fiy);
+            fiz = fma(dz, force, fiz);
+            if (EV) {
+                const double wgt = j < nlocal ? 1.0 : 0.5;
+                e += wgt * 4.0 * eps * sr6 * (sr6 - 1.0);
+                w += wgt * rsq * force;
+            }
+            if (j >= nlocal) continue;
+            double* dst = nullptr;
+            if (j >= i0 && j < i0 + A) {
+                dst = &s_own[3 * (j - i0)];
+            } else {
+                unsigned h = ((unsigned)j * 2654435761u) >> (32 - LOG);
+                for (int p = 0; p < HALF_PROBE && !dst; p++, h = (h + 1) & (SLOTS - 1)) {
+                    int key = __hip_atomic_load(&s_key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (key == -1) {
+                        key = atomicCAS(&s_key[h], -1, j);
+                        if (key == -1) key = j;
+                    }
+                    if (key == j) dst = &s_f[3 * h];
+                }
+            }
+            if (dst) {
+                atomicAdd(dst, -(dx * force));
+                atomicAdd(dst + 1, -(dy * force));
+                atomicAdd(dst + 2, -(dz * force));
+            } else {
+                atomicAdd(&acc[3 * j], -(dx * force));
+                atomicAdd(&acc[3 * j + 1], -(dy * force));
+                atomicAdd(&acc[3 * j + 2], -(dz * force));
+            }
+        }
+    }
+    fix = group_sum<LPA>(fix);
+    fiy = group_sum<LPA>(fiy);
+    fiz = group_sum<LPA>(fiz);
+    if (i < nlocal && lane == 0) {
+        double* own = &s_own[3 * (i - i0)];
+        atomicAdd(own, fix);
+        atomicAdd(own + 1, fiy);
+        atomicAdd(own + 2, fiz);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < 3 * A; k += HALF_T)
+        if (3 * i0 + k < 3 * nlocal) atomicAdd(&acc[3 * i0 + k], s_own[k]);
+    for (int k = threadIdx.x; k < 3 * SLOTS; k += HALF_T) {
+        const int j = s_key[k / 3];
+        if (j >= 0) atomicAdd(&acc[3 * j + k % 3], s_f[k]);
+    }
+    if (EV) {
+        const double be = block_sum(e, s_red);
+        const double bw = block_sum(w, s_red);
+        if (threadIdx.x == 0) {
+            atomicAdd(&ev[0], be);
+            atomicAdd(&ev[1], bw);
+        }
+    }
+}
+
+// The half list's total forces from the accumulators, which are cleared for the next call; with v
+// set also the kicks, the drift and the ghosts of fused_integrate (in place: nothing else reads
+// the positions).
+__global__ void k_take_half(int nlocal, double* __restrict__ acc, double* __restrict__ f, double* x,
+    Fuse fu)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nlocal) return;
+    double fr[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        fr[d]          = acc[3 * i + d];
+        acc[3 * i + d] = 0.0;
+        f[3 * i + d]   = fr[d];
+    }
+    if (!fu.v) return;
+    double v0[3];
+    int ng = 0, g0 = 0;
+    fused_load<true>(fu, i, v0, &ng, &g0);
+    const double x0[3] = { x[3 * i], x[3 * i + 1], x[3 * i + 2] };
+    fused_integrate<1, true>(fu, nlocal, i, 0, v0, x0, ng, g0, fr[0], fr[1], fr[2]);
+}
+
 // ---------------------------------------------------------------- EAM (force_eam.c:19-228)
 // Spline knot of a pair distance (force_eam.c:72-76, 154-158): row m and offset p in [0, 1].
 __device__ inline int eam_knot(double r, double rdr, int nr, double* p)
@@ -1041,6 +1187,7 @@ void freeDeviceGFX950(Atom* atom, Neighbor* neighbor)
         neighbor->d_neighbor.numneigh  = nullptr;
     }
     dfree(S.d_xn);
+    dfree(S.d_acc);
     dfree(S.d_sort);
     dfree(S.d_sort_t);
     dfree(S.d_stencil);
@@ -1395,6 +1542,20 @@ static int lanes_per_atom(int nlocal)
                              : FAST_LPA;
 }
 
+// The same choice for the fast half-list kernel without energies.  us per step (force, gather and
+// integration with the ghosts; 38 listed neighbours) with
+//     atoms     4     8    16    32 lanes
+//       256  16.5  13.7  11.8  10.8
+//      6912  23.4  15.6  12.5  11.6
+//     16384  22.6  15.6  13.8  16.0
+//     32000  24.0  17.4  18.8  23.4
+//     55296  25.6  22.9  28.7  36.5
+//    131072  36.6  41.8  51.5  72.7
+static int half_lanes(int nlocal)
+{
+    return nlocal <= 10000 ? 32 : nlocal <= 24000 ? 16 : nlocal <= 80000 ? 8 : 4;
+}
+
 static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu)
 {
     (void)param;
@@ -1406,13 +1567,23 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
     hipStream_t s    = stream();
     if (S.ev_on) fill_f64(S.d_ev, 0.0, 2);
     const int half = neighbor->half_neigh;
-    if (half) fill_f64(atom->d_atom.fx, 0.0, 3 * (size_t)nall);
+    if (half && strict) fill_f64(atom->d_atom.fx, 0.0, 3 * (size_t)nall);
+    if (half && !strict) {
+        const size_t cap0 = S.cap_acc;
+        grow_n(&S.d_acc, &S.cap_acc, 3 * (size_t)nlocal, 0);
+        if (failed()) return 0.0;
+        if (S.cap_acc != cap0) fill_f64(S.d_acc, 0.0, S.cap_acc);
+    }
     {
         TimedRegion tr(F_FORCE_LJ);
 #define MDG_LJ(L, ST, H, E)                                                                      \
     k_force_lj<L, ST, H, E><<<blocks_for((long long)nlocal * L, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x, atom->d_atom.type,    \
         S.ntypes, S.tab, S.uniform ? 1 : 0, neighbor->d_neighbor.neighbors,                      \
         neighbor->d_neighbor.numneigh, atom->d_atom.fx, S.d_ev, fu)
+#define MDG_LJH(L, E)                                                                            \
+    k_force_lj_half<L, E><<<blocks_for(nlocal, HALF_T / L), HALF_T, 0, s>>>(nlocal,              \
+        atom->d_atom.x, atom->d_atom.type, S.ntypes, S.tab, S.uniform ? 1 : 0,                   \
+        neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, S.d_acc, S.d_ev)
         if (strict) {
             if (half) {
                 if (S.ev_on) MDG_LJ(1, true, true, true);
@@ -1423,8 +1594,14 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
             }
         } else {
             if (half) {
-                if (S.ev_on) MDG_LJ(FAST_LPA, false, true, true);
-                else MDG_LJ(FAST_LPA, false, true, false);
+                const int lanes = half_lanes(nlocal);
+                if (S.ev_on) MDG_LJH(4, true);
+                else if (lanes == 32) MDG_LJH(32, false);
+                else if (lanes == 16) MDG_LJH(16, false);
+                else if (lanes == 8) MDG_LJH(8, false);
+                else MDG_LJH(4, false);
+                k_take_half<<<blocks_for(nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, S.d_acc,
+                    atom->d_atom.fx, atom->d_atom.x, fu);
             } else if (S.ev_on) {
                 MDG_LJ(FAST_LPA, false, false, true);
             } else {
@@ -1436,6 +1613,7 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
                 else MDG_LJ(FAST_LPA, false, false, false);
             }
         }
+#undef MDG_LJH
 #undef MDG_LJ
         MDG_LAUNCH_CHECK("force_lj");
     }
@@ -1549,17 +1727,19 @@ double computeForceFinalInitialGFX950(Parameter* param, Atom* atom, Neighbor* ne
 {
     if (failed() || !S.ready) return 0.0;
     const bool eam = param->force_field == FF_EAM;
-    if (strict_mode() || (!eam && neighbor->half_neigh)) {
-        // the strict kernels and half lists (atomic forces) run the three calls in order
+    if (strict_mode()) {
+        // the strict kernels run the three calls in order
         const double t = eam ? computeForceEamGFX950(param, atom, neighbor, stats)
                              : computeForceLJGFX950(param, atom, neighbor, stats);
         finalIntegrateGFX950(false, param, atom);
         initialIntegrateGFX950(false, param, atom);
         return t;
     }
-    grow_n(&S.d_xn, &S.cap_xn, 3 * S.cap_all, 0);
+    // a half list's positions are moved after its forces are complete, in place
+    const bool in_place = !eam && neighbor->half_neigh;
+    if (!in_place) grow_n(&S.d_xn, &S.cap_xn, 3 * S.cap_all, 0);
     if (failed()) return 0.0;
-    Fuse fu{ { atom->d_atom.vx, S.d_xn, param->dt, param->dtforce } };
+    Fuse fu{ { atom->d_atom.vx, in_place ? atom->d_atom.x : S.d_xn, param->dt, param->dtforce } };
     // (not for large EAM systems: the images' writes in the border atoms' tails hold up their
     // persistent blocks by 15 us a step at 1M atoms, more than the 5 us of the ghost update)
     const bool ghosts = S.gmap_nlocal == atom->Nlocal && S.gmap_nghost == atom->Nghost &&
@@ -1575,8 +1755,10 @@ double computeForceFinalInitialGFX950(Parameter* param, Atom* atom, Neighbor* ne
     const double t = eam ? force_eam(param, atom, neighbor, fu) : force_lj(param, atom, neighbor, fu);
     // the new local positions become the current ones; ghost positions written too if their map
     // is known, else they follow at updatePbc
-    std::swap(atom->d_atom.x, S.d_xn);
-    S.cap_xn         = 3 * S.cap_all;
+    if (!in_place) {
+        std::swap(atom->d_atom.x, S.d_xn);
+        S.cap_xn = 3 * S.cap_all;
+    }
     S.ghosts_current = ghosts && !failed();
     return t;
 }

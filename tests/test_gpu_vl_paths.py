@@ -56,3 +56,81 @@ def test_full_list_forces_at_each_lane_count(dims, mixed):
         _ghosts_follow_owners(sim, sim.state())
     finally:
         sim.close()
+
+
+@pytest.mark.parametrize("mixed", [0, 1], ids=["uniform", "types"])
+@pytest.mark.parametrize("dims", [(4, 4, 4), (13, 13, 15), (15, 14, 16), (21, 17, 18),
+                                  (29, 27, 27)], ids=str)
+def test_half_list_forces_at_each_lane_count(dims, mixed):
+    """32, 16, 16, 8 and 4 lanes per atom; the fused run moves atoms and ghosts; energies."""
+    P = product()
+    print(dims, mixed, flush=True)
+    sim = P.VLSim(nx=dims[0], ny=dims[1], nz=dims[2], half_neigh=1, reneigh_every=5,
+                  **(MIXED if mixed else {}))
+    try:
+        sim.run(13)
+        st = sim.state()
+        want, e, w = _oracle_force(sim, st, 1)
+        assert np.linalg.norm(want) > 10.0
+        assert np.linalg.norm(st["f"] - want) < FORCE_RTOL * np.linalg.norm(want)
+        _ghosts_follow_owners(sim, st)
+        L = P.lib()
+        L.requestEnergyVirialGFX950(1)
+        sim.compute_force()
+        eg, wg = sim.energy_virial()
+        L.requestEnergyVirialGFX950(0)
+        assert abs(eg - e) <= 1e-11 * abs(e) and abs(wg - w) <= 1e-11 * abs(w)
+        assert np.linalg.norm(sim.state(lists=False)["f"] - want) < \
+            FORCE_RTOL * np.linalg.norm(want)
+        L.computeForceFinalInitialGFX950(sim.param_p, sim.atom_p, sim.neighbor_p, sim.stats_p)
+        _ghosts_follow_owners(sim, sim.state())
+    finally:
+        sim.close()
+
+
+def test_half_list_run_follows_full_list_run():
+    """The same trajectory from a half and a full list (FP64 sums in different orders), with the
+    half list's in-place integration against the full list's two buffers."""
+    P = product()
+    out = []
+    for half in (0, 1):
+        sim = P.VLSim(nx=6, ny=7, nz=5, half_neigh=half, reneigh_every=7)
+        try:
+            sim.run(10)
+            sim.run(15)
+            st = sim.state(lists=False)
+            out.append([st[k][:3 * st["nlocal"]] for k in ("x", "v", "f")])
+        finally:
+            sim.close()
+    for a, b in zip(*out):
+        np.testing.assert_allclose(a, b, rtol=0, atol=1e-10 * max(1.0, np.abs(b).max()))
+
+
+@pytest.mark.parametrize("n", [300, 5000])
+def test_half_list_of_scattered_neighbours(n):
+    """Random lists (main-stub's rand pattern): a block's atoms touch more others than its LDS
+    table holds, so the rest go to memory; first and last atom against the oracle."""
+    import ctypes
+    P = product()
+    nn = 38
+    res = P.stub_run("rand", n, nn, 1, ntimes=2, half=1)
+    libc = ctypes.CDLL(None)
+    libc.srand(1)
+    for _ in range(n):
+        libc.rand()  # the types
+    lists = np.empty((n, nn), np.int32)
+    for i in range(n):
+        seen = set()
+        for k in range(nn):
+            j = libc.rand() % n
+            while j == i or j in seen:
+                j = libc.rand() % n
+            seen.add(j)
+            lists[i, k] = j
+    x = np.repeat(np.arange(n) * 1e-5, 3)
+    one = np.ones(16)
+    f, _, _ = ob.force_lj(n, x, np.zeros(n, np.int32), 4, one, one, one * 1e12,
+                          np.full(n, nn, np.int32), lists.reshape(-1), 1)
+    # a handful of close pairs make up each sum: 1e-11 relative covers its reordering
+    assert abs(res["f0"] - f[0]) <= 1e-11 * abs(f[0])
+    assert abs(res["flast"] - f[3 * (n - 1)]) <= 1e-11 * abs(f[3 * (n - 1)])
