@@ -779,7 +779,8 @@ template <int LPA, bool STRICT, bool EV>
 __global__ void __launch_bounds__(BLOCK) k_eam_density(int nlocal, const double* __restrict__ x,
     const int* __restrict__ neighbors, const int* __restrict__ numneigh, double cutforcesq,
     const double* __restrict__ rs, const double* __restrict__ fs, int nr, int nrho, double rdr,
-    double rdrho, double* __restrict__ fp, double* __restrict__ ev, double* __restrict__ eatom)
+    double rdrho, double* __restrict__ fp, double* __restrict__ ev, double* __restrict__ eatom,
+    const int* __restrict__ gcnt, const int* __restrict__ goff)
 {
     __shared__ double s_red[16];
     const int gid  = blockIdx.x * blockDim.x + threadIdx.x;
@@ -787,7 +788,12 @@ __global__ void __launch_bounds__(BLOCK) k_eam_density(int nlocal, const double*
     const int lane = gid % LPA;
     const bool act = i < nlocal;
     double rhoi    = 0, e = 0;
+    int ng = 0, g0 = 0;
     if (act) {
+        if (gcnt) {
+            ng = gcnt[i];
+            g0 = goff[i];
+        }
         const double xt = x[3 * i], yt = x[3 * i + 1], zt = x[3 * i + 2];
         const int nn    = numneigh[i];
         for (int k = lane; k < nn; k += LPA) {
@@ -804,16 +810,20 @@ __global__ void __launch_bounds__(BLOCK) k_eam_density(int nlocal, const double*
         }
     }
     if (LPA > 1) rhoi = group_sum<LPA>(rhoi);
-    if (act && lane == 0) {
+    if (act && (lane == 0 || lane < ng)) {
         double p = 1.0 * rhoi * rdrho + 1.0;
         int m    = (int)p;
         m        = m < nrho - 1 ? m : nrho - 1;
         m        = m > 1 ? m : 1;
         p -= m;
-        p               = p < 1.0 ? p : 1.0;
-        const double* c = fs + m * 7;
-        fp[i]           = (c[0] * p + c[1]) * p + c[2];
-        if (EV) {
+        p                = p < 1.0 ? p : 1.0;
+        const double* c  = fs + m * 7;
+        const double fpi = (c[0] * p + c[1]) * p + c[2];
+        // the atom's images too (else k_ghost_copy copies them)
+        for (int k = lane; k < ng; k += LPA)
+            fp[nlocal + g0 + k] = fpi;
+        if (lane == 0) fp[i] = fpi;
+        if (EV && lane == 0) {
             e = ((c[3] * p + c[4]) * p + c[5]) * p + c[6];
             if (eatom) eatom[i] = e;
         }
@@ -1647,6 +1657,28 @@ void setEamTablesGFX950(int nr, int nrho, double rdr, double rdrho, const double
     S.rdrho = rdrho;
 }
 
+// Lanes per atom of the fast EAM passes.  The LDS-table passes read the whole spline tables into
+// every block first (64 and 160 KB, ~12 us a pass however few atoms there are), so up to 40000
+// atoms the passes read the rows from L2 instead, with an atom's list on as many lanes as the
+// system leaves idle; the density pass then also writes the ghosts' F'.  us per step (both passes,
+// integration, ghosts; 75 listed neighbours) with
+//     atoms  LDS tables, 4     8    16    32    64 lanes
+//       500      30.4        19.8  12.6  10.2   8.9
+//      4000      32.1        20.2  13.3  12.3  13.2
+//      8788      34.6        24.5  18.4  18.3  23.3
+//     16384      33.9        24.3  22.7  29.1  41.8
+//     32000      40.6        35.6  44.1  54.1  74.6
+//     55296      49.3        60.5  70.0  87.0 120.3
+// (with a ghost copy and a ghost update launch of 4 us each before).
+static int eam_lanes(int nlocal)
+{
+    return nlocal <= 1500    ? 64
+           : nlocal <= 9000  ? 32
+           : nlocal <= 20000 ? 16
+           : nlocal <= 40000 ? 8
+                             : FAST_LPA;
+}
+
 static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu)
 {
     if (failed() || !S.ready) return 0.0;
@@ -1660,8 +1692,6 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
     grow_n(&S.d_fp, &S.cap_fp, (size_t)nall + 1, 0);
     if (failed()) return 0.0;
     const bool strict = strict_mode();
-    const int lpa     = strict ? 1 : FAST_LPA;
-    unsigned grid     = blocks_for((long long)nlocal * lpa, BLOCK);
     hipStream_t s     = stream();
     double cutf       = param->cutforce * param->cutforce;
     double* eatom = nullptr;
@@ -1675,10 +1705,12 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
     TimedRegion tr(F_FORCE_EAM);
 #define MDG_EAM(L, ST, E)                                                                        \
     do {                                                                                         \
+        const unsigned grid = blocks_for((long long)nlocal * L, BLOCK);                          \
         k_eam_density<L, ST, E><<<grid, BLOCK, 0, s>>>(nlocal, atom->d_atom.x,                   \
             neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, cutf, S.d_rhor,       \
-            S.d_frho, S.nr, S.nrho, S.rdr, S.rdrho, S.d_fp, S.d_ev, eatom);                      \
-        launch_ghost_copy(S.d_fp, atom);                                                         \
+            S.d_frho, S.nr, S.nrho, S.rdr, S.rdrho, S.d_fp, S.d_ev, eatom,                       \
+            gmap ? S.d_gcnt : nullptr, S.d_goff);                                                \
+        if (!gmap) launch_ghost_copy(S.d_fp, atom);                                              \
         k_eam_force<L, ST, E><<<grid, BLOCK, 0, s>>>(nlocal, atom->d_atom.x,                     \
             neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, cutf, S.d_rhor,       \
             S.d_z2r, S.nr, S.rdr, S.d_fp, atom->d_atom.fx, S.d_ev, eatom, fu);                   \
@@ -1700,14 +1732,28 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
         else MDG_EAM_FT(L, ST, false);                                                           \
     } while (0)
     const bool tab = !ev && S.nr <= TAB_NR && S.ncu > 0 && nlocal > 0;
+    const bool gmap = S.gmap_nlocal == nlocal && S.gmap_nghost == atom->Nghost;
+    const int lanes = eam_lanes(nlocal);
     if (strict) {
         if (ev) MDG_EAM(1, true, true);
         else if (tab) MDG_EAM_TAB(1, true);
         else MDG_EAM(1, true, false);
+    } else if (ev) {
+        if (lanes >= 32) MDG_EAM(32, false, true);
+        else if (lanes >= 8) MDG_EAM(16, false, true);
+        else MDG_EAM(FAST_LPA, false, true);
+    } else if (lanes == 64) {
+        MDG_EAM(64, false, false);
+    } else if (lanes == 32) {
+        MDG_EAM(32, false, false);
+    } else if (lanes == 16) {
+        MDG_EAM(16, false, false);
+    } else if (lanes == 8) {
+        MDG_EAM(8, false, false);
+    } else if (tab) {
+        MDG_EAM_TAB(FAST_LPA, false);
     } else {
-        if (ev) MDG_EAM(FAST_LPA, false, true);
-        else if (tab) MDG_EAM_TAB(FAST_LPA, false);
-        else MDG_EAM(FAST_LPA, false, false);
+        MDG_EAM(FAST_LPA, false, false);
     }
 #undef MDG_EAM_TAB
 #undef MDG_EAM_FT

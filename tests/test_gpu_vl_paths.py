@@ -134,3 +134,37 @@ def test_half_list_of_scattered_neighbours(n):
     # a handful of close pairs make up each sum: 1e-11 relative covers its reordering
     assert abs(res["f0"] - f[0]) <= 1e-11 * abs(f[0])
     assert abs(res["flast"] - f[3 * (n - 1)]) <= 1e-11 * abs(f[3 * (n - 1)])
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 5), (11, 11, 11), (17, 17, 15), (20, 19, 21),
+                                  (22, 22, 21)], ids=str)
+def test_eam_forces_and_energies_at_each_lane_count(dims, tmp_path):
+    """64, 32, 16, 8 lanes per atom with the rows from L2, and the LDS-table passes; the energy
+    passes beside them; ghosts moved by the fused call."""
+    P = product()
+    print(dims, flush=True)
+    path = str(tmp_path / "cu.eam")
+    P.lib().mdbWriteFuncflSynthetic(path.encode())
+    tab = ob.EamTables(path)
+    sim = P.VLSim(nx=dims[0], ny=dims[1], nz=dims[2], force_field=1, lattice_a=3.615, temp=1600.0,
+                  maxwell_seed=5, reneigh_every=5, eam_file=path)
+    try:
+        sim.run(13)
+        st = sim.state()
+        nl = st["nlocal"]
+        cut = sim.param.cutforce ** 2
+        want, ea = ob.force_eam_atom(tab, nl, st["x"], st["border_map"], cut, st["numneigh"],
+                                     st["neighbors"])
+        want = want[:3 * nl]
+        assert np.linalg.norm(want) > 10.0
+        assert np.linalg.norm(st["f"] - want) < FORCE_RTOL * np.linalg.norm(want)
+        _ghosts_follow_owners(sim, st)
+        e = sim.eam_atom_energy()
+        assert np.linalg.norm(e - ea) < FORCE_RTOL * np.linalg.norm(ea)
+        assert np.linalg.norm(sim.state(lists=False)["f"] - want) < \
+            FORCE_RTOL * np.linalg.norm(want)
+        P.lib().computeForceFinalInitialGFX950(sim.param_p, sim.atom_p, sim.neighbor_p,
+                                               sim.stats_p)
+        _ghosts_follow_owners(sim, sim.state())
+    finally:
+        sim.close()
