@@ -8,11 +8,13 @@
 // the same way.  Fast kernels spread each atom's list over LPA lanes and use explicit fma().
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
 
 #include "mdgfx950.h"
+#include "block_scan.h"
 #include "runtime.h"
 
 using namespace mdg;
@@ -67,8 +69,11 @@ struct State {
     int* d_bincount = nullptr;
     int* d_binstart = nullptr;
     size_t cap_bins = 0, cap_binstart = 0;
-    int* d_binatoms = nullptr;
-    size_t cap_binatoms = 0;
+    int *d_binatoms = nullptr, *d_binslots = nullptr;  // in index order; as scattered
+    size_t cap_binatoms = 0, cap_binslots = 0;
+    int* d_binplace = nullptr;  // each atom's place in its bin as scattered
+    double* d_xs    = nullptr;  // positions in the order of d_binatoms: all x, all y, all z
+    size_t cap_binplace = 0, cap_xs = 0;
     bool binned = false;
     // per-atom EAM energies (training labels for the learned potential)
     double* d_eatom = nullptr;
@@ -83,7 +88,7 @@ struct State {
     // locals and ghosts of the last setupPbcGFX950, which d_gcnt, d_goff and d_pbc describe
     // (-1: none)
     int gmap_nlocal = -1, gmap_nghost = -1;
-    bool ghosts_current = false;  // the last fused force call also wrote the ghosts' positions
+    bool ghosts_current = false;  // the last call moved no local atom or moved its ghosts with it
     // neighbour list capacity (elements)
     size_t cap_nb = 0, cap_numneigh = 0;
     // EAM
@@ -216,7 +221,8 @@ __global__ void k_ghost_count(int nlocal, const double* __restrict__ x, Prd prd,
     cnt[i]       = __popc(ghost_mask(xi, prd.p, cut));
 }
 
-__global__ void k_ghost_fill(int nlocal, const double* __restrict__ x, Prd prd, double cut,
+// (the ghosts' positions too, as k_update_pbc writes them)
+__global__ void k_ghost_fill(int nlocal, double* x, Prd prd, double cut,
     const int* __restrict__ off, int* __restrict__ border_map, int* __restrict__ pbc,
     int* __restrict__ type)
 {
@@ -232,7 +238,9 @@ __global__ void k_ghost_fill(int nlocal, const double* __restrict__ x, Prd prd, 
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             int s          = c_ghost_side[c][d];
-            pbc[3 * g + d] = s == 1 ? 1 : (s == 2 ? -1 : 0);
+            const int p    = s == 1 ? 1 : (s == 2 ? -1 : 0);
+            pbc[3 * g + d] = p;
+            x[3 * (nlocal + g) + d] = xi[d] + p * prd.p[d];
         }
         type[nlocal + g] = ti;
         g++;
@@ -250,8 +258,10 @@ __global__ void k_update_pbc(int nlocal, int nghost, double* __restrict__ x,
 }
 
 // ---------------------------------------------------------------- binning (neighbor.c:386-464)
+// Each atom's bin and its place among the bin's atoms as they arrive (one atomic per atom: with a
+// second one in the scatter the two took 29 us each at 1M atoms).
 __global__ void k_bin_count(int nall, const double* __restrict__ x, Grid g, int* __restrict__ bin_of,
-    int* __restrict__ count, int* __restrict__ status)
+    int* __restrict__ place, int* __restrict__ count, int* __restrict__ status)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nall) return;
@@ -262,36 +272,40 @@ __global__ void k_bin_count(int nall, const double* __restrict__ x, Grid g, int*
         return;
     }
     bin_of[i] = b;
-    atomicAdd(&count[b], 1);
+    place[i]  = atomicAdd(&count[b], 1);
 }
 
 __global__ void k_bin_scatter(int nall, const int* __restrict__ bin_of,
-    const int* __restrict__ binstart, int* __restrict__ cursor, int* __restrict__ binatoms)
+    const int* __restrict__ place, const int* __restrict__ binstart, int* __restrict__ slots)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nall) return;
     int b = bin_of[i];
     if (b < 0) return;
-    int slot                  = atomicAdd(&cursor[b], 1);
-    binatoms[binstart[b] + slot] = i;
+    slots[binstart[b] + place[i]] = i;
 }
 
-// Atomics scatter in arbitrary order; the reference fills bins in atom-index order, so each
-// bin (a handful of atoms) is insertion-sorted by index.
-__global__ void k_bin_sort(int mbins, const int* __restrict__ binstart, int* __restrict__ binatoms)
+// Atoms arrive in a bin in arbitrary order; the reference fills bins in atom-index order, so each
+// atom goes to its rank among its bin's (a handful of atoms).  One atom per thread: with one bin
+// per thread (an insertion sort in memory) it took 13 us for 256 atoms and their ghosts.  The
+// positions are copied to the same order (xs: n x, n y, n z), in which the list build's candidates
+// are contiguous.  clear: two status words zeroed for the list build that follows.
+__global__ void k_bin_rank(int n, const int* __restrict__ bin_of, const int* __restrict__ binstart,
+    const int* __restrict__ slots, const double* __restrict__ x, int* __restrict__ binatoms,
+    double* __restrict__ xs, const int* __restrict__ total, int* __restrict__ clear)
 {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= mbins) return;
-    int s = binstart[b], e = binstart[b + 1];
-    for (int p = s + 1; p < e; p++) {
-        int v = binatoms[p];
-        int q = p - 1;
-        while (q >= s && binatoms[q] > v) {
-            binatoms[q + 1] = binatoms[q];
-            q--;
-        }
-        binatoms[q + 1] = v;
-    }
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (clear && m < 2) clear[m] = 0;
+    if (m >= n || m >= *total) return;
+    const int a = slots[m], b = bin_of[a];
+    const int s = binstart[b], e = binstart[b + 1];
+    int r = s;
+    for (int k = s; k < e; k++)
+        r += slots[k] < a;
+    binatoms[r] = a;
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+        xs[(size_t)d * n + r] = x[3 * a + d];
 }
 
 // sortAtom (neighbor.c:466-536): new slot p takes the atom at position p of the bin-major list of
@@ -315,55 +329,76 @@ __global__ void k_sort_gather(int n, const int* __restrict__ order, const double
 
 // ---------------------------------------------------------------- neighbour build
 // (neighbor.c:260-352): stencil bins in order, atoms in bin order, rsq <= cutneighsq.
-// One wavefront per bin.  The bin's local atoms (32 at a time, bin order) sit in LDS; the
-// candidates of the bin's stencil, flattened in the reference's loop order (stencil bins in order,
-// atoms in bin order), are tested 64 at a time, one per lane, against every local atom of the
-// bin, and a ballot gives each accepted candidate its place in that atom's list.  A lane's two
-// loads per candidate are independent of the previous candidate's, and lanes of a wavefront read
-// neighbouring entries of the bin arrays.
-__global__ void __launch_bounds__(BLOCK) k_build_neighbor(int nlocal, const double* __restrict__ x,
-    const int* __restrict__ type, int ntypes, Tables tab, int uniform, int mbins,
+// One block per bin, its local atoms (32 at a time, bin order) in LDS.  The candidates of the bin's
+// stencil are flattened in the reference's loop order (stencil bins in order, atoms in bin order)
+// and taken in segments of NB_SEG, in four passes over the block's threads:
+//   1. the candidates farther from the local atoms' bounding box than the cutoff drop out (about
+//      half of the stencil's; the margin keeps every pair whose own test could pass); the others
+//      stay in order;
+//   2. the rest against every local atom, a ballot per atom and 64 candidates kept in LDS;
+//   3. the ballots' running counts per local atom;
+//   4. each accepted candidate to its place in that atom's list.
+// For small systems, whose few bins leave the chip idle: the passes' latency bounds it (one
+// wavefront per bin with every candidate tested against every atom, as before, took 40 us for 256
+// atoms; this takes 17, of 16384 atoms 35 us; the wavefront kernel below 27 and 41 us, but from
+// 32000 atoms on 50 us against 56, and 794 against 1650 us at 1M).
+constexpr int NB_T = 256, NB_SEG = 1024, NB_Q = 32;
+constexpr int NB_SMALL = 24000;  // atoms up to which the block kernel builds the lists
+
+__global__ void __launch_bounds__(NB_T) k_build_neighbor(int nlocal, int nall, const double* __restrict__ xs,
+    const int* __restrict__ type, int ntypes, Tables tab, int uniform, double cnmax, int mbins,
     const int* __restrict__ binstart, const int* __restrict__ binatoms,
     const int* __restrict__ stencil, int nstencil, int half, int maxneighs,
     int* __restrict__ neighbors, int* __restrict__ numneigh, int* __restrict__ status)
 {
-    __shared__ int s_st[1024];
-    __shared__ double s_x[BLOCK / 64][32][3];
-    __shared__ int s_id[BLOCK / 64][32], s_t[BLOCK / 64][32];
-    for (int k = threadIdx.x; k < nstencil; k += blockDim.x)
-        s_st[k] = stencil[k];
-    __syncthreads();
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64) + w);
+    __shared__ int s_m[NB_SEG], s_cj[NB_SEG];
+    __shared__ unsigned long long s_mask[NB_Q][NB_SEG / 64];
+    __shared__ int s_off[NB_Q][NB_SEG / 64];
+    __shared__ double s_x[NB_Q][3];
+    __shared__ int s_id[NB_Q], s_t[NB_Q], s_cnt[NB_Q], s_scan[33], s_w[NB_T / 64], s_nq;
+    const double* ys = xs + nall;
+    const double* zs = ys + nall;
+    const int b      = blockIdx.x;
     if (b >= mbins) return;
-    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const int beg = binstart[b], end = binstart[b + 1];
-    for (int q0 = beg; q0 < end; q0 += 32) {
-        // this chunk's local atoms, in bin order
-        const int m0 = q0 + lane;
-        int i0 = -1;
-        if (lane < 32 && m0 < end) i0 = binatoms[m0];
-        const bool isloc = i0 >= 0 && i0 < nlocal;
-        const unsigned long long lb = __ballot(isloc);
-        const int nq = __popcll(lb);
-        if (nq == 0) continue;
-        if (isloc) {
-            const int q  = __popcll(lb & lt);
-            s_id[w][q]   = i0;
-            s_t[w][q]    = type[i0];
-            s_x[w][q][0] = x[3 * i0];
-            s_x[w][q][1] = x[3 * i0 + 1];
-            s_x[w][q][2] = x[3 * i0 + 2];
+    // index order inside a bin: its local atoms come first
+    if (beg >= end || binatoms[beg] >= nlocal) return;
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    for (int q0 = beg; q0 < end; q0 += NB_Q) {
+        __syncthreads();
+        if (w == 0) {
+            const int m0 = q0 + lane;
+            int i0       = -1;
+            if (lane < NB_Q && m0 < end) i0 = binatoms[m0];
+            const bool isloc = i0 >= 0 && i0 < nlocal;
+            const unsigned long long lb = __ballot(isloc);
+            if (isloc) {
+                const int q = __popcll(lb & lt);
+                s_id[q]     = i0;
+                s_t[q]      = type[i0];
+                s_x[q][0]   = xs[m0];
+                s_x[q][1]   = ys[m0];
+                s_x[q][2]   = zs[m0];
+            }
+            if (lane < NB_Q) s_cnt[lane] = 0;
+            if (lane == 0) s_nq = __popcll(lb);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        int cnt = 0;  // lane q < nq: length of atom q's list so far
-        for (int s0 = 0; s0 < nstencil; s0 += 64) {
-            const int sidx = s0 + lane;
+        __syncthreads();
+        const int nq = s_nq;
+        if (nq == 0) break;
+        double lo3[3] = { s_x[0][0], s_x[0][1], s_x[0][2] }, hi3[3] = { lo3[0], lo3[1], lo3[2] };
+        for (int q = 1; q < nq; q++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const double v = s_x[q][d];
+                lo3[d]         = fmin(lo3[d], v);
+                hi3[d]         = fmax(hi3[d], v);
+            }
+        for (int c0 = 0; c0 < nstencil; c0 += NB_T) {
             int lo = 0, cc = 0;
-            if (sidx < nstencil) {
-                const int jb = b + s_st[sidx];
+            if (c0 + tid < nstencil) {
+                const int jb = b + stencil[c0 + tid];
                 if (jb < 0 || jb >= mbins) {
                     atomicOr(&status[0], ST_BIN_RANGE);
                 } else {
@@ -371,62 +406,255 @@ __global__ void __launch_bounds__(BLOCK) k_build_neighbor(int nlocal, const doub
                     cc = binstart[jb + 1] - lo;
                 }
             }
-            int inc = cc;
+            int total;
+            const int pre = block_excl_scan(cc, s_scan, &total);
+            for (int g0 = 0; g0 < total; g0 += NB_SEG) {
+                const int segn = min(NB_SEG, total - g0);
+                for (int t = max(pre, g0); t < min(pre + cc, g0 + segn); t++)
+                    s_m[t - g0] = lo + (t - pre);
+                __syncthreads();
+                // 1. the candidates near the local atoms' box, in order
+                int nc = 0;
+                for (int t0 = 0; t0 < segn; t0 += NB_T) {
+                    const int t = t0 + tid;
+                    bool near   = false;
+                    int m       = 0;
+                    if (t < segn) {
+                        m                  = s_m[t];
+                        const double xj[3] = { xs[m], ys[m], zs[m] };
+                        double d2          = 0.0;
 #pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(inc, o, 64);
-                if (lane >= o) inc += v;
+                        for (int d = 0; d < 3; d++) {
+                            const double g = fmax(fmax(lo3[d] - xj[d], xj[d] - hi3[d]), 0.0);
+                            d2             = fma(g, g, d2);
+                        }
+                        near = d2 <= cnmax;
+                    }
+                    const unsigned long long bal = __ballot(near);
+                    if (lane == 0) s_w[w] = __popcll(bal);
+                    __syncthreads();
+                    int at = nc;
+#pragma unroll
+                    for (int k = 0; k < NB_T / 64; k++) {
+                        if (k < w) at += s_w[k];
+                        nc += s_w[k];
+                    }
+                    if (near) s_cj[at + __popcll(bal & lt)] = m;
+                    __syncthreads();
+                }
+                const int nb = (nc + 63) >> 6;
+                // 2. against every local atom, half of the atoms per turn of a wavefront
+                const int qh = (nq + 1) >> 1;
+                for (int u = w; u < 2 * nb; u += NB_T / 64) {
+                    const int bt = u >> 1, qb = (u & 1) * qh, qe = min(nq, qb + qh);
+                    const bool cand = bt * 64 + lane < nc;
+                    int j = 0, tj = 0;
+                    double xj = 0.0, yj = 0.0, zj = 0.0;
+                    if (cand) {
+                        const int m = s_cj[bt * 64 + lane];
+                        j           = binatoms[m];
+                        xj          = xs[m];
+                        yj          = ys[m];
+                        zj          = zs[m];
+                        if (!uniform) tj = type[j];
+                    }
+                    for (int q = qb; q < qe; q++) {
+                        const int i      = s_id[q];
+                        const double dx  = s_x[q][0] - xj;
+                        const double dy  = s_x[q][1] - yj;
+                        const double dz  = s_x[q][2] - zj;
+                        const double rsq = dx * dx + dy * dy + dz * dz;
+                        const double cn  = uniform ? tab.cutn[0] : tab.cutn[s_t[q] * ntypes + tj];
+                        const bool pass  = cand && j != i && !(half && j < i) && rsq <= cn;
+                        const unsigned long long bq = __ballot(pass);
+                        if (lane == 0) s_mask[q][bt] = bq;
+                    }
+                }
+                __syncthreads();
+                // 3. running counts
+                if (tid < nq) {
+                    int n = s_cnt[tid];
+                    for (int bt = 0; bt < nb; bt++) {
+                        s_off[tid][bt] = n;
+                        n += __popcll(s_mask[tid][bt]);
+                    }
+                    s_cnt[tid] = n;
+                }
+                __syncthreads();
+                // 4. the accepted ones to their lists
+                for (int bt = 0; bt < nb; bt++) {
+                    const int j = bt * 64 + lane < nc ? binatoms[s_cj[bt * 64 + lane]] : 0;
+                    for (int q = w; q < nq; q += NB_T / 64) {
+                        const unsigned long long m = s_mask[q][bt];
+                        const int pos              = s_off[q][bt] + __popcll(m & lt);
+                        if ((m >> lane & 1) && pos < maxneighs)
+                            neighbors[(size_t)pos * nlocal + s_id[q]] = j;
+                    }
+                }
+                __syncthreads();
             }
+        }
+        if (tid < nq) {
+            const int n         = s_cnt[tid];
+            numneigh[s_id[tid]] = n;
+            if (n > maxneighs) {
+                atomicOr(&status[0], ST_NB_OVERFLOW);
+                atomicMax(&status[1], n);
+            }
+        }
+    }
+}
+
+// The same for large systems, one wavefront per bin and no barriers: the stencil columns' lanes
+// write the candidates' entries to LDS (each candidate found its column by a binary search of
+// dependent cross-lane reads before), the ones near the local atoms' box are kept in place, in
+// order, and only those are tested against every local atom.  880 -> 794 us for 1M atoms, 147 ->
+// 120 us for 131,000.  The tests' vector instructions (1640 per bin, 400 us) and the texture
+// path's work (the scattered list stores and the candidates' loads, 600 us busy) bound it; bins
+// of one XCD adjacent made it slower (895 us: slabs of ghost bins leave an XCD idle).
+constexpr int NBW_SEG = 1024;
+struct NbLocal {
+    double x, y, z;
+    int id, type;
+};
+
+__device__ inline void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__global__ void __launch_bounds__(BLOCK) k_build_neighbor_wave(int nlocal, int nall,
+    const double* __restrict__ xs, const int* __restrict__ type, int ntypes, Tables tab, int uniform,
+    double cnmax, int mbins, const int* __restrict__ binstart, const int* __restrict__ binatoms,
+    const int* __restrict__ stencil, int nstencil, int half, int maxneighs,
+    int* __restrict__ neighbors, int* __restrict__ numneigh, int* __restrict__ status)
+{
+    __shared__ int s_c[BLOCK / 64][NBW_SEG];
+    __shared__ __align__(16) NbLocal s_l[BLOCK / 64][NB_Q];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64) + w);
+    if (b >= mbins) return;
+    const int beg = binstart[b], end = binstart[b + 1];
+    if (beg >= end || binatoms[beg] >= nlocal) return;
+    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const double* ys = xs + nall;
+    const double* zs = ys + nall;
+    int* s_m         = s_c[w];
+    NbLocal* loc = s_l[w];
+    for (int q0 = beg; q0 < end; q0 += NB_Q) {
+        // this chunk's local atoms, in bin order, and their box
+        const int m0 = q0 + lane;
+        int i0       = -1;
+        if (lane < NB_Q && m0 < end) i0 = binatoms[m0];
+        const bool isloc = i0 >= 0 && i0 < nlocal;
+        const int nq     = __popcll(__ballot(isloc));
+        if (nq == 0) break;  // index order inside a bin: ghosts from here on
+        double lo3[3] = { 1e300, 1e300, 1e300 }, hi3[3] = { -1e300, -1e300, -1e300 };
+        if (isloc) {  // lanes 0 .. nq - 1
+            NbLocal l{ xs[m0], ys[m0], zs[m0], i0, type[i0] };
+            loc[lane] = l;
+            lo3[0] = hi3[0] = l.x;
+            lo3[1] = hi3[1] = l.y;
+            lo3[2] = hi3[2] = l.z;
+        }
+#pragma unroll
+        for (int o = 1; o < NB_Q; o <<= 1)
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                lo3[d] = fmin(lo3[d], __shfl_xor(lo3[d], o, 64));
+                hi3[d] = fmax(hi3[d], __shfl_xor(hi3[d], o, 64));
+            }
+#pragma unroll
+        for (int d = 0; d < 3; d++) {  // lanes 32 .. 63 read those of lanes 0 .. 31
+            lo3[d] = __shfl(lo3[d], lane & (NB_Q - 1), 64);
+            hi3[d] = __shfl(hi3[d], lane & (NB_Q - 1), 64);
+        }
+        int cnt = 0;  // lane q < nq: length of atom q's list so far
+        for (int s0 = 0; s0 < nstencil; s0 += 64) {
+            int lo = 0, cc = 0;
+            if (s0 + lane < nstencil) {
+                const int jb = b + stencil[s0 + lane];
+                if (jb < 0 || jb >= mbins) {
+                    atomicOr(&status[0], ST_BIN_RANGE);
+                } else {
+                    lo = binstart[jb];
+                    cc = binstart[jb + 1] - lo;
+                }
+            }
+            const int inc   = wave_incl_scan(cc);
             const int total = __shfl(inc, 63, 64);
             const int pre   = inc - cc;
-            for (int t0 = 0; t0 < total; t0 += 64) {
-                const int t = t0 + lane;
-                // largest column c with pre[c] <= t (cross-lane reads in every lane)
-                int c = 0;
+            for (int g0 = 0; g0 < total; g0 += NBW_SEG) {
+                const int segn = min(NBW_SEG, total - g0);
+                const int t1   = min(inc, g0 + segn);
+                wave_fence();
+                for (int t = max(pre, g0); t < t1; t++)
+                    s_m[t - g0] = lo + (t - pre);
+                wave_fence();
+                // the candidates near the box stay, in order (a batch is read before its places,
+                // at or below it, are written)
+                int nc = 0;
+                for (int t0 = 0; t0 < segn; t0 += 64) {
+                    bool near = false;
+                    int m     = 0;
+                    if (t0 + lane < segn) {
+                        m                  = s_m[t0 + lane];
+                        const double xj[3] = { xs[m], ys[m], zs[m] };
+                        double d2          = 0.0;
 #pragma unroll
-                for (int step = 32; step > 0; step >>= 1) {
-                    const int pc = __shfl(pre, c + step, 64);
-                    if (pc <= t) c += step;
-                }
-                const int m     = __shfl(lo, c, 64) + (t - __shfl(pre, c, 64));
-                const bool cand = t < total;
-                int j = -1, tj = 0;
-                double xj = 0.0, yj = 0.0, zj = 0.0;
-                if (cand) {
-                    j  = binatoms[m];
-                    xj = x[3 * j];
-                    yj = x[3 * j + 1];
-                    zj = x[3 * j + 2];
-                    if (!uniform) tj = type[j];
-                }
-                for (int q = 0; q < nq; q++) {
-                    const int i     = s_id[w][q];
-                    const double dx = s_x[w][q][0] - xj;
-                    const double dy = s_x[w][q][1] - yj;
-                    const double dz = s_x[w][q][2] - zj;
-                    const double rsq = dx * dx + dy * dy + dz * dz;
-                    const double cn  = uniform ? tab.cutn[0] : tab.cutn[s_t[w][q] * ntypes + tj];
-                    const bool pass  = cand && j != i && !(half && j < i) && rsq <= cn;
-                    const unsigned long long bq = __ballot(pass);
-                    const int base = __builtin_amdgcn_readlane(cnt, q);
-                    if (pass) {
-                        const int pos = base + __popcll(bq & lt);
-                        if (pos < maxneighs) neighbors[(size_t)pos * nlocal + i] = j;
+                        for (int d = 0; d < 3; d++) {
+                            const double g = fmax(fmax(lo3[d] - xj[d], xj[d] - hi3[d]), 0.0);
+                            d2             = fma(g, g, d2);
+                        }
+                        near = d2 <= cnmax;
                     }
-                    if (lane == q) cnt += __popcll(bq);
+                    const unsigned long long bal = __ballot(near);
+                    wave_fence();
+                    if (near) s_m[nc + __popcll(bal & lt)] = m;
+                    wave_fence();
+                    nc += __popcll(bal);
+                }
+                for (int t0 = 0; t0 < nc; t0 += 64) {
+                    const bool cand = t0 + lane < nc;
+                    int j = -1, tj = 0;
+                    double xj = 0.0, yj = 0.0, zj = 0.0;
+                    if (cand) {
+                        const int m = s_m[t0 + lane];
+                        j           = binatoms[m];
+                        xj          = xs[m];
+                        yj          = ys[m];
+                        zj          = zs[m];
+                        if (!uniform) tj = type[j];
+                    }
+                    for (int q = 0; q < nq; q++) {
+                        const NbLocal l  = loc[q];
+                        const double dx  = l.x - xj;
+                        const double dy  = l.y - yj;
+                        const double dz  = l.z - zj;
+                        const double rsq = dx * dx + dy * dy + dz * dz;
+                        const double cn  = uniform ? tab.cutn[0] : tab.cutn[l.type * ntypes + tj];
+                        const bool pass  = cand && j != l.id && !(half && j < l.id) && rsq <= cn;
+                        const unsigned long long bq = __ballot(pass);
+                        const int base = __builtin_amdgcn_readlane(cnt, q);
+                        if (pass) {
+                            const int pos = base + __popcll(bq & lt);
+                            if (pos < maxneighs) neighbors[(size_t)pos * nlocal + l.id] = j;
+                        }
+                        if (lane == q) cnt += __popcll(bq);
+                    }
                 }
             }
         }
         if (lane < nq) {
-            numneigh[s_id[w][lane]] = cnt;
+            numneigh[i0] = cnt;
             if (cnt > maxneighs) {
                 atomicOr(&status[0], ST_NB_OVERFLOW);
                 atomicMax(&status[1], cnt);
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_fence();
     }
 }
 
@@ -1205,6 +1433,9 @@ void freeDeviceGFX950(Atom* atom, Neighbor* neighbor)
     dfree(S.d_bincount);
     dfree(S.d_binstart);
     dfree(S.d_binatoms);
+    dfree(S.d_binslots);
+    dfree(S.d_binplace);
+    dfree(S.d_xs);
     dfree(S.d_eatom);
     dfree(S.d_gcnt);
     dfree(S.d_goff);
@@ -1365,7 +1596,8 @@ void setupNeighborGFX950(Parameter* param)
     S.binned = false;
 }
 
-void binatomsGFX950(Atom* atom)
+// clear_status: the two words of the list build's status zeroed on the way
+static void bin_atoms(Atom* atom, bool clear_status)
 {
     if (failed() || !S.ready || S.g.mbins == 0) {
         if (!failed()) set_error(MDG_ERR_ARG, "binatomsGFX950 before setupNeighborGFX950");
@@ -1374,23 +1606,31 @@ void binatomsGFX950(Atom* atom)
     TimedRegion tr(F_BINNING);
     int nall = atom->Nlocal + atom->Nghost;
     int mb   = S.g.mbins;
+    const size_t cap0 = S.cap_bins;
+    grow_n(&S.d_binplace, &S.cap_binplace, (size_t)nall, 0);
+    grow_n(&S.d_xs, &S.cap_xs, 3 * (size_t)nall, 0);
     grow_n(&S.d_bin_of, &S.cap_bin_of, (size_t)nall, 0);
     grow_n(&S.d_bincount, &S.cap_bins, (size_t)mb + 1, 0);
     grow_n(&S.d_binstart, &S.cap_binstart, (size_t)mb + 1, 0);
     grow_n(&S.d_binatoms, &S.cap_binatoms, (size_t)nall + 1, 0);
+    grow_n(&S.d_binslots, &S.cap_binslots, (size_t)nall + 1, 0);
     if (failed()) return;
     hipStream_t s = stream();
-    fill_i32(S.d_bincount, 0, (size_t)mb + 1);
+    // (all zero between binnings: the scan clears them)
+    if (S.cap_bins != cap0) fill_i32(S.d_bincount, 0, S.cap_bins);
     k_bin_count<<<blocks_for(nall, BLOCK), BLOCK, 0, s>>>(nall, atom->d_atom.x, S.g, S.d_bin_of,
-        S.d_bincount, S.d_status);
-    exclusive_scan(S.d_bincount, S.d_binstart, mb, S.d_binstart + mb);
-    fill_i32(S.d_bincount, 0, (size_t)mb);
-    k_bin_scatter<<<blocks_for(nall, BLOCK), BLOCK, 0, s>>>(nall, S.d_bin_of, S.d_binstart,
-        S.d_bincount, S.d_binatoms);
-    k_bin_sort<<<blocks_for(mb, BLOCK), BLOCK, 0, s>>>(mb, S.d_binstart, S.d_binatoms);
+        S.d_binplace, S.d_bincount, S.d_status);
+    exclusive_scan_take(S.d_bincount, S.d_binstart, mb, S.d_binstart + mb);
+    k_bin_scatter<<<blocks_for(nall, BLOCK), BLOCK, 0, s>>>(nall, S.d_bin_of, S.d_binplace,
+        S.d_binstart, S.d_binslots);
+    k_bin_rank<<<blocks_for(nall, BLOCK), BLOCK, 0, s>>>(nall, S.d_bin_of, S.d_binstart,
+        S.d_binslots, atom->d_atom.x, S.d_binatoms, S.d_xs, S.d_binstart + mb,
+        clear_status ? S.d_status : nullptr);
     MDG_LAUNCH_CHECK("binatoms");
     S.binned = true;
 }
+
+void binatomsGFX950(Atom* atom) { bin_atoms(atom, false); }
 
 void sortAtomGFX950(Atom* atom)
 {
@@ -1432,21 +1672,29 @@ void sortAtomGFX950(Atom* atom)
 void buildNeighborGFX950(Atom* atom, Neighbor* neighbor)
 {
     if (failed() || !S.ready) return;
-    binatomsGFX950(atom);
+    bin_atoms(atom, true);
     if (failed()) return;
     const int nlocal = atom->Nlocal;
+    // the largest list cutoff squared, with a margin over the rounding of a distance to a box
+    double cnmax = 0.0;
+    for (int k = 0; k < S.ntypes * S.ntypes; k++)
+        cnmax = std::max(cnmax, S.tab.cutn[k]);
+    cnmax *= 1.0 + 1e-12;
     for (int attempt = 0; attempt < 8; attempt++) {
         grow_n(&neighbor->d_neighbor.neighbors, &S.cap_nb, (size_t)nlocal * neighbor->maxneighs, 0);
         grow_n(&neighbor->d_neighbor.numneigh, &S.cap_numneigh, (size_t)nlocal, 0);
         if (failed()) return;
-        fill_i32(S.d_status, 0, 2);
+        if (attempt > 0) fill_i32(S.d_status, 0, 2);
         {
             TimedRegion tr(F_NEIGHBOR);
-            k_build_neighbor<<<blocks_for(S.g.mbins, BLOCK / 64), BLOCK, 0, stream()>>>(nlocal,
-                atom->d_atom.x, atom->d_atom.type, S.ntypes, S.tab, S.uniform ? 1 : 0, S.g.mbins,
-                S.d_binstart, S.d_binatoms, S.d_stencil, S.nstencil, neighbor->half_neigh,
-                neighbor->maxneighs, neighbor->d_neighbor.neighbors,
-                neighbor->d_neighbor.numneigh, S.d_status);
+#define MDG_NB(K, G, T)                                                                          \
+    K<<<G, T, 0, stream()>>>(nlocal, nlocal + atom->Nghost, S.d_xs, atom->d_atom.type, S.ntypes, S.tab, \
+        S.uniform ? 1 : 0, cnmax, S.g.mbins, S.d_binstart, S.d_binatoms, S.d_stencil,             \
+        S.nstencil, neighbor->half_neigh, neighbor->maxneighs, neighbor->d_neighbor.neighbors,    \
+        neighbor->d_neighbor.numneigh, S.d_status)
+            if (nlocal <= NB_SMALL) MDG_NB(k_build_neighbor, S.g.mbins, NB_T);
+            else MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK);
+#undef MDG_NB
             MDG_LAUNCH_CHECK("build_neighbor");
         }
         read_status();
@@ -1506,6 +1754,7 @@ void setupPbcGFX950(Atom* atom, Parameter* param)
     atom->Nghost  = nghost;
     S.gmap_nlocal = nlocal;
     S.gmap_nghost = nghost;
+    S.ghosts_current = true;
 }
 
 void updatePbcGFX950(Atom* atom, Parameter* param, bool doReneighbor)
@@ -1809,7 +2058,8 @@ double computeForceFinalInitialGFX950(Parameter* param, Atom* atom, Neighbor* ne
     return t;
 }
 
-// For the run loop: the last call was a fused force call that also moved the ghosts.
+// For the run loop: the last call was setupPbcGFX950, or a fused force call that also moved the
+// ghosts.
 int mdg_vl_ghosts_current(void) { return S.ghosts_current; }
 
 void requestEamAtomEnergyGFX950(int on)

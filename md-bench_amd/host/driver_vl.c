@@ -254,7 +254,7 @@ int mdbVLRun(mdb_vl* s, int nsteps, double* ksum)
         if (reneigh) {
             updateAtomsPbcGFX950(a, p, true);
             setupPbcGFX950(a, p);
-            updatePbcGFX950(a, p, true);
+            if (!mdg_vl_ghosts_current()) updatePbcGFX950(a, p, true);
             buildNeighborGFX950(a, nb);
         } else if (!(integrated && mdg_vl_ghosts_current())) {
             /* (the fused force call wrote the ghosts' positions with the atoms') */

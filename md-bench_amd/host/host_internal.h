@@ -20,7 +20,8 @@ double mdb_wtime(void);
 void mdb_setup_thermo(mdb_thermo* th, Parameter* p, int natoms);
 void mdb_adjust_thermo(const mdb_thermo* th, const Parameter* p, Atom* a);
 void mdb_free_atom_host(Atom* a);
-/* 1 after a fused force call that also wrote the ghosts' new positions (csrc/vl.hip). */
+/* 1 after a fused force call that also wrote the ghosts' new positions, and after setupPbcGFX950
+   (csrc/vl.hip). */
 int mdg_vl_ghosts_current(void);
 
 #endif

@@ -168,3 +168,49 @@ def test_eam_forces_and_energies_at_each_lane_count(dims, tmp_path):
         _ghosts_follow_owners(sim, sim.state())
     finally:
         sim.close()
+
+
+@pytest.mark.parametrize("half", [0, 1])
+@pytest.mark.parametrize("case", [dict(nx=4, ny=4, nz=4), dict(nx=19, ny=18, nz=17),
+                                  dict(nx=19, ny=18, nz=19), dict(nx=5, ny=5, nz=5, skin=3.0),
+                                  dict(nx=7, ny=6, nz=8, squeeze=0.5)], ids=str)
+def test_lists_equal_the_oracles_on_moved_atoms(case, half):
+    """Both list builds (one block or one wavefront per bin): small, below and above the size
+    where the choice changes, stencils of many columns, bins of more than 32 atoms."""
+    P = product()
+    print(case, half, flush=True)
+    x0, _, _ = P.create_lattice(**{k: case[k] for k in ("nx", "ny", "nz")})
+    squeeze = case.get("squeeze", 1.0)  # all atoms in one corner of the box
+    sim = P.VLSim(half_neigh=half, reneigh_every=1000,
+                  **{k: v for k, v in case.items() if k != "squeeze"})
+    try:
+        n = sim.atom.Nlocal
+        L = P.lib()
+        p = sim.param
+        prd = np.array([p.xprd, p.yprd, p.zprd])
+        rng = np.random.default_rng(9)
+        x = x0.reshape(-1, 3) + rng.uniform(-0.15, 0.15, (n, 3))
+        x = squeeze * np.where(x < 0, x + prd, np.where(x >= prd, x - prd, x))
+        host = np.ctypeslib.as_array(sim.atom.x, (3 * n,))
+        host[:] = x.reshape(-1)
+        nghost, sim.atom.Nghost = sim.atom.Nghost, 0  # the host copies hold the local atoms only
+        L.copyDataToGFX950Device(sim.param_p, sim.atom_p)
+        L.updateAtomsPbcGFX950(sim.atom_p, sim.param_p, True)
+        L.setupPbcGFX950(sim.atom_p, sim.param_p)
+        L.updatePbcGFX950(sim.atom_p, sim.param_p, True)
+        L.buildNeighborGFX950(sim.atom_p, sim.neighbor_p)
+        st = sim.state()
+        np.testing.assert_array_equal(st["x"][:3 * n], x.reshape(-1))
+        _ghosts_follow_owners(sim, st)
+        g = ob.vl_grid(case["nx"], case["ny"], case["nz"], p.lattice, p.cutneigh)
+        start, atoms = sim.bins()
+        nn, nb = ob.build_neighbor(g, n, st["x"], np.zeros(n + st["nghost"], np.int32), 4,
+                                   np.full(16, p.cutneigh ** 2), half, cap_per_atom=2000)
+        np.testing.assert_array_equal(st["numneigh"], nn)
+        np.testing.assert_array_equal(st["neighbors"], nb)
+        if "squeeze" in case:
+            assert np.diff(start).max() > 32
+        if "skin" in case:
+            assert nghost > 0 and nn.max() > 200
+    finally:
+        sim.close()
