@@ -101,6 +101,8 @@ struct CPState {
     double *d_ax = nullptr, *d_av = nullptr;
     int* d_at  = nullptr;
     size_t cap_ax = 0, cap_av = 0, cap_at = 0;
+    double* d_vsoa  = nullptr;  // velocities as the struct's three arrays, for host transfers
+    size_t cap_vsoa = 0;
     int *d_abin_of = nullptr, *d_abin_cnt = nullptr, *d_abin_start = nullptr,
         *d_abin_atoms = nullptr;
     size_t cap_abin_of = 0, cap_abin_cnt = 0, cap_abin_start = 0, cap_abin_atoms = 0;
@@ -2896,11 +2898,12 @@ void freeDeviceClusterGFX950(void)
         C.d_jlist, C.d_jkey, C.d_zidx, C.d_gcur, C.d_gbin_start, C.d_gbin_list, C.d_nb,
         C.d_numneigh, C.d_nmasked, C.d_red, C.d_ev, C.d_evp, C.d_status, C.d_sxn, C.d_sr, C.d_srn,
         C.d_tile_cj, C.d_tile_n, C.d_eslot, C.d_rec_off, C.d_rcount, C.d_rstart, C.d_rcur,
-        C.d_rev, C.d_rec, C.d_fown };
+        C.d_rev, C.d_rec, C.d_fown, C.d_vsoa };
     for (void* p : ptrs)
         dfree(p);
     if (C.h_status) (void)hipHostFree(C.h_status);
     if (C.h_red) (void)hipHostFree(C.h_red);
+    release_bounce();
     int M = C.M, N = C.N, rule = C.rule, fm = C.fma_dist, prec = C.precision, comp = C.comp;
     C = CPState();
     C.M = M;
@@ -2915,45 +2918,78 @@ namespace {
 void flush_atoms();
 }
 
-void copyAtomsToClusterGFX950Device(Atom* atom)
+namespace {
+// room for n atoms; what an earlier call left pending on the old ones runs first
+bool atom_arrays(size_t n)
 {
-    if (!ok()) return;
-    flush_atoms();  // requested before this upload, so run before it
-    size_t n = (size_t)atom->Nlocal;
-    C.natoms = atom->Nlocal;
+    if (!ok()) return false;
+    flush_atoms();
+    C.natoms = (int)n;
     grow_n(&C.d_ax, &C.cap_ax, 3 * n + 3, 0);
     grow_n(&C.d_av, &C.cap_av, 3 * n + 3, 0);
     grow_n(&C.d_at, &C.cap_at, n + 1, 0);
-    if (failed()) return;
-    double* v = (double*)malloc(sizeof(double) * 3 * n + 8);
-    for (size_t i = 0; i < n; i++) {
-        v[3 * i]     = atom->vx[i];
-        v[3 * i + 1] = atom->vy[i];
-        v[3 * i + 2] = atom->vz[i];
-    }
-    MDG_HIP(hipMemcpyAsync(C.d_ax, atom->x, 3 * n * sizeof(double), hipMemcpyHostToDevice, stream()));
-    MDG_HIP(hipMemcpyAsync(C.d_av, v, 3 * n * sizeof(double), hipMemcpyHostToDevice, stream()));
-    MDG_HIP(hipMemcpyAsync(C.d_at, atom->type, n * sizeof(int), hipMemcpyHostToDevice, stream()));
-    MDG_HIP(hipStreamSynchronize(stream()));
-    free(v);
+    return !failed();
+}
+
+// v AoS <-> the struct's three arrays, on the device (the host loops over 1M atoms took 3 ms)
+__global__ void k_cp_interleave(int n, const double* __restrict__ soa, double* __restrict__ aos)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+        aos[3 * (size_t)i + d] = soa[(size_t)d * n + i];
+}
+__global__ void k_cp_deinterleave(int n, const double* __restrict__ aos, double* __restrict__ soa)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+        soa[(size_t)d * n + i] = aos[3 * (size_t)i + d];
+}
+}  // namespace
+
+// For the driver: the atoms from x and v AoS.
+void mdg_cp_upload_atoms(const double* x, const double* v, const int* type, int n)
+{
+    if (!atom_arrays((size_t)n)) return;
+    copy_to_device(C.d_ax, x, 3 * (size_t)n * sizeof(double));
+    copy_to_device(C.d_av, v, 3 * (size_t)n * sizeof(double));
+    copy_to_device(C.d_at, type, (size_t)n * sizeof(int));
+}
+
+void copyAtomsToClusterGFX950Device(Atom* atom)
+{
+    const size_t n = (size_t)atom->Nlocal;
+    if (!atom_arrays(n)) return;
+    grow_n(&C.d_vsoa, &C.cap_vsoa, 3 * n + 3, 0);
+    if (failed() || n == 0) return;
+    copy_to_device(C.d_ax, atom->x, 3 * n * sizeof(double));
+    copy_to_device(C.d_vsoa, atom->vx, n * sizeof(double));
+    copy_to_device(C.d_vsoa + n, atom->vy, n * sizeof(double));
+    copy_to_device(C.d_vsoa + 2 * n, atom->vz, n * sizeof(double));
+    k_cp_interleave<<<blocks_for((long long)n, BLOCK), BLOCK, 0, stream()>>>((int)n, C.d_vsoa,
+        C.d_av);
+    MDG_LAUNCH_CHECK("cp_interleave");
+    copy_to_device(C.d_at, atom->type, n * sizeof(int));
 }
 
 void copyAtomsFromClusterGFX950Device(Atom* atom)
 {
     if (!ok()) return;
     flush_atoms();
-    size_t n = (size_t)C.natoms;
-    double* v = (double*)malloc(sizeof(double) * 3 * n + 8);
-    MDG_HIP(hipMemcpyAsync(atom->x, C.d_ax, 3 * n * sizeof(double), hipMemcpyDeviceToHost, stream()));
-    MDG_HIP(hipMemcpyAsync(v, C.d_av, 3 * n * sizeof(double), hipMemcpyDeviceToHost, stream()));
-    MDG_HIP(hipMemcpyAsync(atom->type, C.d_at, n * sizeof(int), hipMemcpyDeviceToHost, stream()));
-    MDG_HIP(hipStreamSynchronize(stream()));
-    for (size_t i = 0; i < n; i++) {
-        atom->vx[i] = v[3 * i];
-        atom->vy[i] = v[3 * i + 1];
-        atom->vz[i] = v[3 * i + 2];
-    }
-    free(v);
+    const size_t n = (size_t)C.natoms;
+    grow_n(&C.d_vsoa, &C.cap_vsoa, 3 * n + 3, 0);
+    if (failed() || n == 0) return;
+    k_cp_deinterleave<<<blocks_for((long long)n, BLOCK), BLOCK, 0, stream()>>>((int)n, C.d_av,
+        C.d_vsoa);
+    MDG_LAUNCH_CHECK("cp_deinterleave");
+    copy_from_device(atom->x, C.d_ax, 3 * n * sizeof(double));
+    copy_from_device(atom->vx, C.d_vsoa, n * sizeof(double));
+    copy_from_device(atom->vy, C.d_vsoa + n, n * sizeof(double));
+    copy_from_device(atom->vz, C.d_vsoa + 2 * n, n * sizeof(double));
+    copy_from_device(atom->type, C.d_at, n * sizeof(int));
 }
 
 // setupNeighbor (src/clusterpair/neighbor.c:108-215), restated on the host.
@@ -3879,8 +3915,6 @@ long long downloadClusterArrayGFX950(const char* name, void* out, long long cap)
 {
     if (!ok()) return -3;
     flush_atoms();  // the atom arrays as the calls so far leave them
-    hipStream_t s = stream();
-    MDG_HIP(hipStreamSynchronize(s));
     const size_t nsl = nslots_all(), nj = (size_t)C.ncj + C.nghost;
     const void* src  = nullptr;
     long long n = 0, es = 4;
@@ -3906,20 +3940,19 @@ long long downloadClusterArrayGFX950(const char* name, void* out, long long cap)
         if (n > cap) return -2;
         if (C.forces_are_f32) {
             float* tmp = (float*)malloc(n * sizeof(float) + 4);
-            MDG_HIP(hipMemcpy(tmp, C.d_sf32, n * sizeof(float), hipMemcpyDeviceToHost));
+            copy_from_device(tmp, C.d_sf32, n * sizeof(float));
             for (long long k = 0; k < n; k++)
                 ((double*)out)[k] = tmp[k];
             free(tmp);
         } else {
-            MDG_HIP(hipMemcpy(out, C.d_sf64, n * sizeof(double), hipMemcpyDeviceToHost));
+            copy_from_device(out, C.d_sf64, n * sizeof(double));
         }
         return failed() ? -3 : n;
     } else if (!strcmp(name, "neighbors")) {
         int* nn   = (int*)malloc(sizeof(int) * (C.nci + 1));
         int* full = (int*)malloc(sizeof(int) * ((size_t)C.nci * C.maxneighs + 1));
-        MDG_HIP(hipMemcpy(nn, C.d_numneigh, C.nci * sizeof(int), hipMemcpyDeviceToHost));
-        MDG_HIP(hipMemcpy(full, C.d_nb, (size_t)C.nci * C.maxneighs * sizeof(int),
-            hipMemcpyDeviceToHost));
+        copy_from_device(nn, C.d_numneigh, C.nci * sizeof(int));
+        copy_from_device(full, C.d_nb, (size_t)C.nci * C.maxneighs * sizeof(int));
         long long k = 0;
         for (int ci = 0; ci < C.nci && k >= 0; ci++)
             for (int m = 0; m < nn[ci]; m++) {
@@ -3936,7 +3969,7 @@ long long downloadClusterArrayGFX950(const char* name, void* out, long long cap)
         return -1;
     }
     if (n > cap) return -2;
-    if (n) MDG_HIP(hipMemcpy(out, src, n * es, hipMemcpyDeviceToHost));
+    copy_from_device(out, src, (size_t)(n * es));
     return failed() ? -3 : n;
 }
 

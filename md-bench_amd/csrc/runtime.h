@@ -62,6 +62,14 @@ bool grow_n(T** ptr, size_t* cap_elems, size_t n, size_t keep_n)
 }
 void dfree(void* p);
 
+// Copies between ordinary host memory and the device on the library stream.  The host memory may
+// be reused when copy_to_device returns (the copy itself is ordered on the stream);
+// copy_from_device returns when the data has arrived.  Large copies go through a few pinned
+// buffers, filled or emptied by as many threads; release_bounce gives the buffers back.
+void copy_to_device(void* dst, const void* src, size_t bytes);
+void copy_from_device(void* dst, const void* src, size_t bytes);
+void release_bounce();
+
 // Fill with a kernel (graph-safe; no hipMemsetAsync on captured streams).
 void fill_i32(int* p, int v, size_t n);
 void fill_f64(double* p, double v, size_t n);

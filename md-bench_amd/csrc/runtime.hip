@@ -5,7 +5,10 @@
 #include <cstdio>
 #include <cstring>
 #include <ctime>
+#include <algorithm>
 #include <mutex>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "mdgfx950.h"
@@ -145,6 +148,123 @@ bool grow(void** ptr, size_t* cap, size_t bytes, size_t keep)
 void dfree(void* p)
 {
     if (p) (void)hipFree(p);
+}
+
+// ---------------------------------------------------------------- host transfers
+// A copy from or to pageable memory runs at the speed of one thread's copy into the runtime's own
+// staging memory (and of its page faults, where the target is new): 25 MB took 1.7-3 ms.  From
+// BOUNCE_MIN bytes on, BOUNCE_T threads each take every BOUNCE_T-th chunk through a pinned buffer
+// of their own (12 MB in all, allocated at the first such copy): 0.6-0.9 ms.  Below, the threads
+// cost more than they save.
+constexpr int BOUNCE_T           = 6;
+constexpr size_t BOUNCE_CHUNK    = 2u << 20, BOUNCE_MIN = 4u << 20;
+static char* g_bounce[BOUNCE_T]  = {};
+static hipEvent_t g_bounce_ev[BOUNCE_T];
+static std::mutex g_bounce_lock;  // one copy at a time uses the buffers
+
+static bool bounce_ready()
+{
+    if (g_bounce[BOUNCE_T - 1]) return true;
+    for (int t = 0; t < BOUNCE_T; t++) {
+        if (g_bounce[t]) continue;
+        void* p = nullptr;
+        if (hipHostMalloc(&p, BOUNCE_CHUNK, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();  // no pinned memory left: the plain copy
+            return false;
+        }
+        if (hipEventCreateWithFlags(&g_bounce_ev[t], hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipHostFree(p);
+            return false;
+        }
+        g_bounce[t] = (char*)p;
+    }
+    return true;
+}
+
+void release_bounce()
+{
+    std::lock_guard<std::mutex> hold(g_bounce_lock);
+    for (int t = 0; t < BOUNCE_T; t++)
+        if (g_bounce[t]) {
+            (void)hipEventSynchronize(g_bounce_ev[t]);
+            (void)hipEventDestroy(g_bounce_ev[t]);
+            (void)hipHostFree(g_bounce[t]);
+            g_bounce[t] = nullptr;
+        }
+}
+
+// fn(chunk, bytes, thread) for every chunk of the copy, on BOUNCE_T threads; the first HIP error
+template <class F>
+static hipError_t bounce(size_t bytes, F fn)
+{
+    int dev = 0;
+    hipError_t e0 = hipGetDevice(&dev);
+    if (e0 != hipSuccess) return e0;
+    hipError_t err[BOUNCE_T] = {};
+    auto work = [&](int t) {
+        hipError_t e = hipSetDevice(dev);
+        for (size_t at = t * BOUNCE_CHUNK; at < bytes && e == hipSuccess;
+             at += BOUNCE_T * BOUNCE_CHUNK)
+            e = fn(at, std::min(BOUNCE_CHUNK, bytes - at), t);
+        err[t] = e;
+    };
+    std::thread threads[BOUNCE_T];
+    int started = 1;
+    try {
+        for (; started < BOUNCE_T; started++)
+            threads[started] = std::thread(work, started);
+    } catch (const std::system_error&) {
+        // no more threads: this one takes the rest's chunks as well
+    }
+    work(0);
+    for (int t = started; t < BOUNCE_T; t++)
+        work(t);
+    for (int t = 1; t < started; t++)
+        threads[t].join();
+    for (int t = 0; t < BOUNCE_T; t++)
+        if (err[t] != hipSuccess) return err[t];
+    return hipSuccess;
+}
+
+void copy_to_device(void* dst, const void* src, size_t bytes)
+{
+    if (failed() || bytes == 0) return;
+    hipStream_t s = stream();
+    std::lock_guard<std::mutex> hold(g_bounce_lock);
+    if (bytes < BOUNCE_MIN || !bounce_ready()) {
+        MDG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+        MDG_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    MDG_HIP(bounce(bytes, [&](size_t at, size_t n, int t) {
+        hipError_t e = hipEventSynchronize(g_bounce_ev[t]);  // the buffer's last copy
+        if (e != hipSuccess) return e;
+        memcpy(g_bounce[t], (const char*)src + at, n);
+        e = hipMemcpyAsync((char*)dst + at, g_bounce[t], n, hipMemcpyHostToDevice, s);
+        return e != hipSuccess ? e : hipEventRecord(g_bounce_ev[t], s);
+    }));
+}
+
+void copy_from_device(void* dst, const void* src, size_t bytes)
+{
+    if (failed() || bytes == 0) return;
+    hipStream_t s = stream();
+    std::lock_guard<std::mutex> hold(g_bounce_lock);
+    if (bytes < BOUNCE_MIN || !bounce_ready()) {
+        MDG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+        MDG_HIP(hipStreamSynchronize(s));
+        return;
+    }
+    MDG_HIP(bounce(bytes, [&](size_t at, size_t n, int t) {
+        hipError_t e = hipEventSynchronize(g_bounce_ev[t]);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(g_bounce[t], (const char*)src + at, n, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(g_bounce_ev[t], s);
+        if (e == hipSuccess) e = hipEventSynchronize(g_bounce_ev[t]);
+        if (e == hipSuccess) memcpy((char*)dst + at, g_bounce[t], n);
+        return e;
+    }));
 }
 
 // ---------------------------------------------------------------- fills

@@ -4,6 +4,7 @@
  * per-step operation and every rebuild on the device.
  */
 #include <math.h>
+#include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -15,6 +16,8 @@
 int mdgfx950Status(void);
 const char* mdgfx950StatusMessage(void);
 void mdgfx950SetStrict(int strict);
+/* csrc/cp.hip: copyAtomsToClusterGFX950Device from x and v AoS */
+void mdg_cp_upload_atoms(const double* x, const double* v, const int* type, int n);
 
 struct mdb_cp {
     Parameter param;
@@ -172,20 +175,40 @@ int mdbCPCreate(const mdb_config* cfg, mdb_cp** out)
     return 0;
 }
 
+struct host_copy {
+    Atom* a;
+    const double *x, *v;
+    const int* type;
+    int n;
+};
+
+static void* copy_to_struct(void* arg)
+{
+    const struct host_copy* c = arg;
+    Atom* a                   = c->a;
+    memcpy(a->x, c->x, sizeof(double) * 3 * c->n);
+    for (int i = 0; i < c->n; i++) {
+        a->vx[i] = c->v[3 * i];
+        a->vy[i] = c->v[3 * i + 1];
+        a->vz[i] = c->v[3 * i + 2];
+    }
+    memcpy(a->type, c->type, sizeof(int) * c->n);
+    return NULL;
+}
+
 int mdbCPSetAtoms(mdb_cp* s, const double* x, const double* v, const int* type, int n)
 {
     Atom* a = &s->atom;
     if (n != a->Nlocal) return 4;
-    memcpy(a->x, x, sizeof(double) * 3 * n);
-    for (int i = 0; i < n; i++) {
-        a->vx[i] = v[3 * i];
-        a->vy[i] = v[3 * i + 1];
-        a->vz[i] = v[3 * i + 2];
-    }
-    memcpy(a->type, type, sizeof(int) * n);
-    copyAtomsToClusterGFX950Device(a);
+    /* the device takes the caller's arrays; the struct's host copies follow beside it */
+    struct host_copy hc = { a, x, v, type, n };
+    pthread_t th;
+    const int beside = n >= 65536 && pthread_create(&th, NULL, copy_to_struct, &hc) == 0;
+    mdg_cp_upload_atoms(x, v, type, n);
     int rc = reneighbour(s);
     if (!rc) computeForceLJClusterGFX950(&s->param, a, &s->neighbor, &s->stats);
+    if (beside) pthread_join(th, NULL);
+    else copy_to_struct(&hc);
     return mdgfx950Status();
 }
 

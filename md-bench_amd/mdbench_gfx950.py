@@ -391,14 +391,28 @@ class CPSim:
         lib().clusterInfoGFX950(arr)
         return dict(zip(self.INFO, arr.tolist()))
 
+    def _size(self, name):
+        """Elements of a named device array (include/mdgfx950_cp.h)."""
+        i = self.info()
+        slots, nj = (i["ncj"] + i["nghost"] + 1) * i["N"], i["ncj"] + i["nghost"]
+        if name == "neighbors":
+            return int(self.get("numneigh").astype(np.int64).sum())
+        return {"slot_x": 3 * slots, "slot_v": 3 * i["nci"] * i["M"],
+                "slot_f": 3 * i["nci"] * i["M"], "slot_t": slots, "ci_natoms": i["nci"],
+                "ci_bin": i["nci"], "ci_bbox": 6 * i["nci"], "cj_natoms": nj,
+                "cj_bbox": 6 * nj, "ghost_map": i["nghost"], "ghost_pbc": 3 * i["nghost"],
+                "numneigh": i["nci"], "numneigh_masked": i["nci"],
+                "cbin_start": i["mbins"] + 1, "cbin_list": nj, "atoms_x": 3 * i["natoms"],
+                "atoms_v": 3 * i["natoms"], "atoms_type": i["natoms"]}.get(name, 0)
+
     def get(self, name):
         dt = np.float64 if name in self.F64 else np.int32
-        cap = 1 << 25
-        buf = np.zeros(cap, dt)
-        n = lib().downloadClusterArrayGFX950(name.encode(), buf.ctypes.data_as(C.c_void_p), cap)
+        buf = np.empty(self._size(name), dt)
+        n = lib().downloadClusterArrayGFX950(name.encode(), buf.ctypes.data_as(C.c_void_p),
+                                             buf.size)
         if n < 0:
             raise RuntimeError("download %s failed (%d): %s" % (name, n, status()[1]))
-        return buf[:n].copy()
+        return buf[:n]
 
     def set(self, name, arr):
         """Overwrites a device array from host (slot_x, slot_v)."""

@@ -1,5 +1,7 @@
 """GPU paths of the cluster-pair kernels that are chosen by size, precision and list type, against
 the CPU oracle and against the separate calls they replace."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -66,4 +68,56 @@ def test_precision_change_between_runs_keeps_one_trajectory():
         assert np.linalg.norm(f32 - f64) < 1e-6 * np.linalg.norm(f64)
     finally:
         P.lib().setClusterPrecisionGFX950(0, 0)
+        sim.close()
+
+
+class _AtomHead(C.Structure):
+    """The leading fields of the cluster-pair Atom (include/mdbench_cp.h)."""
+    _fields_ = [(n, C.c_int) for n in ("Natoms", "Nlocal", "Nghost", "Nmax", "Nclusters_local",
+                                       "Nclusters_ghost", "Nclusters_max", "NmaxGhost", "ncj")] + \
+               [(n, C.POINTER(C.c_double)) for n in ("x", "y", "z", "vx", "vy", "vz")] + \
+               [("border_map", C.POINTER(C.c_int)), ("type", C.POINTER(C.c_int))]
+
+
+@pytest.mark.parametrize("nx", [5, 36])
+def test_atoms_to_and_from_the_device(nx):
+    """Small copies and copies of many chunks (186,624 atoms: 4.5 MB of positions): the arrays
+    arrive whole, and the host struct follows the atoms it was given."""
+    P = product()
+    L = P.lib()
+    sim = P.CPSim(nx=nx, ny=nx, nz=nx, ntimes=0)
+    try:
+        x, v, t = P.create_lattice(nx=nx, ny=nx, nz=nx)
+        n = t.size
+        rng = np.random.default_rng(nx)
+        x = np.clip(x + rng.uniform(0, 0.1, 3 * n), 0.0, nx * (4 / 0.8442) ** (1 / 3) - 1e-6)
+        v = v + rng.standard_normal(3 * n)
+        t = rng.integers(0, 4, n).astype(np.int32)
+        sim.set_atoms(x, v, t)
+        head = _AtomHead.from_address(sim.atom_p)
+
+        def host():
+            g = lambda p, k: np.ctypeslib.as_array(p, (k,))  # noqa: E731
+            return (g(head.x, 3 * n), np.stack([g(head.vx, n), g(head.vy, n), g(head.vz, n)], 1),
+                    g(head.type, n))
+
+        def device():
+            return sim.get("atoms_x"), sim.get("atoms_v").reshape(-1, 3), sim.get("atoms_type")
+
+        want = (x, v.reshape(-1, 3), t)
+        for got in (device(), host()):
+            for a, b in zip(got, want):
+                np.testing.assert_array_equal(a, b)
+        for p, k in ((head.x, 3 * n), (head.vx, n), (head.vy, n), (head.vz, n), (head.type, n)):
+            np.ctypeslib.as_array(p, (k,))[:] = 0
+        L.copyAtomsFromClusterGFX950Device(C.c_void_p(sim.atom_p))
+        for a, b in zip(host(), want):
+            np.testing.assert_array_equal(a, b)
+        np.ctypeslib.as_array(head.vy, (n,))[:] += 1.5
+        np.ctypeslib.as_array(head.type, (n,))[:] = t[::-1]
+        L.copyAtomsToClusterGFX950Device(C.c_void_p(sim.atom_p))
+        want = (x, v.reshape(-1, 3) + [0.0, 1.5, 0.0], t[::-1])
+        for a, b in zip(device(), want):
+            np.testing.assert_array_equal(a, b)
+    finally:
         sim.close()
