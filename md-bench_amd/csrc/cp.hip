@@ -54,6 +54,7 @@ constexpr int BLOCK       = 256;
 constexpr int MAX_DEVICES = 64;
 double* g_scratch[MAX_DEVICES];  // &scratch on each device, resolved once per device
 constexpr int MAXT2       = 64;   // ntypes <= 8
+constexpr int ONE_NCI     = 12000; // i-clusters up to which a wavefront takes one (see k_cp_force_f32_full)
 constexpr int BIN_CAP     = 2048; // atoms per 2D column handled in LDS
 constexpr int JBIN_CAP    = 1024; // j-clusters per column handled in LDS
 constexpr double PAD_BASE = 1.0e12, PAD_STEP = 1.0e3;
@@ -122,6 +123,7 @@ struct CPState {
     double* d_sxn   = nullptr;
     size_t cap_sxn  = 0;
     bool sxn_valid  = false;  // padding, dummy and ghost slots of d_sxn match d_sx
+    bool ghosts_current = false;  // the last call was a force call that moved atoms and ghosts
     bool sxn_recs   = false;  // and those of d_srn match d_sr (FP32 kernels)
     // FP32 j-records of d_sx and d_sxn (make_rec), for the FP32 full-list kernel
     float4 *d_sr = nullptr, *d_srn = nullptr;
@@ -1411,6 +1413,14 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64(int nci, int ncj, int nt
     if (EV) ev_store(e, w, ev);
 }
 
+// What a force kernel that integrates needs to write its atoms' ghost images too.
+struct GhostOut {
+    const int* cnt;  // images of each j-cluster, their first ghost, and the shifts; cnt null: none
+    const int* off;
+    const int* pbc;
+    double prd[3];
+};
+
 // Full lists of i-clusters of four, the same arithmetic and the same order of sums, bit for bit:
 // per i-atom and list entry the N pair forces in order, then the entries in list order.  One
 // wavefront per i-cluster: lane (e, a) takes i-atom a and entry e of a round of 16, so the pairs
@@ -1427,7 +1437,7 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64_full(int nci, int ntypes
     const double* __restrict__ sx, const int* __restrict__ st, const int* __restrict__ nb,
     const int* __restrict__ numneigh, const int* __restrict__ ci_natoms, int maxneighs,
     double* __restrict__ f, double* __restrict__ ev, double* __restrict__ v, double dtforce,
-    double* __restrict__ xn, double dt)
+    double* __restrict__ xn, double dt, int ncj, GhostOut gh)
 {
     constexpr int ROW = 13;  // doubles per entry: 12 sums, one apart so that entries spread
     __shared__ double s_sum[BLOCK / 64][16 * ROW];
@@ -1525,9 +1535,26 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64_full(int nci, int ntypes
             double vv = v0 + dtforce * tot;
             if (xn) {
                 vv     = vv + dtforce * tot;
-                xn[t3] = x0 + dt * vv;
+                x0     = x0 + dt * vv;
+                xn[t3] = x0;
             }
             v[t3] = vv;
+        }
+    }
+    if (xn && gh.cnt) {
+        // small systems: the cluster's ghost images too (k_cp_ghost_update's operations), five
+        // images of 12 coordinates at a time
+        const int cjo = ci * 4 / N, ng = gh.cnt[cjo], g0 = gh.off[cjo];
+        if (ng > 0) {
+            const int c = lane % 12, d = c % 3;
+            const double q = __shfl(x0, c, 64);
+            const int na   = __shfl(nat, 0, 64);
+            if (lane < 60 && c / 3 < na)
+                for (int m = lane / 12; m < ng; m += 5) {
+                    const int g = g0 + m;
+                    xn[3 * ((size_t)(ncj + g) * N + (ci * 4 - cjo * N)) + c] =
+                        q + gh.pbc[3 * g + d] * gh.prd[d];
+                }
         }
     }
     if (EV) ev_store(ee, ww, ev);
@@ -1798,16 +1825,30 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f32(int nci, int ncj, int du
 //   byte.
 // The one-type variant is held to 80 VGPRs, six wavefronts per SIMD, the type-table variant to
 // 96, five, both without spills; the energy and compensated variants keep their register count.
-template <int N, bool EV, bool UNIFORM, bool COMP>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu((COMP || EV) ? 1 : (UNIFORM ? 6 : 5))))
+//
+// ONE (small systems): the whole wavefront works on one i-cluster, 64 / N j-clusters of its list
+// per iteration, in blocks of one wavefront, and adds the four rows' sums at the end.  With four
+// i-clusters a wavefront, a small system is a few wavefronts that each walk a whole list (15
+// iterations of 16 entries' records); with one it is four times as many with four iterations
+// each.  Its tail also writes the cluster's ghost images' positions and records (gh), which a
+// launch of its own does otherwise (k_cp_ghost_update).  us per step, four against one (the
+// line lies at 12000 i-clusters):
+//   i-clusters      216         1728         8000        13824        32768
+//   4x4       11.4 / 5.7  12.1 / 6.7  14.3 / 12.6  17.0 / 17.1  25.8 / 32.4
+//   4x8       13.0 / 5.8  13.3 / 6.7  14.6 / 12.8  18.7 / 17.9  29.1 / 34.5
+//   mixture   15.6 / 6.9  15.9 / 8.2  19.4 / 15.8  22.8 / 22.3  40.6 / 42.7
+struct NoGhosts {};
+template <int N, bool EV, bool UNIFORM, bool COMP, bool ONE>
+__global__ void __launch_bounds__(ONE ? 64 : BLOCK) __attribute__((amdgpu_waves_per_eu((COMP || EV || ONE) ? 1 : (UNIFORM ? 6 : 5))))
 k_cp_force_f32_full(int nci, int ncj, int dummy_cj,
     int ntypes, Tab32 tab, const double* __restrict__ sx, const float4* __restrict__ sr,
     const int* __restrict__ st, const int* __restrict__ nb, const int* __restrict__ numneigh,
     const int* __restrict__ ci_natoms, const double* __restrict__ ci_bbox, RecGrid rg,
     int maxneighs, float* __restrict__ f, double* __restrict__ ev, double* __restrict__ v,
     double dtforce, double* __restrict__ xn, float4* __restrict__ rn, double dt,
-    int* __restrict__ status)
+    int* __restrict__ status, std::conditional_t<ONE, GhostOut, NoGhosts> gh)
 {
+    constexpr int WPB = ONE ? 1 : BLOCK / 64;  // wavefronts per block
     constexpr int CPG    = 16 / N;  // j-clusters per group per iteration
     constexpr bool SPLIT = !UNIFORM;
     __shared__ float s_tab[4][MAXT2];
@@ -1830,12 +1871,12 @@ k_cp_force_f32_full(int nci, int ncj, int dummy_cj,
     // XCD-aware block order, as in k_cp_force_f32 (the grid is a multiple of 8 blocks)
     const int per  = gridDim.x >> 3;
     const int lb   = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    const int wv   = __builtin_amdgcn_readfirstlane(lb * (BLOCK / 64) + (threadIdx.x >> 6));
-    if (wv * 4 >= nci) return;
+    const int wv   = __builtin_amdgcn_readfirstlane(lb * WPB + (threadIdx.x >> 6));
+    if (wv * (ONE ? 1 : 4) >= nci) return;
     const int lane = threadIdx.x & 63, grp = lane >> 4, sub = lane & 15;
     const int jc = sub / N, jj = sub % N;
-    const int ci    = wv * 4 + grp;
-    const bool live = ci < nci;
+    const int ci    = ONE ? wv : wv * 4 + grp;
+    const bool live = ONE || ci < nci;
     // the i-cluster's grid cell: that of the centre of its bounding box (as of the list build;
     // an empty cluster's box is inverted and its centre taken at 0)
     float kI[3] = { 0.f, 0.f, 0.f };
@@ -1880,9 +1921,12 @@ k_cp_force_f32_full(int nci, int ncj, int dummy_cj,
     const int nn = live ? numneigh[ci] : 0;
     // the group's atom count, for the tail, loaded here rather than after the loop
     const int nat = live ? ci_natoms[ci] : 0;
-    int nmax     = max(nn, __shfl_xor(nn, 16, 64));
-    nmax         = max(nmax, __shfl_xor(nmax, 32, 64));
-    nmax         = __builtin_amdgcn_readfirstlane(nmax);
+    int nmax     = nn;
+    if (!ONE) {
+        nmax = max(nn, __shfl_xor(nn, 16, 64));
+        nmax = max(nmax, __shfl_xor(nmax, 32, 64));
+    }
+    nmax = __builtin_amdgcn_readfirstlane(nmax);
     const int* lst = nb + (size_t)(live ? ci : 0) * maxneighs;
     const float c12u = tab.c12[0], eps4u = tab.eps4[0], sig6u = tab.sig6[0];
     float nc6u = -tab.c6[0];
@@ -1947,7 +1991,7 @@ k_cp_force_f32_full(int nci, int ncj, int dummy_cj,
                 int lr;
                 asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0"
                              : "=v"(lr));
-                const int cir     = min(wv * 4 + (lr >> 4), nci - 1);
+                const int cir     = ONE ? wv : min(wv * 4 + (lr >> 4), nci - 1);
                 const double* pi  = sx + 3 * (cir * 4 + a);
                 const double* pj  = sx + 3 * (J.off >> 4);  // slot cj * N + jj
                 const double dxd  = pi[0] - pj[0];
@@ -2000,46 +2044,67 @@ k_cp_force_f32_full(int nci, int ncj, int dummy_cj,
     // ones are used (across chunk boundaries too), and every load in the loop is unconditional
     // (see k_cp_force_f32).
     const unsigned jj16 = 16u * (unsigned)jj;
-    const int bp_base   = ((grp << 4) + jc) << 2;
     auto entry = [&](int k) { return 16u * N * (unsigned)(k < nn ? lst[k] : dummy_cj); };
-    unsigned ec = entry(sub), en = entry(16 + sub);
-    // kb: the wave-uniform index of the next iteration's first entry (a multiple of CPG)
-    auto fetch = [&](int kb, JL& J) {
-        const int kk       = kb & 15;
-        const unsigned src = kk ? ec : en;  // kk == 0: the next chunk's first entry
-        const unsigned cjo = (unsigned)__builtin_amdgcn_ds_bpermute(bp_base + (kk << 2), (int)src);
-        J.off = cjo + jj16;
-        J.r   = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(sr) + J.off);
-    };
-    JL A, B;
-    {
-        const unsigned cjo = (unsigned)__builtin_amdgcn_ds_bpermute(bp_base, (int)ec);
-        A.off = cjo + jj16;
-        A.r   = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(sr) + A.off);
-    }
-    int k0 = 0;
-    auto advance = [&]() {  // after the iteration at k0, when k0 + CPG starts a new chunk
-        k0 += CPG;
-        if (!(k0 & 15)) {
-            ec = en;
-            en = entry(k0 + 16 + sub);
+    if constexpr (ONE) {
+        // lane / N: the lane's entry of an iteration; entries two iterations ahead, records one
+        constexpr int STEP = 64 / N;
+        const int kl       = lane / N;
+        auto record        = [&](unsigned ent) {
+            JL J;
+            J.off = ent + jj16;
+            J.r   = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(sr) + J.off);
+            return J;
+        };
+        JL A = record(entry(kl)), B = record(entry(STEP + kl));
+        unsigned ent = entry(2 * STEP + kl);
+        use(A, std::true_type{});
+        for (int k0 = STEP; k0 < nmax; k0 += STEP) {
+            A   = B;
+            B   = record(ent);
+            ent = entry(k0 + 2 * STEP + kl);
+            use(A, std::false_type{});
         }
-    };
-    fetch(CPG, B);
-    use(A, std::true_type{});
-    advance();
-    while (k0 < nmax) {
-        fetch(k0 + CPG, A);
-        use(B, std::false_type{});
+    } else {
+        const int bp_base = ((grp << 4) + jc) << 2;
+        unsigned ec = entry(sub), en = entry(16 + sub);
+        // kb: the wave-uniform index of the next iteration's first entry (a multiple of CPG)
+        auto fetch = [&](int kb, JL& J) {
+            const int kk       = kb & 15;
+            const unsigned src = kk ? ec : en;  // kk == 0: the next chunk's first entry
+            const unsigned cjo = (unsigned)__builtin_amdgcn_ds_bpermute(bp_base + (kk << 2), (int)src);
+            J.off = cjo + jj16;
+            J.r   = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(sr) + J.off);
+        };
+        JL A, B;
+        {
+            const unsigned cjo = (unsigned)__builtin_amdgcn_ds_bpermute(bp_base, (int)ec);
+            A.off = cjo + jj16;
+            A.r   = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(sr) + A.off);
+        }
+        int k0 = 0;
+        auto advance = [&]() {  // after the iteration at k0, when k0 + CPG starts a new chunk
+            k0 += CPG;
+            if (!(k0 & 15)) {
+                ec = en;
+                en = entry(k0 + 16 + sub);
+            }
+        };
+        fetch(CPG, B);
+        use(A, std::true_type{});
         advance();
-        if (k0 >= nmax) break;
-        fetch(k0 + CPG, B);
-        use(A, std::false_type{});
-        advance();
+        while (k0 < nmax) {
+            fetch(k0 + CPG, A);
+            use(B, std::false_type{});
+            advance();
+            if (k0 >= nmax) break;
+            fetch(k0 + CPG, B);
+            use(A, std::false_type{});
+            advance();
+        }
     }
     // the tail's loads of this lane's atom (the lanes sub < 4 of a group), issued before the
     // group sums so that their latency overlaps them
-    const bool tail = sub < 4 && sub < nat;
+    const bool tail = (ONE ? lane : sub) < min(4, nat);
     const int si_t  = (live ? ci : 0) * 4 + sub;
     double px = 0.0, py = 0.0, pz = 0.0, vx0 = 0.0, vy0 = 0.0, vz0 = 0.0;
     if (tail) {
@@ -2071,9 +2136,18 @@ k_cp_force_f32_full(int nci, int ncj, int dummy_cj,
         row_step(std::integral_constant<int, DPP_XOR2>{});
         row_step(std::integral_constant<int, DPP_HALF_MIRROR>{});
         row_step(std::integral_constant<int, DPP_MIRROR>{});
+        if (ONE)
+#pragma unroll
+            for (int o = 16; o < 64; o <<= 1)
+#pragma unroll
+                for (int a = 0; a < 4; a++) {
+                    fx[a] += __shfl_xor(fx[a], o, 64);
+                    fy[a] += __shfl_xor(fy[a], o, 64);
+                    fz[a] += __shfl_xor(fz[a], o, 64);
+                }
     } else {
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) {
+        for (int o = 1; o < (ONE ? 64 : 16); o <<= 1) {
 #pragma unroll
             for (int a = 0; a < 4; a++) {
                 const float ox = __shfl_xor(fx[a], o, 64), oy = __shfl_xor(fy[a], o, 64),
@@ -2116,10 +2190,40 @@ k_cp_force_f32_full(int nci, int ncj, int dummy_cj,
                 xn[3 * si + 1] = nyp;
                 xn[3 * si + 2] = nzp;
                 rn[si]         = make_rec(nxp, nyp, nzp, st[si], rg, status);
+                if constexpr (ONE) {
+                    px = nxp;
+                    py = nyp;
+                    pz = nzp;
+                }
             }
             v[3 * si]     = vx;
             v[3 * si + 1] = vy;
             v[3 * si + 2] = vz;
+        }
+    }
+    if constexpr (ONE) {
+        // the ghost images of the cluster's atoms, by the operations of k_cp_ghost_update: lane
+        // (m, a) takes images m, m + 16, ... and atom a
+        if (xn && gh.cnt) {
+            const int cj = ci * 4 / N, a = lane & 3;
+            const int ng = gh.cnt[cj], g0 = gh.off[cj];
+            if (ng > 0) {  // wave-uniform
+                const double qx = __shfl(px, a, 64), qy = __shfl(py, a, 64), qz = __shfl(pz, a, 64);
+                const int ta = st[ci * 4 + a];
+                for (int m = lane >> 2; m < ng; m += 16) {
+                    const int g = g0 + m;
+                    if (a < nat) {
+                        const int sg   = (ncj + g) * N + (ci * 4 - cj * N) + a;
+                        const double x = qx + gh.pbc[3 * g] * gh.prd[0];
+                        const double y = qy + gh.pbc[3 * g + 1] * gh.prd[1];
+                        const double z = qz + gh.pbc[3 * g + 2] * gh.prd[2];
+                        xn[3 * sg]     = x;
+                        xn[3 * sg + 1] = y;
+                        xn[3 * sg + 2] = z;
+                        rn[sg]         = make_rec(x, y, z, ta, rg, status);
+                    }
+                }
+            }
         }
     }
     if (EV) ev_store(e, w, ev);
@@ -2799,8 +2903,9 @@ size_t nslots_all() { return ((size_t)C.ncj + C.nghost + 1) * C.N; }
 
 bool ensure_slots(size_t nslot, size_t keep_slots)
 {
-    C.sxn_valid = false;
-    C.rec_valid = false;
+    C.sxn_valid      = false;
+    C.rec_valid      = false;
+    C.ghosts_current = false;
     grow_n(&C.d_sx, &C.cap_sx, 3 * nslot, 3 * keep_slots);
     grow_n(&C.d_st, &C.cap_st, nslot, keep_slots);
     return !failed();
@@ -3555,6 +3660,9 @@ enum { FUSED_FINAL = 1, FUSED_INITIAL = 2 };
 static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
     bool fuse_initial, double* secs);
 
+// For the run loop: the last call was a fused force call that also moved the ghosts.
+int mdg_cp_ghosts_current(void) { return C.ghosts_current; }
+
 double computeForceLJClusterGFX950(Parameter* param, Atom* atom, Neighbor* neighbor, Stats* stats)
 {
     (void)atom;
@@ -3628,6 +3736,10 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
         xn = C.d_sxn;
         rn = recs ? C.d_srn : nullptr;
     }
+    bool ghosts_moved = false;  // this call also writes the next step's ghost positions
+    GhostOut gho      = {};
+    const GhostOut ghost_out{ C.d_gcnt, C.d_goff, C.d_pbc, { param->xprd, param->yprd,
+        param->zprd } };
     TimedRegion tr(F_FORCE_CP);
     if (C.precision == 0 &&
         ((size_t)C.ncj + C.nghost + 1 >= (1u << 24) || nslots_all() * 24 >= (1ull << 32))) {
@@ -3655,10 +3767,12 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
         if (failed()) return 0;
         const int uni = C.uniform ? 1 : 0;
         if (full64 && fuse_final) fused = FUSED_FINAL | (xn ? FUSED_INITIAL : 0);
+        ghosts_moved = full64 && xn && nci <= ONE_NCI;
+        if (ghosts_moved && C.nghost > 0) gho = ghost_out;
 #define MDG_F64C(NN, E, U)                                                                       \
     k_cp_force_f64_full<NN, E, U><<<grid, BLOCK, 0, s>>>(nci, C.ntypes, C.t64, C.d_sx, C.d_st,    \
         C.d_nb, C.d_numneigh, C.d_ci_natoms, C.maxneighs, C.d_sf64, evp,                          \
-        fused ? C.d_sv : nullptr, param->dtforce, xn, param->dt)
+        fused ? C.d_sv : nullptr, param->dtforce, xn, param->dt, C.ncj, gho)
 #define MDG_F64C_N(NN)                                                                           \
     do {                                                                                         \
         if (C.ev_on) {                                                                           \
@@ -3703,6 +3817,15 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
         double* evp    = ev_parts(tiled ? (size_t)C.ntiles * TILE_WAVES
                                         : (size_t)(half ? grid : grid4) * (BLOCK / 64));
         if (failed()) return 0;
+        // small systems: a wavefront per i-cluster, which also moves the ghosts when it integrates
+        const bool one = !half && !C.ev_on && !C.comp && nci <= ONE_NCI;
+        ghosts_moved   = one && xn != nullptr;
+        if (ghosts_moved && C.nghost > 0) gho = ghost_out;
+#define MDG_F32_ONE(NN, U)                                                                       \
+    k_cp_force_f32_full<NN, false, U, false, true><<<(nci + 7) & ~7, 64, 0, s>>>(nci, C.ncj,       \
+        C.dummy_cj, C.ntypes, C.t32, C.d_sx, C.d_sr, C.d_st, C.d_nb, C.d_numneigh,                 \
+        C.d_ci_natoms, C.d_ci_bbox, C.rg, C.maxneighs, C.d_sf32, evp, fuse_v, param->dtforce, xn,  \
+        rn, param->dt, C.d_status + ST_REC_WORD, gho)
 #define MDG_F32(NN, H, E, U, CO)                                                                 \
     do {                                                                                         \
         if (H)                                                                                   \
@@ -3710,10 +3833,10 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
                 C.ntypes, C.t32, C.d_sx, C.d_st, C.d_nb, C.d_numneigh, C.d_ci_natoms,             \
                 C.maxneighs, C.d_sf32, evp);                                                      \
         else                                                                                     \
-            k_cp_force_f32_full<NN, E, U, CO><<<grid4, BLOCK, 0, s>>>(nci, C.ncj, C.dummy_cj,     \
+            k_cp_force_f32_full<NN, E, U, CO, false><<<grid4, BLOCK, 0, s>>>(nci, C.ncj, C.dummy_cj,     \
                 C.ntypes, C.t32, C.d_sx, C.d_sr, C.d_st, C.d_nb, C.d_numneigh, C.d_ci_natoms,     \
                 C.d_ci_bbox, C.rg, C.maxneighs, C.d_sf32, evp, fuse_v, param->dtforce, xn,       \
-                rn, param->dt, C.d_status + ST_REC_WORD);                                        \
+                rn, param->dt, C.d_status + ST_REC_WORD, NoGhosts{});                            \
     } while (0)
 #define MDG_F32_U(NN, H, E)                                                                      \
     do {                                                                                         \
@@ -3760,8 +3883,15 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
             else MDG_HT_N(8);
 #undef MDG_HT_N
 #undef MDG_HT
+        } else if (one && C.N == 4) {
+            if (C.uniform) MDG_F32_ONE(4, true);
+            else MDG_F32_ONE(4, false);
+        } else if (one) {
+            if (C.uniform) MDG_F32_ONE(8, true);
+            else MDG_F32_ONE(8, false);
         } else if (C.N == 4) MDG_F32_N(4);
         else MDG_F32_N(8);
+#undef MDG_F32_ONE
 #undef MDG_F32_N
 #undef MDG_F32_U
 #undef MDG_F32
@@ -3782,6 +3912,7 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
             C.rec_valid = false;
         }
     }
+    C.ghosts_current = (fused & FUSED_INITIAL) && ghosts_moved && !failed();
     *secs = wtime() - t0;
     return fused;
 }
@@ -3797,7 +3928,8 @@ void initialIntegrateClusterGFX950(Parameter* param, Atom* atom)
         set_error(E_ARG, "initialIntegrateClusterGFX950 before the first force call");
         return;
     }
-    C.rec_valid = false;  // the records follow at the next FP32 force call
+    C.rec_valid      = false;  // the records follow at the next FP32 force call
+    C.ghosts_current = false;
     if (C.forces_are_f32)
         k_cp_initial<float><<<blocks_for(n3, BLOCK), BLOCK, 0, stream()>>>(n3, C.M, C.d_ci_natoms,
             C.d_sx, C.d_sv, C.d_sf32, param->dt, param->dtforce);
@@ -3905,7 +4037,7 @@ long long uploadClusterArrayGFX950(const char* name, const void* in, long long n
     else if (!strcmp(name, "slot_v")) { dst = C.d_sv; avail = 3LL * C.nci * C.M; }
     if (!dst) return -1;
     if (n > avail || n < 0) return -2;
-    if (dst == C.d_sx) C.sxn_valid = C.rec_valid = false;
+    if (dst == C.d_sx) C.sxn_valid = C.rec_valid = C.ghosts_current = false;
     MDG_HIP(hipMemcpyAsync(dst, in, (size_t)n * sizeof(double), hipMemcpyHostToDevice, stream()));
     MDG_HIP(hipStreamSynchronize(stream()));
     return failed() ? -3 : n;

@@ -16,6 +16,8 @@
 int mdgfx950Status(void);
 const char* mdgfx950StatusMessage(void);
 void mdgfx950SetStrict(int strict);
+/* csrc/cp.hip: 1 after a fused force call that also wrote the ghosts' new positions */
+int mdg_cp_ghosts_current(void);
 /* csrc/cp.hip: copyAtomsToClusterGFX950Device from x and v AoS */
 void mdg_cp_upload_atoms(const double* x, const double* v, const int* type, int n);
 
@@ -222,7 +224,8 @@ int mdbCPRun(mdb_cp* s, int nsteps, double* ksum)
         if (!integrated) initialIntegrateClusterGFX950(p, a);
         if ((n + 1) % p->reneigh_every) {
             if (!((n + 1) % p->prune_every)) pruneNeighborClusterGFX950(p, a, nb);
-            updatePbcClusterGFX950(a, p, false);
+            /* (a small system's fused force call wrote the ghosts with the atoms) */
+            if (!(integrated && mdg_cp_ghosts_current())) updatePbcClusterGFX950(a, p, false);
         } else {
             updateSingleAtomsGFX950(p, a);
             updateAtomsPbcClusterGFX950(a, p, false);

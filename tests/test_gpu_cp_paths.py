@@ -51,6 +51,34 @@ def test_fp64_fused_run_equals_traced_run(N, mixture):
         np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("mixture", [0, 1], ids=["lj", "ka"])
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("N", [4, 8])
+@pytest.mark.parametrize("nx", [4, 22, 23])
+def test_fused_run_equals_traced_run_around_the_small_size(nx, N, precision, mixture):
+    """Up to 12000 i-clusters (22^3 cells) a wavefront takes one i-cluster and the fused call
+    moves the ghosts; above, four, and a launch of their own does.  Either way a traced run,
+    which integrates and moves ghosts separately, gives the same bits, ghosts included."""
+    out = []
+    for trace in (False, True):
+        sim = product().CPSim(nx=nx, ny=nx, nz=nx, cluster_m=4, cluster_n=N, ntimes=0,
+                              precision=precision, reneigh_every=6, **(MIX if mixture else {}))
+        try:
+            sim.run(8, trace=trace)
+            sim.run(5, trace=trace)
+            i = sim.info()
+            cjn = sim.get("cj_natoms")
+            slots = (np.arange(cjn.size)[:, None] * N + np.arange(N))[np.arange(N) < cjn[:, None]]
+            live = _live_slots(sim.get("ci_natoms"), 4)
+            out.append([sim.get("slot_x").reshape(-1, 3)[slots]] +
+                       [sim.get(k).reshape(-1, 3)[live] for k in ("slot_v", "slot_f")])
+            assert (i["nci"] <= 12000) == (nx < 23)
+        finally:
+            sim.close()
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_precision_change_between_runs_keeps_one_trajectory():
     """FP32 and FP64 calls in turn on one simulation share the position buffers: the FP64 forces
     after an FP32 stretch equal those of a simulation set to the same atoms."""
