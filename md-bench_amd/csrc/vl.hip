@@ -23,6 +23,12 @@ namespace {
 
 constexpr int BLOCK     = 256;
 constexpr int MAXTYPES2 = 64;  // ntypes <= 8
+// LJ passes of full lists stage their neighbours' positions in LDS (k_force_lj_staged, k_stage_build)
+// above STAGE_MIN atoms, where the list is kept for STAGE_USES force calls or more: at 1.05 M atoms a
+// call gains 60 us and the tables cost 300 us per list; whole steps with a list per 20 measured 323 us
+// without and 277 with, at 702 k atoms 218 and 187, at 630 k 184 and 173, at 520 k (the list just fits
+// the last-level cache) 136 and 146.
+constexpr int STAGE_MIN = 600000, STAGE_USES = 8, STAGE_RETRY = 32;
 constexpr int FUSE_GHOSTS_EAM = 300000;  // EAM systems up to this size move ghosts in the force call
 constexpr int FAST_LPA  = 4;   // lanes per atom in the fast force kernels of large systems
 
@@ -91,6 +97,15 @@ struct State {
     bool ghosts_current = false;  // the last call moved no local atom or moved its ghosts with it
     // neighbour list capacity (elements)
     size_t cap_nb = 0, cap_numneigh = 0;
+    // staged neighbour positions (k_stage_build): per block of atoms the atoms its lists name, and
+    // each list entry's place among them; stage_nlocal atoms of stage_max entries (-1: none)
+    int *d_stage = nullptr, *d_stage_n = nullptr;
+    unsigned short* d_hint = nullptr;
+    size_t cap_stage = 0, cap_stage_n = 0, cap_hint = 0;
+    int stage_nlocal = -1, stage_max = 0;
+    // whether tables pay is judged by the last lists (speed only, the results are the same): the force
+    // calls of the last two, overflowing blocks (a running count, see k_stage_build), lists to leave out
+    int list_uses = -1, last_uses = -1, stage_over = 0, stage_skip = 0;
     // EAM
     double* d_fp = nullptr;
     size_t cap_fp = 0;
@@ -101,7 +116,7 @@ struct State {
     double* d_red = nullptr;
     size_t cap_red = 0;
     double* d_ev = nullptr;
-    int* d_status = nullptr;  // [0] flags, [1] max numneigh, [2] scan total
+    int* d_status = nullptr;  // [0] flags, [1] max numneigh, [2] scan total, [3] staging overflows
     int* h_status = nullptr;  // pinned
     double* h_red = nullptr;  // pinned
     bool ev_on = false;
@@ -826,6 +841,201 @@ __global__ void __launch_bounds__(BLOCK) k_force_lj(int nlocal, const double* __
     }
 }
 
+// ---------------------------------------------------------------- staged neighbour positions
+// A large system's force pass is bound by the texture path's address rate: two loads of 64 different
+// lines for the positions of 64 pairs.  So a block of STAGE_T threads takes STAGE_A consecutive atoms
+// (of one region of the box in the lattice's order), reads the positions of all the distinct atoms
+// that its lists name into LDS once, and its pairs read them there.  Which atoms those are, and each
+// list entry's place among them, is worked out when the list is built (k_stage_build).  Both are
+// only hints: a pair uses the staged position only if the staged atom is the one its list entry
+// names, and loads it from memory otherwise (a list written by someone else, a region with more than
+// STAGE_CAP distinct neighbours).  1.05 M atoms: 276 us per call with the positions gathered, 217
+// staged (half the VALU's time, 60 % of the texture path's, the list and hints at 2.2 TB/s).  The two
+// blocks that a CU's LDS and waves hold set STAGE_CAP; a 256-atom lattice block names 1300 - 1700.
+constexpr int STAGE_T = 1024, STAGE_A = 256, STAGE_CAP = 2000, STAGE_LOG = 10;
+
+// tab: STAGE_CAP atoms per block, tab_n: how many (0: too many), hint[k * nlocal + i]: the place.
+// Atoms are taken by pages of 64: a block's neighbours lie in a hundred or two of them, found in a
+// small hash table; a page's members are bits of a word, so that a list entry is entered with an OR
+// and an atom's place is its page's first plus the members below it (pages in table order).  LDS
+// atomics bound it: 285 - 305 us at 1.05 M atoms (800 us for the list itself), 322 where every entry
+// is an OR without the read before it.
+__global__ void __launch_bounds__(STAGE_T) k_stage_build(int nlocal,
+    const int* __restrict__ neighbors, const int* __restrict__ numneigh, int maxneighs,
+    int* __restrict__ tab, int* __restrict__ tab_n, unsigned short* __restrict__ hint,
+    int* __restrict__ overflows)
+{
+    constexpr int SLOTS = STAGE_T, LPA = STAGE_T / STAGE_A, PROBES = 16;
+    __shared__ int s_page[SLOTS];
+    __shared__ unsigned long long s_bits[SLOTS];
+    __shared__ unsigned short s_first[SLOTS];
+    __shared__ int s_scan[33], s_bad;
+    s_page[threadIdx.x] = -1;
+    s_bits[threadIdx.x] = 0ull;
+    if (threadIdx.x == 0) s_bad = 0;
+    __syncthreads();
+    const int i    = blockIdx.x * STAGE_A + threadIdx.x / LPA;
+    const int lane = threadIdx.x % LPA;
+    const int nn   = i < nlocal ? min(numneigh[i], maxneighs) : 0;
+    auto start     = [](int p) { return ((unsigned)p * 2654435761u) >> (32 - STAGE_LOG); };
+    auto enter = [&](int j) {
+        const int p = j >> 6;
+        unsigned h  = start(p);
+        int left    = PROBES;
+        for (; left; left--, h = (h + 1) & (SLOTS - 1)) {
+            int key = __hip_atomic_load(&s_page[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (key == -1) {
+                key = atomicCAS(&s_page[h], -1, p);
+                if (key == -1) key = p;
+            }
+            if (key == p) break;
+        }
+        // (most entries name an atom that is there already: a read instead of an atomic)
+        const unsigned long long bit = 1ull << (j & 63);
+        if (!left) s_bad = 1;
+        else if (!(__hip_atomic_load(&s_bits[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & bit))
+            atomicOr(&s_bits[h], bit);
+    };
+    for (int k = lane; k < nn; k += LPA)
+        enter(neighbors[(size_t)k * nlocal + i]);
+    __syncthreads();
+    unsigned long long bits = s_bits[threadIdx.x];
+    int n;
+    int at = block_excl_scan(__popcll(bits), s_scan, &n);
+    const bool ok = n <= STAGE_CAP && !s_bad;
+    if (threadIdx.x == 0) {
+        tab_n[blockIdx.x] = ok ? n : 0;
+        if (!ok) atomicAdd(overflows, 1);
+    }
+    if (!ok) return;
+    s_first[threadIdx.x] = (unsigned short)at;
+    const int page = s_page[threadIdx.x];
+    for (; bits; bits &= bits - 1)
+        tab[(size_t)blockIdx.x * STAGE_CAP + at++] = page * 64 + __ffsll((long long)bits) - 1;
+    __syncthreads();
+    auto place = [&](int j) {
+        const int p = j >> 6;
+        unsigned h  = start(p);
+        for (int left = PROBES; left > 1 && s_page[h] != p; left--)
+            h = (h + 1) & (SLOTS - 1);
+        return (unsigned short)(s_first[h] + __popcll(s_bits[h] & ((1ull << (j & 63)) - 1)));
+    };
+    for (int k = lane; k < nn; k += LPA)
+        hint[(size_t)k * nlocal + i] = place(neighbors[(size_t)k * nlocal + i]);
+}
+
+// LJ, full lists, fast, without energies: the pairs, their order and arithmetic are those of
+// k_force_lj with four lanes per atom.
+template <bool UNIFORM>
+__global__ void __launch_bounds__(STAGE_T) k_force_lj_staged(int nlocal, int nall, int nblocks,
+    const double* __restrict__ x, const int* __restrict__ type, int ntypes, Tables tab,
+    const int* __restrict__ neighbors, const int* __restrict__ numneigh, int maxhint,
+    const int* __restrict__ stage, const int* __restrict__ stage_n,
+    const unsigned short* __restrict__ hint, double* __restrict__ f, Fuse fu)
+{
+    constexpr int LPA = STAGE_T / STAGE_A;
+    __shared__ double s_pos[3 * STAGE_CAP];
+    __shared__ int s_key[STAGE_CAP];
+    __shared__ unsigned char s_type[UNIFORM ? 1 : STAGE_CAP];
+    __shared__ double s_tab[3][UNIFORM ? 1 : MAXTYPES2];
+    // blocks of one XCD adjacent (the grid is a multiple of 8)
+    const int per = gridDim.x >> 3;
+    const int b   = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (b >= nblocks) return;
+    if (!UNIFORM)
+        for (int k = threadIdx.x; k < ntypes * ntypes; k += STAGE_T) {
+            s_tab[0][k] = tab.eps[k];
+            s_tab[1][k] = tab.sig6[k];
+            s_tab[2][k] = tab.cutf[k];
+        }
+    const int ns = stage_n[b];
+    if (threadIdx.x == 0 && ns == 0) s_key[0] = -1;
+    for (int k = threadIdx.x; k < ns; k += STAGE_T) {
+        const int j = stage[(size_t)b * STAGE_CAP + k];
+        const bool in = (unsigned)j < (unsigned)nall;
+        s_key[k]      = in ? j : -1;
+        if (in) {
+            s_pos[3 * k]     = x[3 * j];
+            s_pos[3 * k + 1] = x[3 * j + 1];
+            s_pos[3 * k + 2] = x[3 * j + 2];
+            if (!UNIFORM) s_type[k] = (unsigned char)type[j];
+        }
+    }
+    const int i    = b * STAGE_A + threadIdx.x / LPA;
+    const int lane = threadIdx.x % LPA;
+    const bool act = i < nlocal;
+    double fix = 0, fiy = 0, fiz = 0;
+    double v0[3] = {}, x0[3] = {};
+    int ng = 0, g0 = 0, nn = 0, ti = 0;
+    if (act) {
+        if (fu.v && (lane == 0 || fu.gcnt)) fused_load<true>(fu, i, v0, &ng, &g0);
+        x0[0] = x[3 * i];
+        x0[1] = x[3 * i + 1];
+        x0[2] = x[3 * i + 2];
+        nn    = numneigh[i];
+        if (!UNIFORM) ti = type[i] * ntypes;
+    }
+    __syncthreads();
+    // entries and hints two iterations ahead
+    const size_t step = (size_t)LPA * nlocal;
+    const int* lst             = neighbors + (size_t)lane * nlocal + i;
+    const unsigned short* hnt  = hint + (size_t)lane * nlocal + i;
+    const int nh               = ns ? min(nn, maxhint) : 0;
+    auto next = [&](int k, int* j, int* h) {
+        if (k < nn) *j = *lst;
+        *h = 0;
+        if (k < nh) *h = *hnt;
+        lst += step;
+        hnt += step;
+    };
+    int j1 = 0, h1 = 0, j2 = 0, h2 = 0;
+    next(lane, &j1, &h1);
+    next(lane + LPA, &j2, &h2);
+    for (int k = lane; k < nn; k += LPA) {
+        const int j = j1;
+        int h       = h1;
+        j1          = j2;
+        h1          = h2;
+        next(k + 2 * LPA, &j2, &h2);
+        h = h < ns ? h : 0;
+        double xj = s_pos[3 * h], yj = s_pos[3 * h + 1], zj = s_pos[3 * h + 2];
+        int tj = 0;
+        if (!UNIFORM) tj = s_type[h];
+        // (kept as LDS reads: the compiler would merge them with the loads below into flat loads,
+        // which take the texture path again)
+        asm volatile("" : "+v"(xj), "+v"(yj), "+v"(zj));
+        if (__builtin_expect(s_key[h] != j, 0)) {
+            xj = x[3 * j];
+            yj = x[3 * j + 1];
+            zj = x[3 * j + 2];
+            if (!UNIFORM) tj = type[j];
+        }
+        const double dx = x0[0] - xj, dy = x0[1] - yj, dz = x0[2] - zj;
+        const double rsq  = fma(dx, dx, fma(dy, dy, dz * dz));
+        const double cutf = UNIFORM ? tab.cutf[0] : s_tab[2][ti + tj];
+        if (rsq < cutf) {
+            const double eps   = UNIFORM ? tab.eps[0] : s_tab[0][ti + tj];
+            const double sig6  = UNIFORM ? tab.sig6[0] : s_tab[1][ti + tj];
+            const double sr2   = 1.0 / rsq;
+            const double sr6   = sr2 * sr2 * sr2 * sig6;
+            const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
+            fix                = fma(dx, force, fix);
+            fiy                = fma(dy, force, fiy);
+            fiz                = fma(dz, force, fiz);
+        }
+    }
+    fix = group_sum<LPA>(fix);
+    fiy = group_sum<LPA>(fiy);
+    fiz = group_sum<LPA>(fiz);
+    if (act && lane == 0) {
+        f[3 * i]     = fix;
+        f[3 * i + 1] = fiy;
+        f[3 * i + 2] = fiz;
+    }
+    if (fu.v && act && (lane == 0 || fu.gcnt))
+        fused_integrate<LPA, true>(fu, nlocal, i, lane, v0, x0, ng, g0, fix, fiy, fiz);
+}
+
 // Half lists, fast: a block takes HALF_T / LPA consecutive atoms (of one region of the box, in the
 // lattice's or the bin sort's order) and adds the forces on their listed neighbours in LDS, those
 // of its own atoms in place, those of other atoms in a hash table keyed by the atom, and only then
@@ -1313,6 +1523,33 @@ bool ensure_status()
     return !failed();
 }
 
+void stage_release()
+{
+    dfree(S.d_stage);
+    dfree(S.d_stage_n);
+    dfree(S.d_hint);
+    S.d_stage = S.d_stage_n = nullptr;
+    S.d_hint    = nullptr;
+    S.cap_stage = S.cap_stage_n = S.cap_hint = 0;
+    S.stage_nlocal = -1;
+}
+
+// Room for n elements, or false: a system that fits the device without the tables runs without them.
+template <typename T>
+bool stage_room(T** p, size_t* cap, size_t n)
+{
+    if (n <= *cap) return true;
+    dfree(*p);
+    *cap = 0;
+    if (hipMalloc((void**)p, n * sizeof(T)) != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+        return false;
+    }
+    *cap = n;
+    return true;
+}
+
 void read_status()
 {
     MDG_HIP(hipMemcpyAsync(S.h_status, S.d_status, 16 * sizeof(int), hipMemcpyDeviceToHost,
@@ -1398,7 +1635,9 @@ void initDeviceGFX950(Parameter* param, Atom* atom, Neighbor* neighbor)
     grow_n(&dn->numneigh, &S.cap_numneigh, (size_t)atom->Nlocal, 0);
     S.binned = false;
     S.ready  = true;
-    S.gmap_nlocal = -1;
+    S.gmap_nlocal  = -1;
+    S.stage_nlocal = S.list_uses = S.last_uses = -1;
+    S.stage_skip   = 0;
     copyDataToGFX950Device(param, atom);
 }
 
@@ -1440,6 +1679,7 @@ void freeDeviceGFX950(Atom* atom, Neighbor* neighbor)
     dfree(S.d_gcnt);
     dfree(S.d_goff);
     dfree(S.d_pbc);
+    stage_release();
     dfree(S.d_fp);
     dfree(S.d_rhor);
     dfree(S.d_frho);
@@ -1669,6 +1909,41 @@ void sortAtomGFX950(Atom* atom)
     S.binned = false;  // the bins name the old indices
 }
 
+// The staging tables of a full list just built (after a wait for the stream), where they pay: not
+// for lists that are soon replaced, and not while most blocks' neighbours do not fit (atoms in the
+// bin sort's order, rows of one bin's width: 321 us per step with the tables tried on every list,
+// 311 without); those try again after STAGE_RETRY lists.
+static void stage_build(int nlocal, Neighbor* neighbor)
+{
+    const int over = S.h_status[3] - S.stage_over;
+    const int uses = S.last_uses < 0 ? STAGE_USES : std::max(S.list_uses, S.last_uses);
+    const int nb   = (nlocal + STAGE_A - 1) / STAGE_A;
+    S.stage_over   = S.h_status[3];
+    S.last_uses    = S.list_uses;
+    S.list_uses    = 0;
+    if (S.stage_nlocal == nlocal && over > nb / 2) S.stage_skip = STAGE_RETRY;
+    S.stage_nlocal = -1;
+    if (neighbor->half_neigh || strict_mode() || nlocal <= STAGE_MIN || S.d_rhor) return;
+    if (uses < STAGE_USES) return;
+    if (S.stage_skip > 0) {
+        S.stage_skip--;
+        return;
+    }
+    const int mn = neighbor->maxneighs;
+    if (!stage_room(&S.d_stage, &S.cap_stage, (size_t)nb * STAGE_CAP) ||
+        !stage_room(&S.d_stage_n, &S.cap_stage_n, (size_t)nb) ||
+        !stage_room(&S.d_hint, &S.cap_hint, (size_t)nlocal * mn)) {
+        stage_release();
+        return;
+    }
+    TimedRegion tr(F_NEIGHBOR);
+    k_stage_build<<<nb, STAGE_T, 0, stream()>>>(nlocal, neighbor->d_neighbor.neighbors,
+        neighbor->d_neighbor.numneigh, mn, S.d_stage, S.d_stage_n, S.d_hint, S.d_status + 3);
+    MDG_LAUNCH_CHECK("stage_build");
+    S.stage_nlocal = nlocal;
+    S.stage_max    = mn;
+}
+
 void buildNeighborGFX950(Atom* atom, Neighbor* neighbor)
 {
     if (failed() || !S.ready) return;
@@ -1703,9 +1978,13 @@ void buildNeighborGFX950(Atom* atom, Neighbor* neighbor)
             set_error(MDG_ERR_BIN, "an atom lies outside the bin grid (coord2bin out of range)");
             return;
         }
-        if (!(S.h_status[0] & ST_NB_OVERFLOW)) return;
+        if (!(S.h_status[0] & ST_NB_OVERFLOW)) {
+            stage_build(nlocal, neighbor);
+            return;
+        }
         // neighbor.c:336-345: grow to 1.2x the largest count and rebuild
         neighbor->maxneighs = (int)(S.h_status[1] * 1.2) + 1;
+        stage_release();  // room for the list first
     }
     set_error(MDG_ERR_CAPACITY, "neighbour list did not converge");
 }
@@ -1824,6 +2103,7 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
     const int nall   = nlocal + atom->Nghost;
     const bool strict = strict_mode();
     hipStream_t s    = stream();
+    if (S.list_uses >= 0) S.list_uses++;
     if (S.ev_on) fill_f64(S.d_ev, 0.0, 2);
     const int half = neighbor->half_neigh;
     if (half && strict) fill_f64(atom->d_atom.fx, 0.0, 3 * (size_t)nall);
@@ -1869,7 +2149,18 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
                 else if (lanes == 32) MDG_LJ(32, false, false, false);
                 else if (lanes == 16) MDG_LJ(16, false, false, false);
                 else if (lanes == 8) MDG_LJ(8, false, false, false);
-                else MDG_LJ(FAST_LPA, false, false, false);
+                else if (S.stage_nlocal == nlocal) {
+                    const int nb        = (nlocal + STAGE_A - 1) / STAGE_A;
+                    const unsigned grid = ((unsigned)nb + 7) & ~7u;
+#define MDG_LJS(U)                                                                               \
+    k_force_lj_staged<U><<<grid, STAGE_T, 0, s>>>(nlocal, nall, nb, atom->d_atom.x,              \
+        atom->d_atom.type, S.ntypes, S.tab, neighbor->d_neighbor.neighbors,                      \
+        neighbor->d_neighbor.numneigh, S.stage_max, S.d_stage, S.d_stage_n, S.d_hint,            \
+        atom->d_atom.fx, fu)
+                    if (S.uniform) MDG_LJS(true);
+                    else MDG_LJS(false);
+#undef MDG_LJS
+                } else MDG_LJ(FAST_LPA, false, false, false);
             }
         }
 #undef MDG_LJH

@@ -59,6 +59,27 @@ def test_full_list_forces_at_each_lane_count(dims, mixed):
 
 
 @pytest.mark.parametrize("mixed", [0, 1], ids=["uniform", "types"])
+@pytest.mark.parametrize("resort", [0, 10], ids=["lattice", "sorted"])
+def test_staged_positions_of_large_full_lists(resort, mixed):
+    """The size from which a block's neighbours are staged in LDS, with a last block of 92 atoms;
+    in the bin sort's order most blocks name more atoms than the stage holds."""
+    P = product()
+    print(resort, mixed, flush=True)
+    sim = P.VLSim(nx=53, ny=57, nz=51, reneigh_every=10, resort_every=resort,
+                  **(MIXED if mixed else {}))
+    try:
+        sim.run(13)
+        st = sim.state()
+        assert st["nlocal"] == 616284
+        want, _, _ = _oracle_force(sim, st, 0)
+        assert np.linalg.norm(want) > 10.0
+        assert np.linalg.norm(st["f"] - want) < FORCE_RTOL * np.linalg.norm(want)
+        _ghosts_follow_owners(sim, st)
+    finally:
+        sim.close()
+
+
+@pytest.mark.parametrize("mixed", [0, 1], ids=["uniform", "types"])
 @pytest.mark.parametrize("dims", [(4, 4, 4), (13, 13, 15), (15, 14, 16), (21, 17, 18),
                                   (29, 27, 27)], ids=str)
 def test_half_list_forces_at_each_lane_count(dims, mixed):
