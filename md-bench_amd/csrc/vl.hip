@@ -1280,6 +1280,17 @@ __global__ void k_ghost_copy(int nlocal, int nghost, double* __restrict__ a,
     a[nlocal + g] = a[border_map[g]];
 }
 
+// The ghosts' rows (position, F' of the owner) of the table passes
+__global__ void k_ghost_rows(int nlocal, int nghost, const double* __restrict__ x,
+    double2* __restrict__ xf, const int* __restrict__ border_map)
+{
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= nghost) return;
+    const size_t i = (size_t)nlocal + g;
+    xf[2 * i]      = make_double2(x[3 * i], x[3 * i + 1]);
+    xf[2 * i + 1]  = make_double2(x[3 * i + 2], xf[2 * (size_t)border_map[g] + 1].y);
+}
+
 template <int LPA, bool STRICT, bool EV>
 __global__ void __launch_bounds__(BLOCK) k_eam_force(int nlocal, const double* __restrict__ x,
     const int* __restrict__ neighbors, const int* __restrict__ numneigh, double cutforcesq,
@@ -1361,6 +1372,12 @@ __global__ void __launch_bounds__(BLOCK) k_eam_force(int nlocal, const double* _
 // the blocks are persistent: TAB_BLOCK threads, one block per 64 KB / 160 KB of a CU's LDS,
 // each over a contiguous range of atoms (ranges of one XCD adjacent, as in the cluster-pair
 // kernels).  Operations and their order are those of k_eam_density / k_eam_force.
+// The density pass leaves a row of 32 bytes per atom, its position and F', for the force pass: with
+// one block per CU (4 waves per SIMD) that pass waited for a gather of the position and another of F'
+// per pair.  One aligned row, in one cache line, loaded a pair ahead of its use: 451 -> 345 us at
+// 1.05 M atoms (377 a pair ahead but without the rows), 53 -> 45 at 131 k; the rows cost the density
+// pass 6 us of 255.  The density pass itself gains nothing from loads ahead (281 us): two blocks a CU
+// hide them, and it is bound by the cache lines that its gathers fill.
 constexpr int TAB_BLOCK = 1024;
 constexpr int TAB_NR    = 2000;
 
@@ -1369,7 +1386,7 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_density_tab(int nlocal, int p
     const double* __restrict__ x, const int* __restrict__ neighbors,
     const int* __restrict__ numneigh, double cutforcesq, const double* __restrict__ rs,
     const double* __restrict__ fs, int nr, int nrho, double rdr, double rdrho,
-    double* __restrict__ fp)
+    double2* __restrict__ xf)
 {
     __shared__ double s_rs[TAB_NR * 4];  // value coefficients c3..c6 of each rho row
     for (int k = threadIdx.x; k < nr * 4; k += TAB_BLOCK)
@@ -1409,7 +1426,8 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_density_tab(int nlocal, int p
             p -= m;
             p               = p < 1.0 ? p : 1.0;
             const double* c = fs + m * 7;
-            fp[i]           = (c[0] * p + c[1]) * p + c[2];
+            xf[2 * i]       = make_double2(x[3 * i], x[3 * i + 1]);
+            xf[2 * i + 1]   = make_double2(x[3 * i + 2], (c[0] * p + c[1]) * p + c[2]);
         }
     }
 }
@@ -1418,10 +1436,9 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_density_tab(int nlocal, int p
 // systems' passes, which do not write them, ran 1 % slower).
 template <int LPA, bool STRICT, bool GH>
 __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per_block,
-    const double* __restrict__ x, const int* __restrict__ neighbors,
+    const double2* __restrict__ xf, const int* __restrict__ neighbors,
     const int* __restrict__ numneigh, double cutforcesq, const double* __restrict__ rs,
-    const double* __restrict__ zs, int nr, double rdr, const double* __restrict__ fp,
-    double* __restrict__ f, FuseOf<GH> fu)
+    const double* __restrict__ zs, int nr, double rdr, double* __restrict__ f, FuseOf<GH> fu)
 {
     __shared__ double s_t[TAB_NR * 10];  // per row: rho c0..c2, then z2r c0..c6
     for (int k = threadIdx.x; k < nr * 10; k += TAB_BLOCK) {
@@ -1442,24 +1459,33 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per
         int ng = 0, g0 = 0;
         if (fu.v && act && (lane == 0 || GH)) fused_load<GH>(fu, i, v0, &ng, &g0);
         if (act) {
-            const double xt = x[3 * i], yt = x[3 * i + 1], zt = x[3 * i + 2];
+            const double2 ri0 = xf[2 * i], ri1 = xf[2 * i + 1];
+            const double xt = ri0.x, yt = ri0.y, zt = ri1.x;
             x0[0]            = xt;
             x0[1]            = yt;
             x0[2]            = zt;
-            const double fpi = fp[i];
+            const double fpi = ri1.y;
             const int nn     = numneigh[i];
+            // the list two entries ahead, the neighbour's row one ahead
+            auto list = [&](int k) { return k < nn ? neighbors[(size_t)k * nlocal + i] : i; };
+            int j1     = list(lane), j2 = list(lane + LPA);
+            double2 n0 = xf[2 * (size_t)j1], n1 = xf[2 * (size_t)j1 + 1];
             for (int k = lane; k < nn; k += LPA) {
-                const int j = neighbors[(size_t)k * nlocal + i];
-                double dx   = xt - x[3 * j];
-                double dy   = yt - x[3 * j + 1];
-                double dz   = zt - x[3 * j + 2];
+                const double fpj = n1.y;
+                double dx        = xt - n0.x;
+                double dy        = yt - n0.y;
+                double dz        = zt - n1.x;
+                j1               = j2;
+                j2               = list(k + 2 * LPA);
+                n0               = xf[2 * (size_t)j1];
+                n1               = xf[2 * (size_t)j1 + 1];
                 double rsq  = STRICT ? dx * dx + dy * dy + dz * dz : fma(dx, dx, fma(dy, dy, dz * dz));
                 if (rsq < cutforcesq) {
                     double r = sqrt(rsq);
                     double p, phi;
                     const int m        = eam_knot(r, rdr, nr, &p);
                     const double* row  = s_t + m * 10;
-                    const double fpair = eam_fpair(row, row + 3, p, r, fpi, fp[j], &phi);
+                    const double fpair = eam_fpair(row, row + 3, p, r, fpi, fpj, &phi);
                     if (STRICT) {
                         fix += dx * fpair;
                         fiy += dy * fpair;
@@ -2198,7 +2224,7 @@ void setEamTablesGFX950(int nr, int nrho, double rdr, double rdrho, const double
 }
 
 // Lanes per atom of the fast EAM passes.  The LDS-table passes read the whole spline tables into
-// every block first (64 and 160 KB, ~12 us a pass however few atoms there are), so up to 40000
+// every block first (64 and 160 KB, ~12 us a pass however few atoms there are), so up to 34000
 // atoms the passes read the rows from L2 instead, with an atom's list on as many lanes as the
 // system leaves idle; the density pass then also writes the ghosts' F'.  us per step (both passes,
 // integration, ghosts; 75 listed neighbours) with
@@ -2209,13 +2235,15 @@ void setEamTablesGFX950(int nr, int nrho, double rdr, double rdrho, const double
 //     16384      33.9        24.3  22.7  29.1  41.8
 //     32000      40.6        35.6  44.1  54.1  74.6
 //     55296      49.3        60.5  70.0  87.0 120.3
-// (with a ghost copy and a ghost update launch of 4 us each before).
+// (the tables' column with a ghost copy and a ghost update launch of 4 us each, and before their force
+// pass read rows of position and F' a pair ahead; since then 38.9 against 35.5 with 8 lanes at 32000,
+// 42.9 against 45.2 at 37044 and 43.9 against 51.1 at 42592).
 static int eam_lanes(int nlocal)
 {
     return nlocal <= 1500    ? 64
            : nlocal <= 9000  ? 32
            : nlocal <= 20000 ? 16
-           : nlocal <= 40000 ? 8
+           : nlocal <= 34000 ? 8
                              : FAST_LPA;
 }
 
@@ -2229,7 +2257,7 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
     const double t0 = wtime();
     const int nlocal = atom->Nlocal;
     const int nall   = nlocal + atom->Nghost;
-    grow_n(&S.d_fp, &S.cap_fp, (size_t)nall + 1, 0);
+    grow_n(&S.d_fp, &S.cap_fp, 4 * (size_t)nall + 1, 0);  // F', or rows of position and F'
     if (failed()) return 0.0;
     const bool strict = strict_mode();
     hipStream_t s     = stream();
@@ -2257,21 +2285,26 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
     } while (0)
     // without the energy and for tables of up to TAB_NR rows: the LDS-table passes
 #define MDG_EAM_FT(L, ST, G)                                                                     \
-    k_eam_force_tab<L, ST, G><<<gf, TAB_BLOCK, 0, s>>>(nlocal, pf, atom->d_atom.x,               \
+    k_eam_force_tab<L, ST, G><<<gf, TAB_BLOCK, 0, s>>>(nlocal, pf, xf,                           \
         neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, cutf, S.d_rhor, S.d_z2r,  \
-        S.nr, S.rdr, S.d_fp, atom->d_atom.fx, fu)
+        S.nr, S.rdr, atom->d_atom.fx, fu)
 #define MDG_EAM_TAB(L, ST)                                                                       \
     do {                                                                                         \
         const unsigned gd = 2u * (unsigned)S.ncu, gf = (unsigned)S.ncu;                          \
         const int pd = (int)((nlocal + gd - 1) / gd), pf = (int)((nlocal + gf - 1) / gf);        \
         k_eam_density_tab<L, ST><<<gd, TAB_BLOCK, 0, s>>>(nlocal, pd, atom->d_atom.x,            \
             neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, cutf, S.d_rhor,       \
-            S.d_frho, S.nr, S.nrho, S.rdr, S.rdrho, S.d_fp);                                     \
-        launch_ghost_copy(S.d_fp, atom);                                                         \
+            S.d_frho, S.nr, S.nrho, S.rdr, S.rdrho, xf);                                         \
+        if (atom->Nghost > 0) {                                                                  \
+            k_ghost_rows<<<blocks_for(atom->Nghost, BLOCK), BLOCK, 0, s>>>(nlocal, atom->Nghost, \
+                atom->d_atom.x, xf, atom->d_atom.border_map);                                    \
+            MDG_LAUNCH_CHECK("ghost_rows");                                                      \
+        }                                                                                        \
         if (fu.gcnt) MDG_EAM_FT(L, ST, true);                                                    \
         else MDG_EAM_FT(L, ST, false);                                                           \
     } while (0)
-    const bool tab = !ev && S.nr <= TAB_NR && S.ncu > 0 && nlocal > 0;
+    double2* xf     = (double2*)S.d_fp;
+    const bool tab  = !ev && S.nr <= TAB_NR && S.ncu > 0 && nlocal > 0;
     const bool gmap = S.gmap_nlocal == nlocal && S.gmap_nghost == atom->Nghost;
     const int lanes = eam_lanes(nlocal);
     if (strict) {
