@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -118,6 +119,8 @@ struct State {
     double* d_ev = nullptr;
     int* d_status = nullptr;  // [0] flags, [1] max numneigh, [2] scan total, [3] staging overflows
     int* h_status = nullptr;  // pinned
+    int* h_flag   = nullptr;  // pinned, written by kernels (HF_*)
+    int xs_ld = 0;            // length of d_xs's three runs
     double* h_red = nullptr;  // pinned
     bool ev_on = false;
     double ev_last[2]{};
@@ -262,6 +265,89 @@ __global__ void k_ghost_fill(int nlocal, double* x, Prd prd, double cut,
     }
 }
 
+// The ghosts' counts and offsets of a small system in one block (and, with wrap, the atoms' return
+// into the box before): thread t owns atoms t * per onwards, so that the ghosts stay in the order of
+// their owners.  The total goes to the host's word too.  More than room ghosts: go is set to 0 and
+// the launches behind this one, made before the host knows the total, do nothing.
+// Launches bound a small system's rebuild (about 5 us each with the gap before it): wrap, count,
+// scan and the status copy were four (9.5 us of kernels for 256 atoms, 3.5 here).
+constexpr int SETUP_T = 1024, SETUP_I = 8, SETUP_SMALL = SETUP_T * SETUP_I;
+enum { HF_TOTAL, HF_OVERFLOW, HF_RANGE };  // words that kernels write for the host
+
+__global__ void __launch_bounds__(SETUP_T) k_ghost_setup(int n, double* __restrict__ x, int wrap,
+    Prd prd, double cut, int* __restrict__ cnt, int* __restrict__ off, int* __restrict__ status,
+    int room, int* __restrict__ go, int* __restrict__ host)
+{
+    __shared__ int sh[33];
+    const int per = (n + SETUP_T - 1) / SETUP_T;
+    const int b   = threadIdx.x * per;
+    int c[SETUP_I], sum = 0;
+    double r[SETUP_I][3];  // (all loads first)
+#pragma unroll
+    for (int k = 0; k < SETUP_I; k++)
+        if (k < per)
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+                r[k][d] = x[3 * min(b + k, n - 1) + d];
+#pragma unroll
+    for (int k = 0; k < SETUP_I; k++) {
+        c[k] = 0;
+        if (k >= per || b + k >= n) continue;
+        const int i = b + k;
+        int prod    = 1;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            double xx = r[k][d];
+            if (wrap) {  // (k_wrap)
+                if (xx < 0.0) x[3 * i + d] = xx += prd.p[d];
+                else if (xx >= prd.p[d]) x[3 * i + d] = xx -= prd.p[d];
+            }
+            prod *= 1 + (xx < cut) + (xx >= (prd.p[d] - cut));
+        }
+        c[k] = prod - 1;  // = the bits of ghost_mask
+        sum += c[k];
+    }
+    int total;
+    int at = block_excl_scan(sum, sh, &total);
+#pragma unroll
+    for (int k = 0; k < SETUP_I; k++) {
+        if (k >= per || b + k >= n) continue;
+        cnt[b + k] = c[k];
+        off[b + k] = at;
+        at += c[k];
+    }
+    if (threadIdx.x == 0) {
+        status[0] = status[1] = 0;
+        status[2] = total;
+        *go       = total <= room;
+        host[HF_TOTAL] = total;
+    }
+}
+
+// k_ghost_fill with a thread per atom and image: with a thread per atom, 256 atoms of up to seven
+// images took 6.9 us (3.1 so).
+__global__ void __launch_bounds__(BLOCK) k_ghost_fill_small(int nlocal, double* x, Prd prd, double cut,
+    const int* __restrict__ off, int* __restrict__ border_map, int* __restrict__ pbc,
+    int* __restrict__ type, const int* __restrict__ go)
+{
+    if (!*go) return;
+    const int i = (blockIdx.x * BLOCK + threadIdx.x) >> 5, c = threadIdx.x & 31;
+    if (i >= nlocal) return;  // (for the two halves of a wavefront by themselves)
+    double xi[3] = { x[3 * i], x[3 * i + 1], x[3 * i + 2] };
+    const unsigned m = ghost_mask(xi, prd.p, cut);
+    if (!(m >> c & 1)) return;
+    const int g   = off[i] + __popc(m & ((1u << c) - 1));
+    border_map[g] = i;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const int s             = c_ghost_side[c][d];
+        const int p             = s == 1 ? 1 : (s == 2 ? -1 : 0);
+        pbc[3 * g + d]          = p;
+        x[3 * (nlocal + g) + d] = xi[d] + p * prd.p[d];
+    }
+    type[nlocal + g] = type[i];
+}
+
 __global__ void k_update_pbc(int nlocal, int nghost, double* __restrict__ x,
     const int* __restrict__ border_map, const int* __restrict__ pbc, Prd prd)
 {
@@ -307,8 +393,10 @@ __global__ void k_bin_scatter(int nall, const int* __restrict__ bin_of,
 // are contiguous.  clear: two status words zeroed for the list build that follows.
 __global__ void k_bin_rank(int n, const int* __restrict__ bin_of, const int* __restrict__ binstart,
     const int* __restrict__ slots, const double* __restrict__ x, int* __restrict__ binatoms,
-    double* __restrict__ xs, const int* __restrict__ total, int* __restrict__ clear)
+    double* __restrict__ xs, const int* __restrict__ total, int* __restrict__ clear,
+    const int* __restrict__ go = nullptr)
 {
+    if (go && !*go) return;
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (clear && m < 2) clear[m] = 0;
     if (m >= n || m >= *total) return;
@@ -321,6 +409,113 @@ __global__ void k_bin_rank(int n, const int* __restrict__ bin_of, const int* __r
 #pragma unroll
     for (int d = 0; d < 3; d++)
         xs[(size_t)d * n + r] = x[3 * a + d];
+}
+
+// Counts, scan and scatter in one block for a small system, with the counts and starts in LDS and an
+// atom's bin and place in registers; ORDER (up to BIN1_ORDER atoms): the slots in LDS too, and
+// k_bin_rank's work.  n: nlocal plus the ghosts counted by k_ghost_setup where nghost is not null.
+// 256 atoms and 1500 ghosts: 15 us in four launches, 7.7 in one.  4000 atoms and 5500 ghosts: 25 us in
+// four launches, 17.5 in two, 24 in one (6 for the ranks and 9 for the writes, which many blocks share
+// better).
+constexpr int BIN1_T = 1024, BIN1_I = 16, BIN1_N = BIN1_T * BIN1_I, BIN1_BINS = 16384;
+constexpr int BIN1_ORDER = 4 * BIN1_T;
+
+template <bool ORDER>
+__global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __restrict__ nghost,
+    int ld, const double* __restrict__ x, Grid g, int* __restrict__ binstart,
+    int* __restrict__ bin_of, int* __restrict__ slots, int* __restrict__ binatoms,
+    double* __restrict__ xs, int* __restrict__ status, int clear, const int* __restrict__ go)
+{
+    constexpr int NI = ORDER ? BIN1_ORDER / BIN1_T : BIN1_I;
+    __shared__ int s_bin[BIN1_BINS];  // atoms per bin, then the bins' starts
+    __shared__ int s_slot[ORDER ? BIN1_ORDER : 1];
+    __shared__ int sh[33];
+    if (go && !*go) return;
+    const int n   = nlocal + (nghost ? *nghost : 0);
+    const int tid = threadIdx.x;
+    for (int b = tid; b < g.mbins; b += BIN1_T)
+        s_bin[b] = 0;
+    __syncthreads();
+    int bin[NI], place[NI];
+    double r[4][3];  // (four atoms' loads together)
+#pragma unroll
+    for (int k = 0; k < NI; k++) {
+        bin[k] = -1;
+        if (k * BIN1_T >= n) continue;  // (uniform)
+        if ((k & 3) == 0)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+                    r[q][d] = x[3 * min((k + q) * BIN1_T + tid, n - 1) + d];
+        const int i = k * BIN1_T + tid;
+        if (i >= n) continue;
+        const int b = coord2bin(g, r[k & 3][0], r[k & 3][1], r[k & 3][2]);
+        if (b < 0 || b >= g.mbins) {
+            if (!clear) atomicOr(&status[0], ST_BIN_RANGE);
+            continue;
+        }
+        bin[k]   = b;
+        place[k] = atomicAdd(&s_bin[b], 1);
+    }
+    __syncthreads();
+    // thread t's bins t * per onwards
+    const int per = (g.mbins + BIN1_T - 1) / BIN1_T;
+    const int b0 = tid * per, b1 = min(b0 + per, g.mbins);
+    int sum = 0, total;
+    for (int b = b0; b < b1; b++)
+        sum += s_bin[b];
+    int at = block_excl_scan(sum, sh, &total);
+    for (int b = b0; b < b1; b++) {
+        const int c = s_bin[b];
+        s_bin[b]    = at;
+        at += c;
+    }
+    __syncthreads();
+    for (int b = tid; b < g.mbins; b += BIN1_T)
+        binstart[b] = s_bin[b];
+    if (tid == 0) {
+        binstart[g.mbins] = total;
+        if (clear) status[0] = status[1] = 0;
+    }
+#pragma unroll
+    for (int k = 0; k < NI; k++) {
+        const int i = k * BIN1_T + tid;
+        if (!ORDER && i < n) bin_of[i] = bin[k];
+        if (bin[k] >= 0) (ORDER ? s_slot : slots)[s_bin[bin[k]] + place[k]] = i;
+    }
+    if (!ORDER) return;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NI; k++) {
+        if (bin[k] < 0) continue;
+        const int i = k * BIN1_T + tid;
+        const int s = s_bin[bin[k]], e = bin[k] + 1 < g.mbins ? s_bin[bin[k] + 1] : total;
+        int m = s;
+        for (int q = s; q < e; q++)
+            m += s_slot[q] < i;
+        binatoms[m] = i;
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+            xs[(size_t)d * ld + m] = r[k][d];
+    }
+}
+
+// Launches the binning of up to BIN1_N atoms (nlocal and *nghost), max_n at most, in few launches.
+void launch_bins_small(int nlocal, const int* nghost, int max_n, const double* x, bool clear,
+    const int* go)
+{
+    hipStream_t s = stream();
+    if (max_n <= BIN1_ORDER) {
+        k_bin_single<true><<<1, BIN1_T, 0, s>>>(nlocal, nghost, S.xs_ld, x, S.g, S.d_binstart,
+            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, S.d_status, clear, go);
+    } else {
+        k_bin_single<false><<<1, BIN1_T, 0, s>>>(nlocal, nghost, S.xs_ld, x, S.g, S.d_binstart,
+            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, S.d_status, clear, go);
+        k_bin_rank<<<blocks_for(max_n, BLOCK), BLOCK, 0, s>>>(S.xs_ld, S.d_bin_of, S.d_binstart,
+            S.d_binslots, x, S.d_binatoms, S.d_xs, S.d_binstart + S.g.mbins, nullptr, go);
+    }
+    MDG_LAUNCH_CHECK("binatoms");
 }
 
 // sortAtom (neighbor.c:466-536): new slot p takes the atom at position p of the bin-major list of
@@ -360,21 +555,22 @@ __global__ void k_sort_gather(int n, const int* __restrict__ order, const double
 constexpr int NB_T = 256, NB_SEG = 1024, NB_Q = 32;
 constexpr int NB_SMALL = 24000;  // atoms up to which the block kernel builds the lists
 
-__global__ void __launch_bounds__(NB_T) k_build_neighbor(int nlocal, int nall, const double* __restrict__ xs,
+__global__ void __launch_bounds__(NB_T) k_build_neighbor(int nlocal, int ld, const double* __restrict__ xs,
     const int* __restrict__ type, int ntypes, Tables tab, int uniform, double cnmax, int mbins,
     const int* __restrict__ binstart, const int* __restrict__ binatoms,
     const int* __restrict__ stencil, int nstencil, int half, int maxneighs,
-    int* __restrict__ neighbors, int* __restrict__ numneigh, int* __restrict__ status)
+    int* __restrict__ neighbors, int* __restrict__ numneigh, int* __restrict__ status,
+    int* __restrict__ host, const int* __restrict__ go)
 {
     __shared__ int s_m[NB_SEG], s_cj[NB_SEG];
     __shared__ unsigned long long s_mask[NB_Q][NB_SEG / 64];
     __shared__ int s_off[NB_Q][NB_SEG / 64];
     __shared__ double s_x[NB_Q][3];
     __shared__ int s_id[NB_Q], s_t[NB_Q], s_cnt[NB_Q], s_scan[33], s_w[NB_T / 64], s_nq;
-    const double* ys = xs + nall;
-    const double* zs = ys + nall;
+    const double* ys = xs + ld;
+    const double* zs = ys + ld;
     const int b      = blockIdx.x;
-    if (b >= mbins) return;
+    if (b >= mbins || (go && !*go)) return;
     const int beg = binstart[b], end = binstart[b + 1];
     // index order inside a bin: its local atoms come first
     if (beg >= end || binatoms[beg] >= nlocal) return;
@@ -415,7 +611,7 @@ __global__ void __launch_bounds__(NB_T) k_build_neighbor(int nlocal, int nall, c
             if (c0 + tid < nstencil) {
                 const int jb = b + stencil[c0 + tid];
                 if (jb < 0 || jb >= mbins) {
-                    atomicOr(&status[0], ST_BIN_RANGE);
+                    host[HF_RANGE] = 1;
                 } else {
                     lo = binstart[jb];
                     cc = binstart[jb + 1] - lo;
@@ -513,7 +709,7 @@ __global__ void __launch_bounds__(NB_T) k_build_neighbor(int nlocal, int nall, c
             const int n         = s_cnt[tid];
             numneigh[s_id[tid]] = n;
             if (n > maxneighs) {
-                atomicOr(&status[0], ST_NB_OVERFLOW);
+                host[HF_OVERFLOW] = 1;
                 atomicMax(&status[1], n);
             }
         }
@@ -540,7 +736,7 @@ __device__ inline void wave_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__global__ void __launch_bounds__(BLOCK) k_build_neighbor_wave(int nlocal, int nall,
+__global__ void __launch_bounds__(BLOCK) k_build_neighbor_wave(int nlocal, int ld,
     const double* __restrict__ xs, const int* __restrict__ type, int ntypes, Tables tab, int uniform,
     double cnmax, int mbins, const int* __restrict__ binstart, const int* __restrict__ binatoms,
     const int* __restrict__ stencil, int nstencil, int half, int maxneighs,
@@ -554,8 +750,8 @@ __global__ void __launch_bounds__(BLOCK) k_build_neighbor_wave(int nlocal, int n
     const int beg = binstart[b], end = binstart[b + 1];
     if (beg >= end || binatoms[beg] >= nlocal) return;
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const double* ys = xs + nall;
-    const double* zs = ys + nall;
+    const double* ys = xs + ld;
+    const double* zs = ys + ld;
     int* s_m         = s_c[w];
     NbLocal* loc = s_l[w];
     for (int q0 = beg; q0 < end; q0 += NB_Q) {
@@ -1541,6 +1737,7 @@ bool ensure_status()
     if (!S.d_status) {
         MDG_HIP(hipMalloc(&S.d_status, 16 * sizeof(int)));
         MDG_HIP(hipHostMalloc(&S.h_status, 16 * sizeof(int), hipHostMallocDefault));
+        MDG_HIP(hipHostMalloc(&S.h_flag, 16 * sizeof(int), hipHostMallocCoherent));
         MDG_HIP(hipMalloc(&S.d_ev, 4 * sizeof(double)));
         MDG_HIP(hipHostMalloc(&S.h_red, 4 * sizeof(double), hipHostMallocDefault));
         if (failed()) return false;
@@ -1714,6 +1911,7 @@ void freeDeviceGFX950(Atom* atom, Neighbor* neighbor)
     dfree(S.d_ev);
     dfree(S.d_status);
     if (S.h_status) (void)hipHostFree(S.h_status);
+    if (S.h_flag) (void)hipHostFree(S.h_flag);
     if (S.h_red) (void)hipHostFree(S.h_red);
     S = State();
 }
@@ -1882,6 +2080,12 @@ static void bin_atoms(Atom* atom, bool clear_status)
     grow_n(&S.d_binslots, &S.cap_binslots, (size_t)nall + 1, 0);
     if (failed()) return;
     hipStream_t s = stream();
+    S.xs_ld       = nall;
+    S.binned      = true;
+    if (nall <= BIN1_N && mb <= BIN1_BINS) {
+        launch_bins_small(nall, nullptr, nall, atom->d_atom.x, clear_status, nullptr);
+        return;
+    }
     // (all zero between binnings: the scan clears them)
     if (S.cap_bins != cap0) fill_i32(S.d_bincount, 0, S.cap_bins);
     k_bin_count<<<blocks_for(nall, BLOCK), BLOCK, 0, s>>>(nall, atom->d_atom.x, S.g, S.d_bin_of,
@@ -1893,7 +2097,6 @@ static void bin_atoms(Atom* atom, bool clear_status)
         S.d_binslots, atom->d_atom.x, S.d_binatoms, S.d_xs, S.d_binstart + mb,
         clear_status ? S.d_status : nullptr);
     MDG_LAUNCH_CHECK("binatoms");
-    S.binned = true;
 }
 
 void binatomsGFX950(Atom* atom) { bin_atoms(atom, false); }
@@ -1970,47 +2173,75 @@ static void stage_build(int nlocal, Neighbor* neighbor)
     S.stage_max    = mn;
 }
 
-void buildNeighborGFX950(Atom* atom, Neighbor* neighbor)
+// Launches the list build over the bins; go: see k_ghost_setup.
+static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
 {
-    if (failed() || !S.ready) return;
-    bin_atoms(atom, true);
-    if (failed()) return;
     const int nlocal = atom->Nlocal;
     // the largest list cutoff squared, with a margin over the rounding of a distance to a box
     double cnmax = 0.0;
     for (int k = 0; k < S.ntypes * S.ntypes; k++)
         cnmax = std::max(cnmax, S.tab.cutn[k]);
     cnmax *= 1.0 + 1e-12;
-    for (int attempt = 0; attempt < 8; attempt++) {
-        grow_n(&neighbor->d_neighbor.neighbors, &S.cap_nb, (size_t)nlocal * neighbor->maxneighs, 0);
-        grow_n(&neighbor->d_neighbor.numneigh, &S.cap_numneigh, (size_t)nlocal, 0);
-        if (failed()) return;
-        if (attempt > 0) fill_i32(S.d_status, 0, 2);
-        {
-            TimedRegion tr(F_NEIGHBOR);
-#define MDG_NB(K, G, T)                                                                          \
-    K<<<G, T, 0, stream()>>>(nlocal, nlocal + atom->Nghost, S.d_xs, atom->d_atom.type, S.ntypes, S.tab, \
-        S.uniform ? 1 : 0, cnmax, S.g.mbins, S.d_binstart, S.d_binatoms, S.d_stencil,             \
-        S.nstencil, neighbor->half_neigh, neighbor->maxneighs, neighbor->d_neighbor.neighbors,    \
-        neighbor->d_neighbor.numneigh, S.d_status)
-            if (nlocal <= NB_SMALL) MDG_NB(k_build_neighbor, S.g.mbins, NB_T);
-            else MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK);
+    grow_n(&neighbor->d_neighbor.neighbors, &S.cap_nb, (size_t)nlocal * neighbor->maxneighs, 0);
+    grow_n(&neighbor->d_neighbor.numneigh, &S.cap_numneigh, (size_t)nlocal, 0);
+    if (failed()) return;
+    TimedRegion tr(F_NEIGHBOR);
+#define MDG_NB(K, G, T, ...)                                                                     \
+    K<<<G, T, 0, stream()>>>(nlocal, S.xs_ld, S.d_xs, atom->d_atom.type, S.ntypes, S.tab,        \
+        S.uniform ? 1 : 0, cnmax, S.g.mbins, S.d_binstart, S.d_binatoms, S.d_stencil,            \
+        S.nstencil, neighbor->half_neigh, neighbor->maxneighs, neighbor->d_neighbor.neighbors,   \
+        neighbor->d_neighbor.numneigh, S.d_status __VA_ARGS__)
+#define MDG_COMMA ,
+    if (nlocal <= NB_SMALL) {
+        S.h_flag[HF_OVERFLOW] = S.h_flag[HF_RANGE] = 0;  // (no earlier list build is running)
+        MDG_NB(k_build_neighbor, S.g.mbins, NB_T, MDG_COMMA S.h_flag MDG_COMMA go);
+    } else {
+        MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK);
+    }
+#undef MDG_COMMA
 #undef MDG_NB
-            MDG_LAUNCH_CHECK("build_neighbor");
-        }
+    MDG_LAUNCH_CHECK("build_neighbor");
+}
+
+// Waits for the list build; false: the lists were too short and have been given more room.
+static bool lists_done(int nlocal, Neighbor* neighbor)
+{
+    bool range, overflow;
+    if (nlocal <= NB_SMALL) {
+        MDG_HIP(hipStreamSynchronize(stream()));
+        if (failed()) return true;
+        range    = S.h_flag[HF_RANGE] != 0;
+        overflow = S.h_flag[HF_OVERFLOW] != 0;
+        if (overflow) read_status();  // the longest list
+    } else {
         read_status();
+        range    = (S.h_status[0] & ST_BIN_RANGE) != 0;
+        overflow = (S.h_status[0] & ST_NB_OVERFLOW) != 0;
+    }
+    if (failed()) return true;
+    if (range) {
+        set_error(MDG_ERR_BIN, "an atom lies outside the bin grid (coord2bin out of range)");
+        return true;
+    }
+    if (!overflow) {
+        stage_build(nlocal, neighbor);
+        return true;
+    }
+    // neighbor.c:336-345: grow to 1.2x the largest count and rebuild
+    neighbor->maxneighs = (int)(S.h_status[1] * 1.2) + 1;
+    stage_release();  // room for the list first
+    fill_i32(S.d_status, 0, 2);
+    return false;
+}
+
+void buildNeighborGFX950(Atom* atom, Neighbor* neighbor)
+{
+    if (failed() || !S.ready) return;
+    bin_atoms(atom, true);
+    for (int attempt = 0; attempt < 8; attempt++) {
         if (failed()) return;
-        if (S.h_status[0] & ST_BIN_RANGE) {
-            set_error(MDG_ERR_BIN, "an atom lies outside the bin grid (coord2bin out of range)");
-            return;
-        }
-        if (!(S.h_status[0] & ST_NB_OVERFLOW)) {
-            stage_build(nlocal, neighbor);
-            return;
-        }
-        // neighbor.c:336-345: grow to 1.2x the largest count and rebuild
-        neighbor->maxneighs = (int)(S.h_status[1] * 1.2) + 1;
-        stage_release();  // room for the list first
+        launch_lists(atom, neighbor, nullptr);
+        if (failed() || lists_done(atom->Nlocal, neighbor)) return;
     }
     set_error(MDG_ERR_CAPACITY, "neighbour list did not converge");
 }
@@ -2026,26 +2257,36 @@ void setupPbcGFX950(Atom* atom, Parameter* param)
     grow_n(&S.d_gcnt, &S.cap_gcnt, (size_t)nlocal + 1, 0);
     grow_n(&S.d_goff, &S.cap_goff, (size_t)nlocal + 1, 0);
     if (failed()) return;
-    hipStream_t s = stream();
-    k_ghost_count<<<blocks_for(nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x, prd,
-        param->cutneigh, S.d_gcnt);
-    exclusive_scan(S.d_gcnt, S.d_goff, nlocal, S.d_status + 2);
-    read_status();
-    if (failed()) return;
-    int nghost = S.h_status[2];
+    hipStream_t s    = stream();
+    const bool small = nlocal <= SETUP_SMALL;
+    int nghost;
+    if (small) {
+        k_ghost_setup<<<1, SETUP_T, 0, s>>>(nlocal, atom->d_atom.x, 0, prd, param->cutneigh,
+            S.d_gcnt, S.d_goff, S.d_status, INT_MAX, S.d_status + 4, S.h_flag);
+        MDG_LAUNCH_CHECK("ghost_setup");
+        MDG_HIP(hipStreamSynchronize(s));
+        if (failed()) return;
+        nghost = S.h_flag[HF_TOTAL];
+    } else {
+        k_ghost_count<<<blocks_for(nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x, prd,
+            param->cutneigh, S.d_gcnt);
+        exclusive_scan(S.d_gcnt, S.d_goff, nlocal, S.d_status + 2);
+        read_status();
+        if (failed()) return;
+        nghost = S.h_status[2];
+    }
     // grow atom arrays (keep the locals), ghost map and shifts
     size_t need = (size_t)nlocal + nghost;
     if (need > S.cap_all) {
         int keep_ghost = atom->Nghost;
         atom->Nghost   = 0;  // only locals carry data worth keeping
         DeviceAtom* d  = &atom->d_atom;
-        size_t c       = S.cap_all * 3;
-        grow_n(&d->x, &c, 3 * need, 3 * (size_t)nlocal);
-        c = S.cap_all * 3;
-        grow_n(&d->fx, &c, 3 * need, 0);
-        c = S.cap_all;
-        grow_n(&d->type, &c, need, (size_t)nlocal);
-        S.cap_all    = need;
+        size_t cx = S.cap_all * 3, cf = cx, ct = S.cap_all;
+        grow_n(&d->x, &cx, 3 * need, 3 * (size_t)nlocal);
+        grow_n(&d->fx, &cf, 3 * need, 0);
+        grow_n(&d->type, &ct, need, (size_t)nlocal);
+        // (with the headroom: a rebuild whose ghosts have room waits once)
+        S.cap_all    = failed() ? S.cap_all : std::min({ cx / 3, cf / 3, ct });
         atom->Nghost = keep_ghost;
     }
     size_t gc = S.cap_ghost;
@@ -2053,13 +2294,89 @@ void setupPbcGFX950(Atom* atom, Parameter* param)
     S.cap_ghost = gc;
     grow_n(&S.d_pbc, &S.cap_pbc, 3 * (size_t)nghost + 3, 0);
     if (failed()) return;
-    k_ghost_fill<<<blocks_for(nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x, prd,
-        param->cutneigh, S.d_goff, atom->d_atom.border_map, S.d_pbc, atom->d_atom.type);
+    if (small)
+        k_ghost_fill_small<<<blocks_for(32LL * nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x,
+            prd, param->cutneigh, S.d_goff, atom->d_atom.border_map, S.d_pbc, atom->d_atom.type,
+            S.d_status + 4);
+    else
+        k_ghost_fill<<<blocks_for(nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x, prd,
+            param->cutneigh, S.d_goff, atom->d_atom.border_map, S.d_pbc, atom->d_atom.type);
     MDG_LAUNCH_CHECK("ghost_fill");
     atom->Nghost  = nghost;
     S.gmap_nlocal = nlocal;
     S.gmap_nghost = nghost;
     S.ghosts_current = true;
+}
+
+// A run's rebuild: updateAtomsPbcGFX950, setupPbcGFX950, updatePbcGFX950 and buildNeighborGFX950.  Of a
+// small system whose buffers have room for its ghosts, everything is launched before the host waits
+// (once, for the lists): the launches behind the ghosts' count take it from device memory.  With the
+// kernels of few launches a rebuild takes 16 us less for 256 atoms (of about 75) and 25 for 4000.
+void mdg_vl_reneighbour(Parameter* param, Atom* atom, Neighbor* neighbor)
+{
+    if (failed() || !S.ready) return;
+    const int nlocal = atom->Nlocal;
+    const size_t ld  = std::min(S.cap_all, (size_t)BIN1_N);
+    const size_t room = std::min({ ld - std::min(ld, (size_t)nlocal), S.cap_ghost, S.cap_pbc / 3 });
+    const int mb = S.g.mbins;
+    if (nlocal <= 0 || nlocal > SETUP_SMALL || mb <= 0 || mb > BIN1_BINS || room == 0) {
+        updateAtomsPbcGFX950(atom, param, true);
+        setupPbcGFX950(atom, param);
+        if (!S.ghosts_current) updatePbcGFX950(atom, param, true);
+        buildNeighborGFX950(atom, neighbor);
+        return;
+    }
+    S.gmap_nlocal    = -1;
+    S.ghosts_current = false;
+    S.binned         = false;
+    S.xs_ld          = (int)ld;
+    const Prd prd{ { param->xprd, param->yprd, param->zprd } };
+    grow_n(&S.d_gcnt, &S.cap_gcnt, (size_t)nlocal + 1, 0);
+    grow_n(&S.d_goff, &S.cap_goff, (size_t)nlocal + 1, 0);
+    grow_n(&S.d_xs, &S.cap_xs, 3 * ld, 0);
+    grow_n(&S.d_bin_of, &S.cap_bin_of, ld, 0);
+    grow_n(&S.d_binslots, &S.cap_binslots, ld + 1, 0);
+    grow_n(&S.d_binstart, &S.cap_binstart, (size_t)mb + 1, 0);
+    grow_n(&S.d_binatoms, &S.cap_binatoms, ld + 1, 0);
+    if (failed()) return;
+    hipStream_t s = stream();
+    int* go       = S.d_status + 4;
+    {
+        TimedRegion tr(F_PBC);
+        k_ghost_setup<<<1, SETUP_T, 0, s>>>(nlocal, atom->d_atom.x, 1, prd, param->cutneigh, S.d_gcnt,
+            S.d_goff, S.d_status, (int)room, go, S.h_flag);
+        k_ghost_fill_small<<<blocks_for(32LL * nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x,
+            prd, param->cutneigh, S.d_goff, atom->d_atom.border_map, S.d_pbc, atom->d_atom.type, go);
+        MDG_LAUNCH_CHECK("ghost_setup");
+    }
+    {
+        TimedRegion tr(F_BINNING);
+        launch_bins_small(nlocal, S.d_status + 2, (int)ld, atom->d_atom.x, true, go);
+    }
+    if (failed()) return;
+    launch_lists(atom, neighbor, go);
+    if (failed()) return;
+    MDG_HIP(hipStreamSynchronize(s));
+    if (failed()) return;
+    const int nghost = S.h_flag[HF_TOTAL];
+    if ((size_t)nghost > room) {  // nothing was built (the atoms are in the box)
+        setupPbcGFX950(atom, param);
+        buildNeighborGFX950(atom, neighbor);
+        return;
+    }
+    atom->Nghost     = nghost;
+    S.gmap_nlocal    = nlocal;
+    S.gmap_nghost    = nghost;
+    S.ghosts_current = true;
+    S.binned         = true;
+    for (int attempt = 1; !lists_done(nlocal, neighbor); attempt++) {
+        if (attempt == 8) {
+            set_error(MDG_ERR_CAPACITY, "neighbour list did not converge");
+            return;
+        }
+        launch_lists(atom, neighbor, nullptr);
+        if (failed()) return;
+    }
 }
 
 void updatePbcGFX950(Atom* atom, Parameter* param, bool doReneighbor)

@@ -252,10 +252,7 @@ int mdbVLRun(mdb_vl* s, int nsteps, double* ksum)
         if (resort) sortAtomGFX950(a);
         if (!integrated) initialIntegrateGFX950(reneigh, p, a);
         if (reneigh) {
-            updateAtomsPbcGFX950(a, p, true);
-            setupPbcGFX950(a, p);
-            if (!mdg_vl_ghosts_current()) updatePbcGFX950(a, p, true);
-            buildNeighborGFX950(a, nb);
+            mdg_vl_reneighbour(p, a, nb);
         } else if (!(integrated && mdg_vl_ghosts_current())) {
             /* (the fused force call wrote the ghosts' positions with the atoms') */
             updatePbcGFX950(a, p, false);

@@ -23,5 +23,8 @@ void mdb_free_atom_host(Atom* a);
 /* 1 after a fused force call that also wrote the ghosts' new positions, and after setupPbcGFX950
    (csrc/vl.hip). */
 int mdg_vl_ghosts_current(void);
+/* updateAtomsPbcGFX950, setupPbcGFX950, updatePbcGFX950 and buildNeighborGFX950 of a run's rebuild
+   (csrc/vl.hip). */
+void mdg_vl_reneighbour(Parameter* p, Atom* a, Neighbor* nb);
 
 #endif

@@ -235,3 +235,40 @@ def test_lists_equal_the_oracles_on_moved_atoms(case, half):
             assert nghost > 0 and nn.max() > 200
     finally:
         sim.close()
+
+
+@pytest.mark.parametrize("half", [0, 1])
+@pytest.mark.parametrize("case", [dict(nx=4, ny=4, nz=4), dict(nx=10, ny=10, nz=10),
+                                  dict(nx=12, ny=13, nz=13), dict(nx=13, ny=13, nz=13),
+                                  dict(nx=5, ny=5, nz=5, squeeze=0.2)], ids=str)
+def test_lists_of_a_runs_rebuild(case, half):
+    """The rebuild inside a run, with one wait or in order by the size; squeezed into a corner every
+    atom has seven images, more than there was room for, and the lists outgrow theirs too."""
+    P = product()
+    print(case, half, flush=True)
+    dims = {k: case[k] for k in ("nx", "ny", "nz")}
+    sim = P.VLSim(half_neigh=half, reneigh_every=1 if "squeeze" in case else 3, **dims)
+    try:
+        n = sim.atom.Nlocal
+        p = sim.param
+        ghosts0 = sim.atom.Nghost
+        if "squeeze" in case:
+            x0, _, _ = P.create_lattice(**dims)
+            np.ctypeslib.as_array(sim.atom.x, (3 * n,))[:] = case["squeeze"] * x0.reshape(-1)
+            sim.atom.Nghost = 0  # the host copies hold the local atoms only
+            P.lib().copyDataToGFX950Device(sim.param_p, sim.atom_p)
+            sim.run(1)
+        else:
+            sim.run(3)
+        st = sim.state()
+        _ghosts_follow_owners(sim, st)
+        if "squeeze" in case:
+            assert st["nghost"] == 7 * n > 1.5 * ghosts0
+        nn, nb = ob.build_neighbor(ob.vl_grid(case["nx"], case["ny"], case["nz"], p.lattice,
+                                              p.cutneigh), n, st["x"],
+                                   np.zeros(n + st["nghost"], np.int32), 4,
+                                   np.full(16, p.cutneigh ** 2), half, cap_per_atom=2500)
+        np.testing.assert_array_equal(st["numneigh"], nn)
+        np.testing.assert_array_equal(st["neighbors"], nb)
+    finally:
+        sim.close()
