@@ -34,6 +34,7 @@
 
 #include "mdgfx950_cp.h"
 #include "block_scan.h"
+#include "fp64.h"
 #include "runtime.h"
 
 extern "C" int mdgfx950Status(void);  // mdgfx950.h (not includable beside the cluster structs)
@@ -1484,7 +1485,7 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64_full(int nci, int ntypes
                 if (cj * N + b != si && rsq < cut) {
                     const double eps   = UNIFORM ? tab.eps[0] : s_tab[0][tij];
                     const double sig6  = UNIFORM ? tab.sig6[0] : s_tab[1][tij];
-                    const double sr2   = 1.0 / rsq;
+                    const double sr2   = EV ? 1.0 / rsq : recip_normal(rsq);
                     const double sr6   = sr2 * sr2 * sr2 * sig6;
                     const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
                     fix += dx * force;

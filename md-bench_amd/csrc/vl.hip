@@ -16,6 +16,7 @@
 
 #include "mdgfx950.h"
 #include "block_scan.h"
+#include "fp64.h"
 #include "runtime.h"
 
 using namespace mdg;
@@ -984,7 +985,7 @@ __global__ void __launch_bounds__(BLOCK) k_force_lj(int nlocal, const double* __
                 cutf    = s_tab[2][tij];
             }
             if (rsq < cutf) {
-                double sr2   = 1.0 / rsq;
+                double sr2   = STRICT || EV ? 1.0 / rsq : recip_normal(rsq);
                 double sr6   = sr2 * sr2 * sr2 * sig6;
                 double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
                 if (STRICT) {
@@ -1212,7 +1213,7 @@ __global__ void __launch_bounds__(STAGE_T) k_force_lj_staged(int nlocal, int nal
         if (rsq < cutf) {
             const double eps   = UNIFORM ? tab.eps[0] : s_tab[0][ti + tj];
             const double sig6  = UNIFORM ? tab.sig6[0] : s_tab[1][ti + tj];
-            const double sr2   = 1.0 / rsq;
+            const double sr2   = recip_normal(rsq);
             const double sr6   = sr2 * sr2 * sr2 * sig6;
             const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
             fix                = fma(dx, force, fix);
@@ -1289,7 +1290,7 @@ __global__ void __launch_bounds__(HALF_T) k_force_lj_half(int nlocal, const doub
                 cutf          = s_tab[2][tij];
             }
             if (!(rsq < cutf)) continue;
-            const double sr2   = 1.0 / rsq;
+            const double sr2   = recip_normal(rsq);
             const double sr6   = sr2 * sr2 * sr2 * sig6;
             const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
             fix = fma(dx, force, fix);
@@ -1395,13 +1396,12 @@ __device__ inline double eam_rho(const double* c, double p)
 
 // The pair force over r (force_eam.c:188-206) from the derivative coefficients c0..c2 of the rho
 // row (cr) and the full z2r row (cz); phi for the energy
-__device__ inline double eam_fpair(const double* cr, const double* cz, double p, double r,
+__device__ inline double eam_fpair(const double* cr, const double* cz, double p, double recip,
     double fpi, double fpj, double* phi_out)
 {
     double rhoip = (cr[0] * p + cr[1]) * p + cr[2];
     double z2p   = (cz[0] * p + cz[1]) * p + cz[2];
     double z2    = ((cz[3] * p + cz[4]) * p + cz[5]) * p + cz[6];
-    double recip = 1.0 / r;
     double phi   = z2 * recip;
     double phip  = z2p * recip - phi * recip;
     double psip  = fpi * rhoip + fpj * rhoip + phip;
@@ -1517,10 +1517,16 @@ __global__ void __launch_bounds__(BLOCK) k_eam_force(int nlocal, const double* _
             double dz   = zt - x[3 * j + 2];
             double rsq  = STRICT ? dx * dx + dy * dy + dz * dz : fma(dx, dx, fma(dy, dy, dz * dz));
             if (rsq < cutforcesq) {
-                double r = sqrt(rsq);
+                double r, recip;
+                if (STRICT || EV) {
+                    r     = sqrt(rsq);
+                    recip = 1.0 / r;
+                } else {
+                    recip = root_recip_normal(rsq, &r);
+                }
                 double p, phi;
                 const int m        = eam_knot(r, rdr, nr, &p);
-                const double fpair = eam_fpair(rs + m * 7, zs + m * 7, p, r, fpi, fp[j], &phi);
+                const double fpair = eam_fpair(rs + m * 7, zs + m * 7, p, recip, fpi, fp[j], &phi);
                 if (STRICT) {
                     fix += dx * fpair;
                     fiy += dy * fpair;
@@ -1677,11 +1683,17 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per
                 n1               = xf[2 * (size_t)j1 + 1];
                 double rsq  = STRICT ? dx * dx + dy * dy + dz * dz : fma(dx, dx, fma(dy, dy, dz * dz));
                 if (rsq < cutforcesq) {
-                    double r = sqrt(rsq);
+                    double r, recip;
+                    if (STRICT) {
+                        r     = sqrt(rsq);
+                        recip = 1.0 / r;
+                    } else {
+                        recip = root_recip_normal(rsq, &r);
+                    }
                     double p, phi;
                     const int m        = eam_knot(r, rdr, nr, &p);
                     const double* row  = s_t + m * 10;
-                    const double fpair = eam_fpair(row, row + 3, p, r, fpi, fpj, &phi);
+                    const double fpair = eam_fpair(row, row + 3, p, recip, fpi, fpj, &phi);
                     if (STRICT) {
                         fix += dx * fpair;
                         fiy += dy * fpair;

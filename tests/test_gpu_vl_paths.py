@@ -272,3 +272,38 @@ def test_lists_of_a_runs_rebuild(case, half):
         np.testing.assert_array_equal(st["neighbors"], nb)
     finally:
         sim.close()
+
+
+@pytest.mark.parametrize("kind", ["lj", "lj-half", "eam", "eam-table"])
+def test_atoms_at_one_place(kind):
+    """Two atoms at distance zero: the fast kernels' reciprocals have no special cases, so their forces
+    have to be no numbers where the strict kernels' are, and the other atoms' the strict ones."""
+    P = product()
+    print(kind, flush=True)
+    n = 22 if kind == "eam-table" else 6
+    kw = dict(force_field=1, lattice_a=3.615, temp=300.0, maxwell_seed=5) if "eam" in kind else \
+        dict(half_neigh=int(kind == "lj-half"))
+    sim = P.VLSim(nx=n, ny=n, nz=n, reneigh_every=1000, **kw)
+    L = P.lib()
+    try:
+        nl = sim.atom.Nlocal
+        x = sim.state(lists=False)["x"][:3 * nl].copy()
+        x[300:303] = x[0:3]
+        np.ctypeslib.as_array(sim.atom.x, (3 * nl,))[:] = x
+        sim.atom.Nghost = 0  # the host copies hold the local atoms only
+        L.copyDataToGFX950Device(sim.param_p, sim.atom_p)
+        L.updateAtomsPbcGFX950(sim.atom_p, sim.param_p, True)
+        L.setupPbcGFX950(sim.atom_p, sim.param_p)
+        L.buildNeighborGFX950(sim.atom_p, sim.neighbor_p)
+        sim.compute_force()
+        fast = sim.state(lists=False)["f"].reshape(-1, 3)
+        L.mdgfx950SetStrict(1)
+        sim.compute_force()
+        strict = sim.state(lists=False)["f"].reshape(-1, 3)
+        bad = ~np.isfinite(strict)
+        assert bad.any(axis=1).sum() == 2 and bad[0].all() and bad[100].all()
+        np.testing.assert_array_equal(~np.isfinite(fast), bad)
+        assert np.linalg.norm((fast - strict)[~bad]) < FORCE_RTOL * np.linalg.norm(strict[~bad])
+    finally:
+        L.mdgfx950SetStrict(0)
+        sim.close()
