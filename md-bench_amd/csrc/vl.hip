@@ -27,10 +27,10 @@ constexpr int BLOCK     = 256;
 constexpr int MAXTYPES2 = 64;  // ntypes <= 8
 // LJ passes of full lists stage their neighbours' positions in LDS (k_force_lj_staged, k_stage_build)
 // above STAGE_MIN atoms, where the list is kept for STAGE_USES force calls or more: at 1.05 M atoms a
-// call gains 60 us and the tables cost 300 us per list; whole steps with a list per 20 measured 323 us
-// without and 277 with, at 702 k atoms 218 and 187, at 630 k 184 and 173, at 520 k (the list just fits
-// the last-level cache) 136 and 146.
-constexpr int STAGE_MIN = 600000, STAGE_USES = 8, STAGE_RETRY = 32;
+// call gains 84 us and the tables cost 300 us per list; whole steps with a list per 20 measured 323 us
+// without and 255 with, at 702 k atoms 218 and 170, at 562 k 148 and 137, at 500 k (the list just fits
+// the last-level cache) 126 and 127.
+constexpr int STAGE_MIN = 520000, STAGE_USES = 8, STAGE_RETRY = 32;
 constexpr int FUSE_GHOSTS_EAM = 300000;  // EAM systems up to this size move ghosts in the force call
 constexpr int FAST_LPA  = 4;   // lanes per atom in the fast force kernels of large systems
 
@@ -1046,9 +1046,10 @@ __global__ void __launch_bounds__(BLOCK) k_force_lj(int nlocal, const double* __
 // list entry's place among them, is worked out when the list is built (k_stage_build).  Both are
 // only hints: a pair uses the staged position only if the staged atom is the one its list entry
 // names, and loads it from memory otherwise (a list written by someone else, a region with more than
-// STAGE_CAP distinct neighbours).  1.05 M atoms: 276 us per call with the positions gathered, 217
-// staged (half the VALU's time, 60 % of the texture path's, the list and hints at 2.2 TB/s).  The two
-// blocks that a CU's LDS and waves hold set STAGE_CAP; a 256-atom lattice block names 1300 - 1700.
+// STAGE_CAP distinct neighbours).  1.05 M atoms: 276 us per call with the positions gathered, 192
+// staged (60 % of the VALU's time and half the LDS's; the list and hints at 2.5 TB/s).  The two blocks
+// that a CU's LDS and waves hold set STAGE_CAP; a 256-atom lattice block names 1300 - 1700.  Blocks
+// of 512 threads and 128 atoms took the same, three or four sets of entries ahead too.
 constexpr int STAGE_T = 1024, STAGE_A = 256, STAGE_CAP = 2000, STAGE_LOG = 10;
 
 // tab: STAGE_CAP atoms per block, tab_n: how many (0: too many), hint[k * nlocal + i]: the place.
@@ -1126,14 +1127,14 @@ __global__ void __launch_bounds__(STAGE_T) k_stage_build(int nlocal,
 template <bool UNIFORM>
 __global__ void __launch_bounds__(STAGE_T) k_force_lj_staged(int nlocal, int nall, int nblocks,
     const double* __restrict__ x, const int* __restrict__ type, int ntypes, Tables tab,
-    const int* __restrict__ neighbors, const int* __restrict__ numneigh, int maxhint,
+    const int* __restrict__ neighbors, const int* __restrict__ numneigh, int maxneighs,
     const int* __restrict__ stage, const int* __restrict__ stage_n,
     const unsigned short* __restrict__ hint, double* __restrict__ f, Fuse fu)
 {
     constexpr int LPA = STAGE_T / STAGE_A;
-    __shared__ double s_pos[3 * STAGE_CAP];
-    __shared__ int s_key[STAGE_CAP];
-    __shared__ unsigned char s_type[UNIFORM ? 1 : STAGE_CAP];
+    __shared__ double s_pos[3 * STAGE_CAP + 3];
+    __shared__ int s_key[STAGE_CAP + 1];  // the one behind the last: no atom
+    __shared__ unsigned char s_type[UNIFORM ? 1 : STAGE_CAP + 1];
     __shared__ double s_tab[3][UNIFORM ? 1 : MAXTYPES2];
     // blocks of one XCD adjacent (the grid is a multiple of 8)
     const int per = gridDim.x >> 3;
@@ -1146,7 +1147,7 @@ __global__ void __launch_bounds__(STAGE_T) k_force_lj_staged(int nlocal, int nal
             s_tab[2][k] = tab.cutf[k];
         }
     const int ns = stage_n[b];
-    if (threadIdx.x == 0 && ns == 0) s_key[0] = -1;
+    if (threadIdx.x == 0) s_key[ns] = -1;
     for (int k = threadIdx.x; k < ns; k += STAGE_T) {
         const int j = stage[(size_t)b * STAGE_CAP + k];
         const bool in = (unsigned)j < (unsigned)nall;
@@ -1173,44 +1174,40 @@ __global__ void __launch_bounds__(STAGE_T) k_force_lj_staged(int nlocal, int nal
         if (!UNIFORM) ti = type[i] * ntypes;
     }
     __syncthreads();
-    // entries and hints two iterations ahead
-    const size_t step = (size_t)LPA * nlocal;
-    const int* lst             = neighbors + (size_t)lane * nlocal + i;
-    const unsigned short* hnt  = hint + (size_t)lane * nlocal + i;
-    const int nh               = ns ? min(nn, maxhint) : 0;
-    auto next = [&](int k, int* j, int* h) {
-        if (k < nn) *j = *lst;
-        *h = 0;
-        if (k < nh) *h = *hnt;
-        lst += step;
-        hnt += step;
+    // Entries and hints two iterations ahead, in two sets of registers.  The loads are unconditional
+    // (a lane behind its list's end reads the row's first entry, as all such lanes do) and a memory
+    // fallback waits where it is, so that the waits in the loop are for the older set alone: with a
+    // branch around the loads the compiler waited for all of them in every iteration (207 us).
+    const unsigned at = lane * (unsigned)nlocal + (act ? i : 0);
+    auto next = [&](int k0, int* j, unsigned* h) {
+        const unsigned e = k0 + lane < nn ? at : 0;
+        const size_t row = (size_t)min(k0, maxneighs - 1) * nlocal;
+        *j = *(const int*)((const char*)(neighbors + row) + 4u * e);
+        *h = *(const unsigned short*)((const char*)(hint + row) + 2u * e);
     };
-    int j1 = 0, h1 = 0, j2 = 0, h2 = 0;
-    next(lane, &j1, &h1);
-    next(lane + LPA, &j2, &h2);
-    for (int k = lane; k < nn; k += LPA) {
-        const int j = j1;
-        int h       = h1;
-        j1          = j2;
-        h1          = h2;
-        next(k + 2 * LPA, &j2, &h2);
-        h = h < ns ? h : 0;
+    auto pair = [&](int k0, int* pj, unsigned* ph) {
+        const int j      = *pj;
+        const unsigned h = min(*ph, (unsigned)ns);
         double xj = s_pos[3 * h], yj = s_pos[3 * h + 1], zj = s_pos[3 * h + 2];
         int tj = 0;
         if (!UNIFORM) tj = s_type[h];
+        const int key = s_key[h];
+        next(k0 + 2 * LPA, pj, ph);
         // (kept as LDS reads: the compiler would merge them with the loads below into flat loads,
         // which take the texture path again)
         asm volatile("" : "+v"(xj), "+v"(yj), "+v"(zj));
-        if (__builtin_expect(s_key[h] != j, 0)) {
+        const bool in = k0 + lane < nn;
+        if (__builtin_expect(in && key != j, 0)) {
             xj = x[3 * j];
             yj = x[3 * j + 1];
             zj = x[3 * j + 2];
             if (!UNIFORM) tj = type[j];
+            asm volatile("" : "+v"(xj), "+v"(yj), "+v"(zj), "+v"(tj));
         }
         const double dx = x0[0] - xj, dy = x0[1] - yj, dz = x0[2] - zj;
         const double rsq  = fma(dx, dx, fma(dy, dy, dz * dz));
         const double cutf = UNIFORM ? tab.cutf[0] : s_tab[2][ti + tj];
-        if (rsq < cutf) {
+        if (in && rsq < cutf) {
             const double eps   = UNIFORM ? tab.eps[0] : s_tab[0][ti + tj];
             const double sig6  = UNIFORM ? tab.sig6[0] : s_tab[1][ti + tj];
             const double sr2   = recip_normal(rsq);
@@ -1220,6 +1217,14 @@ __global__ void __launch_bounds__(STAGE_T) k_force_lj_staged(int nlocal, int nal
             fiy                = fma(dy, force, fiy);
             fiz                = fma(dz, force, fiz);
         }
+    };
+    int j1, j2;
+    unsigned h1, h2;
+    next(0, &j1, &h1);
+    next(LPA, &j2, &h2);
+    for (int k0 = 0; k0 + lane < nn; k0 += 2 * LPA) {
+        pair(k0, &j1, &h1);
+        pair(k0 + LPA, &j2, &h2);
     }
     fix = group_sum<LPA>(fix);
     fiy = group_sum<LPA>(fiy);
@@ -2164,7 +2169,8 @@ static void stage_build(int nlocal, Neighbor* neighbor)
     S.list_uses    = 0;
     if (S.stage_nlocal == nlocal && over > nb / 2) S.stage_skip = STAGE_RETRY;
     S.stage_nlocal = -1;
-    if (neighbor->half_neigh || strict_mode() || nlocal <= STAGE_MIN || S.d_rhor) return;
+    if (neighbor->half_neigh || strict_mode() || nlocal <= STAGE_MIN || nlocal > (1 << 27) || S.d_rhor)
+        return;
     if (uses < STAGE_USES) return;
     if (S.stage_skip > 0) {
         S.stage_skip--;
@@ -2504,7 +2510,7 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
                 else if (lanes == 32) MDG_LJ(32, false, false, false);
                 else if (lanes == 16) MDG_LJ(16, false, false, false);
                 else if (lanes == 8) MDG_LJ(8, false, false, false);
-                else if (S.stage_nlocal == nlocal) {
+                else if (S.stage_nlocal == nlocal && S.stage_max == neighbor->maxneighs) {
                     const int nb        = (nlocal + STAGE_A - 1) / STAGE_A;
                     const unsigned grid = ((unsigned)nb + 7) & ~7u;
 #define MDG_LJS(U)                                                                               \
