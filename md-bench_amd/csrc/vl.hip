@@ -934,6 +934,84 @@ __device__ inline void fused_load(const FuseOf<GH>& fu, int i, double* v0, int* 
         }
 }
 
+// A lane's list entries (lane, lane + LPA, ... of atom i) in order.  The loads have no branch around
+// them, which would make the compiler wait for all loads in flight: behind the list's end the first
+// entry is read again.
+template <int LPA>
+struct ListWalk {
+    const int *p, *p0;
+    size_t step;
+    int nn;
+    __device__ ListWalk(const int* neighbors, int nlocal, int i, int lane, int n)
+        : p(neighbors + (size_t)lane * nlocal + i), p0(neighbors + i), step((size_t)LPA * nlocal),
+          nn(n)
+    {
+    }
+    __device__ int next(int k)
+    {
+        const int j = *(k < nn ? p : p0);
+        p += step;
+        return j;
+    }
+};
+
+// The value of the neighbouring lane (lane ^ 1)
+__device__ inline int swap1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false); }
+__device__ inline double swap1(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = swap1((int)b), hi = swap1((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// What two neighbouring lanes load together of their two atoms j (both lanes active): each 16 bytes of
+// the even lane's atom, then of the odd lane's.  A load's cost is the cache lines that neighbouring
+// lanes name, a lookup per clock: a lane alone needs two for its atom's 24 or 32 bytes, two together
+// one for each of the two.  The lanes exchange halves when the values are used (registers still
+// being loaded are not touched before).
+struct alignas(8) Pos2 {
+    double a, b;
+};
+template <bool PAIR>
+struct GatherPos {  // position j of x: even lane (x, y), odd lane (y, z)
+    Pos2 p, q;
+    __device__ void load(const double* __restrict__ x, int j, bool odd)
+    {
+        const int jo = PAIR ? swap1(j) : j;
+        p = *reinterpret_cast<const Pos2*>(x + 3 * (size_t)(odd ? jo : j) + odd);
+        q = *reinterpret_cast<const Pos2*>(x + 3 * (size_t)(odd ? j : jo) + (PAIR ? odd : 1));
+    }
+    __device__ double3 get(bool odd) const
+    {
+        if (!PAIR) return make_double3(p.a, p.b, q.b);
+        const double r = swap1(odd ? p.b : q.a);
+        return make_double3(odd ? r : p.a, odd ? q.a : p.b, odd ? q.b : r);
+    }
+};
+template <bool PAIR>
+struct GatherRow {  // row j of four doubles
+    double2 p, q;
+    __device__ void load(const double2* __restrict__ rows, int j, bool odd)
+    {
+        const int jo = PAIR ? swap1(j) : j;
+        p            = rows[2 * (size_t)(odd ? jo : j) + odd];
+        q            = rows[2 * (size_t)(odd ? j : jo) + (PAIR ? odd : 1)];
+    }
+    __device__ void get(bool odd, double2* r0, double2* r1) const
+    {
+        if (!PAIR) {
+            *r0 = p;
+            *r1 = q;
+            return;
+        }
+        double2 t = odd ? p : q;
+        t.x       = swap1(t.x);
+        t.y       = swap1(t.y);
+        *r0       = odd ? t : p;
+        *r1       = odd ? q : t;
+    }
+};
+
 // ---------------------------------------------------------------- LJ (force_lj.c:17-206)
 // One atom per LPA lanes.  STRICT: LPA == 1, reference order, no fma.
 template <int LPA, bool STRICT, bool HALF, bool EV>
@@ -1579,12 +1657,14 @@ __global__ void __launch_bounds__(BLOCK) k_eam_force(int nlocal, const double* _
 // the blocks are persistent: TAB_BLOCK threads, one block per 64 KB / 160 KB of a CU's LDS,
 // each over a contiguous range of atoms (ranges of one XCD adjacent, as in the cluster-pair
 // kernels).  Operations and their order are those of k_eam_density / k_eam_force.
-// The density pass leaves a row of 32 bytes per atom, its position and F', for the force pass: with
-// one block per CU (4 waves per SIMD) that pass waited for a gather of the position and another of F'
-// per pair.  One aligned row, in one cache line, loaded a pair ahead of its use: 451 -> 345 us at
-// 1.05 M atoms (377 a pair ahead but without the rows), 53 -> 45 at 131 k; the rows cost the density
-// pass 6 us of 255.  The density pass itself gains nothing from loads ahead (281 us): two blocks a CU
-// hide them, and it is bound by the cache lines that its gathers fill.
+// The density pass leaves a row of 32 bytes per atom, its position and F', for the force pass: one
+// aligned row in one cache line instead of a position and an F'.  Both passes load list entries two
+// or three pairs ahead and positions or rows one, in two sets of registers, and two neighbouring
+// lanes load their two atoms together (GatherPos, GatherRow): they were bound by the L1's lookups,
+// one per lane and load, and the force pass (one block per CU, 4 waves per SIMD) by latency.  Force
+// pass at 1.05 M atoms 451 -> 288 us (377 loading ahead, 343 with rows, 299 without branches around
+// the list loads), at 131 k 53 -> 41; density 255 -> 262 (the rows cost 6; loads ahead alone 270) and
+// 30 -> 28.  Bound now: FP64 instructions and lookups alike.
 constexpr int TAB_BLOCK = 1024;
 constexpr int TAB_NR    = 2000;
 
@@ -1611,17 +1691,33 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_density_tab(int nlocal, int p
         if (act) {
             const double xt = x[3 * i], yt = x[3 * i + 1], zt = x[3 * i + 2];
             const int nn    = numneigh[i];
-            for (int k = lane; k < nn; k += LPA) {
-                const int j = neighbors[(size_t)k * nlocal + i];
-                double dx   = xt - x[3 * j];
-                double dy   = yt - x[3 * j + 1];
-                double dz   = zt - x[3 * j + 2];
-                double rsq  = STRICT ? dx * dx + dy * dy + dz * dz : fma(dx, dx, fma(dy, dy, dz * dz));
-                if (rsq < cutforcesq) {
+            // the list two or three entries ahead, positions one, in two sets of registers
+            ListWalk<LPA> list(neighbors, nlocal, i, lane, nn);
+            GatherPos<(LPA > 1)> pa, pb;
+            const bool odd = LPA > 1 && (lane & 1);
+            auto pair = [&](int k, const GatherPos<(LPA > 1)>& w) {
+                const double3 q  = w.get(odd);
+                const double dx  = xt - q.x;
+                const double dy  = yt - q.y;
+                const double dz  = zt - q.z;
+                const double rsq = STRICT ? dx * dx + dy * dy + dz * dz
+                                          : fma(dx, dx, fma(dy, dy, dz * dz));
+                if (k < nn && rsq < cutforcesq) {
                     double p;
                     const int m = eam_knot(sqrt(rsq), rdr, nr, &p);
                     rhoi += eam_rho(s_rs + m * 4, p);
                 }
+            };
+            int ja = list.next(lane), jb = list.next(lane + LPA);
+            pa.load(x, nn > 0 ? ja : i, odd);
+            ja = list.next(lane + 2 * LPA);
+            for (int k = lane; k - lane < nn; k += 2 * LPA) {  // (all lanes of the atom)
+                pb.load(x, jb, odd);
+                jb = list.next(k + 3 * LPA);
+                pair(k, pa);
+                pa.load(x, ja, odd);
+                ja = list.next(k + 4 * LPA);
+                pair(k + LPA, pb);
             }
         }
         if (LPA > 1) rhoi = group_sum<LPA>(rhoi);
@@ -1673,21 +1769,19 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per
             x0[2]            = zt;
             const double fpi = ri1.y;
             const int nn     = numneigh[i];
-            // the list two entries ahead, the neighbour's row one ahead
-            auto list = [&](int k) { return k < nn ? neighbors[(size_t)k * nlocal + i] : i; };
-            int j1     = list(lane), j2 = list(lane + LPA);
-            double2 n0 = xf[2 * (size_t)j1], n1 = xf[2 * (size_t)j1 + 1];
-            for (int k = lane; k < nn; k += LPA) {
-                const double fpj = n1.y;
-                double dx        = xt - n0.x;
-                double dy        = yt - n0.y;
-                double dz        = zt - n1.x;
-                j1               = j2;
-                j2               = list(k + 2 * LPA);
-                n0               = xf[2 * (size_t)j1];
-                n1               = xf[2 * (size_t)j1 + 1];
-                double rsq  = STRICT ? dx * dx + dy * dy + dz * dz : fma(dx, dx, fma(dy, dy, dz * dz));
-                if (rsq < cutforcesq) {
+            // the list two or three entries ahead, rows one, in two sets of registers
+            ListWalk<LPA> list(neighbors, nlocal, i, lane, nn);
+            GatherRow<(LPA > 1)> ra, rb;
+            const bool odd = LPA > 1 && (lane & 1);
+            auto pair = [&](int k, const GatherRow<(LPA > 1)>& w) {
+                double2 r0, r1;
+                w.get(odd, &r0, &r1);
+                const double dx  = xt - r0.x;
+                const double dy  = yt - r0.y;
+                const double dz  = zt - r1.x;
+                const double rsq = STRICT ? dx * dx + dy * dy + dz * dz
+                                          : fma(dx, dx, fma(dy, dy, dz * dz));
+                if (k < nn && rsq < cutforcesq) {
                     double r, recip;
                     if (STRICT) {
                         r     = sqrt(rsq);
@@ -1698,7 +1792,7 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per
                     double p, phi;
                     const int m        = eam_knot(r, rdr, nr, &p);
                     const double* row  = s_t + m * 10;
-                    const double fpair = eam_fpair(row, row + 3, p, recip, fpi, fpj, &phi);
+                    const double fpair = eam_fpair(row, row + 3, p, recip, fpi, r1.y, &phi);
                     if (STRICT) {
                         fix += dx * fpair;
                         fiy += dy * fpair;
@@ -1709,6 +1803,17 @@ __global__ void __launch_bounds__(TAB_BLOCK) k_eam_force_tab(int nlocal, int per
                         fiz = fma(dz, fpair, fiz);
                     }
                 }
+            };
+            int ja = list.next(lane), jb = list.next(lane + LPA);
+            ra.load(xf, nn > 0 ? ja : i, odd);
+            ja = list.next(lane + 2 * LPA);
+            for (int k = lane; k - lane < nn; k += 2 * LPA) {  // (all lanes of the atom)
+                rb.load(xf, jb, odd);
+                jb = list.next(k + 3 * LPA);
+                pair(k, ra);
+                ra.load(xf, ja, odd);
+                ja = list.next(k + 4 * LPA);
+                pair(k + LPA, rb);
             }
         }
         if (LPA > 1) {
