@@ -2664,10 +2664,10 @@ void setEamTablesGFX950(int nr, int nrho, double rdr, double rdrho, const double
 }
 
 // Lanes per atom of the fast EAM passes.  The LDS-table passes read the whole spline tables into
-// every block first (64 and 160 KB, ~12 us a pass however few atoms there are), so up to 34000
-// atoms the passes read the rows from L2 instead, with an atom's list on as many lanes as the
-// system leaves idle; the density pass then also writes the ghosts' F'.  us per step (both passes,
-// integration, ghosts; 75 listed neighbours) with
+// every block first (64 and 160 KB, ~12 us a pass however few atoms there are), so up to 20000
+// atoms (40000 with tables that do not fit) the passes read the rows from L2 instead, with an atom's
+// list on as many lanes as the system leaves idle; the density pass then also writes the ghosts' F'.
+// us per step (both passes, integration, ghosts; 75 listed neighbours) with
 //     atoms  LDS tables, 4     8    16    32    64 lanes
 //       500      30.4        19.8  12.6  10.2   8.9
 //      4000      32.1        20.2  13.3  12.3  13.2
@@ -2675,16 +2675,15 @@ void setEamTablesGFX950(int nr, int nrho, double rdr, double rdrho, const double
 //     16384      33.9        24.3  22.7  29.1  41.8
 //     32000      40.6        35.6  44.1  54.1  74.6
 //     55296      49.3        60.5  70.0  87.0 120.3
-// (the tables' column with a ghost copy and a ghost update launch of 4 us each, and before their force
-// pass read rows of position and F' a pair ahead; since then 38.9 against 35.5 with 8 lanes at 32000,
-// 42.9 against 45.2 at 37044 and 43.9 against 51.1 at 42592).
-static int eam_lanes(int nlocal)
+// (the tables' column before two lanes loaded a neighbour together; since then 28.2 against 29.5 with
+// 8 lanes at 23328, 29.7 against 35.4 at 32000 and 34.9 against 45.5 at 37044).
+static int eam_lanes(int nlocal, bool tab)
 {
-    return nlocal <= 1500    ? 64
-           : nlocal <= 9000  ? 32
-           : nlocal <= 20000 ? 16
-           : nlocal <= 34000 ? 8
-                             : FAST_LPA;
+    return nlocal <= 1500             ? 64
+           : nlocal <= 9000           ? 32
+           : nlocal <= 20000          ? 16
+           : !tab && nlocal <= 40000  ? 8
+                                      : FAST_LPA;
 }
 
 static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu)
@@ -2746,7 +2745,7 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
     double2* xf     = (double2*)S.d_fp;
     const bool tab  = !ev && S.nr <= TAB_NR && S.ncu > 0 && nlocal > 0;
     const bool gmap = S.gmap_nlocal == nlocal && S.gmap_nghost == atom->Nghost;
-    const int lanes = eam_lanes(nlocal);
+    const int lanes = eam_lanes(nlocal, tab);
     if (strict) {
         if (ev) MDG_EAM(1, true, true);
         else if (tab) MDG_EAM_TAB(1, true);

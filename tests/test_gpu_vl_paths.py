@@ -307,3 +307,34 @@ def test_atoms_at_one_place(kind):
     finally:
         L.mdgfx950SetStrict(0)
         sim.close()
+
+
+@pytest.mark.parametrize("dims", [(18, 17, 17), (22, 22, 21)], ids=str)
+def test_eam_tables_too_long_for_lds(dims, tmp_path):
+    """2400 rows: 8 and 4 lanes per atom with the rows from L2."""
+    P = product()
+    print(dims, flush=True)
+    path = tmp_path / "cu.eam"
+    P.lib().mdbWriteFuncflSynthetic(str(path).encode())
+    lines = path.read_text().split("\n")
+    nrho, drho, nr, dr, rc = lines[2].split()
+    n, m = int(nr), 2400
+    vals = np.array(" ".join(lines[3:]).split(), float).reshape(3, n)
+    fine = np.arange(m) * float(dr) * n / m
+    rows = [vals[0]] + [np.interp(fine, np.arange(n) * float(dr), v) for v in vals[1:]]
+    path.write_text("\n".join(lines[:2] + ["%s %s %d %.16e %s" % (nrho, drho, m, fine[1], rc)] +
+                              ["%.16e" % v for r in rows for v in r]) + "\n")
+    tab = ob.EamTables(str(path))
+    sim = P.VLSim(nx=dims[0], ny=dims[1], nz=dims[2], force_field=1, lattice_a=3.615, temp=1600.0,
+                  maxwell_seed=5, reneigh_every=5, eam_file=str(path))
+    try:
+        sim.run(6)
+        st = sim.state()
+        want, _ = ob.force_eam_atom(tab, st["nlocal"], st["x"], st["border_map"],
+                                    sim.param.cutforce ** 2, st["numneigh"], st["neighbors"])
+        want = want[:3 * st["nlocal"]]
+        assert np.linalg.norm(want) > 10.0
+        assert np.linalg.norm(st["f"] - want) < FORCE_RTOL * np.linalg.norm(want)
+        _ghosts_follow_owners(sim, st)
+    finally:
+        sim.close()
