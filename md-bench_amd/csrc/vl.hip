@@ -1373,7 +1373,7 @@ __global__ void __launch_bounds__(HALF_T) k_force_lj_half(int nlocal, const doub
                 cutf          = s_tab[2][tij];
             }
             if (!(rsq < cutf)) continue;
-            const double sr2   = recip_normal(rsq);
+            const double sr2   = EV ? 1.0 / rsq : recip_normal(rsq);
             const double sr6   = sr2 * sr2 * sr2 * sig6;
             const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
             fix = fma(dx, force, fix);
