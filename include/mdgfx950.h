@@ -100,10 +100,12 @@ double computeForceEamGFX950(Parameter* param, Atom* atom, Neighbor* neighbor, S
    the NEXT step's initialIntegrate (src/verletlist/main.c loop) in one call.  The fast full-list
    kernels kick each atom twice with the force they have just written and drift it into a second
    position buffer, which becomes atom->d_atom.x; the same FP64 operations in the same order as
-   the three calls.  Ghost positions are stale until updatePbcGFX950, as after initialIntegrate.
-   Velocities are left at the next half step: callers reading full-step velocities after a step
-   (thermo, the last step) call the three separately there.  Strict kernels and half lists run
-   the three calls in order. */
+   the three calls.  Half lists do so in place, after all their forces are summed.  Ghost positions
+   are stale until updatePbcGFX950, as after initialIntegrate, or already follow their owners
+   (systems whose border atoms' images the same kernel writes); updatePbcGFX950 gives the same
+   positions either way.  Velocities are left at the next half step: callers reading full-step
+   velocities after a step (thermo, the last step) call the three separately there.  Strict kernels
+   run the three calls in order. */
 double computeForceFinalInitialGFX950(Parameter* param, Atom* atom, Neighbor* neighbor,
     Stats* stats);
 /* uploads one pair table in the reference's 7-coefficient layout (src/common/eam.h:20-29,

@@ -1398,6 +1398,106 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64(int nci, int ncj, int nt
     if (EV) ev_store(e, w, ev);
 }
 
+// Half lists of i-clusters of four: one wavefront per i-cluster, lane (e, a) takes i-atom a and entry e
+// of a round of 16.  A j-atom's four pair forces are added over the lanes of its i-atoms first, so
+// that one atomic per coordinate goes to memory instead of four; the i-forces are summed over the
+// entries.  One thread per i-slot walking its list (k_cp_force_f64, still the 1x2 clusters' kernel)
+// took 438 us a step for 98,000 atoms of 4x4 clusters, this 103 (864 atoms 150 and 17; 4x8 clusters 468
+// and 131).  Bound: FP64 atomics and the registers' 4 - 6 wavefronts per SIMD.
+template <int N, bool EV, bool UNIFORM>
+__global__ void __launch_bounds__(BLOCK) k_cp_force_f64_half(int nci, int ncj, int ntypes, Tab64 tab,
+    const double* __restrict__ sx, const int* __restrict__ st, const int* __restrict__ nb,
+    const int* __restrict__ numneigh, int maxneighs, double* __restrict__ f, double* __restrict__ ev)
+{
+    __shared__ double s_tab[3][MAXT2];
+    if (!UNIFORM) {
+        for (int k = threadIdx.x; k < ntypes * ntypes; k += BLOCK) {
+            s_tab[0][k] = tab.eps[k];
+            s_tab[1][k] = tab.sig6[k];
+            s_tab[2][k] = tab.cutf[k];
+        }
+        __syncthreads();
+    }
+    // i-clusters of one XCD adjacent (the grid is a multiple of 8 blocks)
+    const int per = gridDim.x >> 3;
+    const int lb  = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    const int w   = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int ci  = __builtin_amdgcn_readfirstlane(lb * (BLOCK / 64) + w);
+    if (ci >= nci) return;
+    const int a = lane & 3, e = lane >> 2, si = ci * 4 + a;
+    const int own   = N == 4 ? ci : ci >> 1;
+    const double xt = sx[3 * si], yt = sx[3 * si + 1], zt = sx[3 * si + 2];
+    const int ti    = UNIFORM ? 0 : st[si] * ntypes;
+    const int* lst  = nb + (size_t)ci * maxneighs;
+    const int nn    = numneigh[ci];
+    double fi[3] = {}, ee = 0.0, ww = 0.0;
+    int cj = e < nn ? lst[e] : -1;
+    for (int k0 = 0; k0 < nn; k0 += 16) {
+        const int kn  = k0 + 16 + e;
+        const int cjn = kn < nn ? lst[kn] : -1;
+        if (cj >= 0) {  // (the same for the four lanes of an entry)
+            double xj[N][3];
+            int tj[N];
+#pragma unroll
+            for (int b = 0; b < N; b++) {
+                const int sj = cj * N + b;
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+                    xj[b][d] = sx[3 * (size_t)sj + d];
+                tj[b] = UNIFORM ? 0 : st[sj];
+            }
+            double mine[N / 4][3];  // the sums of j-atoms a, a + 4
+#pragma unroll
+            for (int b = 0; b < N; b++) {
+                const double dr[3] = { xt - xj[b][0], yt - xj[b][1], zt - xj[b][2] };
+                const double rsq   = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
+                const int tij      = ti + tj[b];
+                const double cut   = UNIFORM ? tab.cutf[0] : s_tab[2][tij];
+                double g[3]        = {};
+                if ((cj != own || si < cj * N + b) && rsq < cut) {
+                    const double eps   = UNIFORM ? tab.eps[0] : s_tab[0][tij];
+                    const double sig6  = UNIFORM ? tab.sig6[0] : s_tab[1][tij];
+                    const double sr2   = EV ? 1.0 / rsq : recip_normal(rsq);
+                    const double sr6   = sr2 * sr2 * sr2 * sig6;
+                    const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
+#pragma unroll
+                    for (int d = 0; d < 3; d++) {
+                        g[d] = dr[d] * force;
+                        fi[d] += g[d];
+                    }
+                    if (EV) {
+                        const double wgt = cj < ncj ? 1.0 : 0.5;
+                        ee += wgt * 4.0 * eps * sr6 * (sr6 - 1.0);
+                        ww += wgt * rsq * force;
+                    }
+                }
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    g[d] += __shfl_xor(g[d], 1, 64);
+                    g[d] += __shfl_xor(g[d], 2, 64);
+                    if ((b & 3) == a) mine[b >> 2][d] = g[d];
+                }
+            }
+            if (cj < ncj)
+#pragma unroll
+                for (int q = 0; q < N / 4; q++)
+#pragma unroll
+                    for (int d = 0; d < 3; d++)
+                        if (mine[q][d] != 0.0)
+                            atomicAdd(&f[3 * (size_t)(cj * N + 4 * q + a) + d], -mine[q][d]);
+        }
+        cj = cjn;
+    }
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+#pragma unroll
+        for (int o = 4; o < 64; o <<= 1)
+            fi[d] += __shfl_xor(fi[d], o, 64);
+        if (e == 0) atomicAdd(&f[3 * (size_t)si + d], fi[d]);
+    }
+    if (EV) ev_store(ee, ww, ev);
+}
+
 // What a force kernel that integrates needs to write its atoms' ghost images too.
 struct GhostOut {
     const int* cnt;  // images of each j-cluster, their first ghost, and the shifts; cnt null: none
@@ -3746,8 +3846,8 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
         grow_n(&C.d_sf64, &C.cap_sf64, 3 * nslots_all(), 0);
         if (failed()) return 0;
         if (half) fill_f64(C.d_sf64, 0.0, 3 * nslots_all());
-        const unsigned grid = full64 ? (blocks_for(nci, BLOCK / 64) + 7) & ~7u
-                                     : blocks_for((long long)nloc, BLOCK);
+        const unsigned grid = C.M == 4 ? (blocks_for(nci, BLOCK / 64) + 7) & ~7u
+                                       : blocks_for((long long)nloc, BLOCK);
         double* evp = ev_parts((size_t)grid * (BLOCK / 64));
         if (failed()) return 0;
         const int uni = C.uniform ? 1 : 0;
@@ -3771,22 +3871,32 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
 #define MDG_F64(MM, NN, H, E)                                                                    \
     k_cp_force_f64<MM, NN, H, E><<<grid, BLOCK, 0, s>>>(nci, C.ncj, C.ntypes, uni, C.t64, C.d_sx, \
         C.d_st, C.d_nb, C.d_numneigh, C.maxneighs, C.d_sf64, evp)
-#define MDG_F64_SHAPE(MM, NN)                                                                    \
+#define MDG_F64H(NN, E, U)                                                                       \
+    k_cp_force_f64_half<NN, E, U><<<grid, BLOCK, 0, s>>>(nci, C.ncj, C.ntypes, C.t64, C.d_sx,      \
+        C.d_st, C.d_nb, C.d_numneigh, C.maxneighs, C.d_sf64, evp)
+#define MDG_F64H_N(NN)                                                                           \
     do {                                                                                         \
-        if (C.ev_on) MDG_F64(MM, NN, true, true);                                                \
-        else MDG_F64(MM, NN, true, false);                                                       \
+        if (C.ev_on) {                                                                           \
+            if (C.uniform) MDG_F64H(NN, true, true);                                             \
+            else MDG_F64H(NN, true, false);                                                      \
+        } else {                                                                                 \
+            if (C.uniform) MDG_F64H(NN, false, true);                                            \
+            else MDG_F64H(NN, false, false);                                                     \
+        }                                                                                        \
     } while (0)
         if (full64) {
             if (C.N == 4) MDG_F64C_N(4);
             else MDG_F64C_N(8);
-        } else if (C.M == 4 && C.N == 4) MDG_F64_SHAPE(4, 4);
-        else if (C.M == 4 && C.N == 8) MDG_F64_SHAPE(4, 8);
-        else if (half) MDG_F64_SHAPE(1, 2);
+        } else if (C.M == 4 && C.N == 4) MDG_F64H_N(4);
+        else if (C.M == 4) MDG_F64H_N(8);
+        else if (half && C.ev_on) MDG_F64(1, 2, true, true);
+        else if (half) MDG_F64(1, 2, true, false);
         else if (C.ev_on) MDG_F64(1, 2, false, true);
         else MDG_F64(1, 2, false, false);
 #undef MDG_F64C_N
 #undef MDG_F64C
-#undef MDG_F64_SHAPE
+#undef MDG_F64H_N
+#undef MDG_F64H
 #undef MDG_F64
         C.forces_are_f32 = false;
     } else {

@@ -33,6 +33,36 @@ def test_fp64_full_list_forces_equal_oracle(N, nx):
 
 @pytest.mark.parametrize("mixture", [0, 1], ids=["lj", "ka"])
 @pytest.mark.parametrize("N", [4, 8])
+@pytest.mark.parametrize("nx", [4, 9])
+def test_fp64_half_list_forces_equal_full_list_forces(nx, N, mixture):
+    """The same clusters with half and with full lists: sums of the same ~60 FP64 pair forces in
+    another order (atomics), energies of the same pairs."""
+    out = []
+    for half in (0, 1):
+        sim = product().CPSim(nx=nx, ny=nx + 1, nz=nx, cluster_m=4, cluster_n=N, precision=1, ntimes=0,
+                              half_neigh=half, **(MIX if mixture else dict(temp=0.5)))
+        try:
+            if half:
+                sim.set_atoms(*atoms)
+            else:
+                sim.run(15)
+                sim.run(1)
+                product().lib().updateSingleAtomsGFX950(C.c_void_p(sim.param_p),
+                                                        C.c_void_p(sim.atom_p))
+                atoms = [sim.get("atoms_" + k).copy() for k in ("x", "v", "type")]
+                sim.set_atoms(*atoms)
+            live = _live_slots(sim.get("ci_natoms"), 4)
+            out.append((sim.get("slot_f").reshape(-1, 3)[live], *sim.energy_virial()))
+        finally:
+            sim.close()
+    (ff, ef, wf), (fh, eh, wh) = out
+    assert np.linalg.norm(ff) > 10.0
+    assert np.linalg.norm(fh - ff) < 1e-12 * np.linalg.norm(ff)
+    assert abs(eh - ef) <= 1e-11 * abs(ef) and abs(wh - wf) <= 1e-11 * max(abs(wf), abs(ef))
+
+
+@pytest.mark.parametrize("mixture", [0, 1], ids=["lj", "ka"])
+@pytest.mark.parametrize("N", [4, 8])
 def test_fp64_fused_run_equals_traced_run(N, mixture):
     """The kicks and the drift inside the FP64 force call are the separate calls' operations (a
     traced run makes those): positions, velocities and forces equal to the bit over rebuilds."""
