@@ -178,7 +178,8 @@ def bench_vl(args, mod, resort=0):
                        "atoms": natoms, "avg_neighbors": sum_nn / nlocal},
             "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": None,
-                         "kernel": "k_force_lj (fast, 4 lanes/atom)",
+                         "kernel": "k_force_lj_staged (positions in LDS) where a block's neighbours "
+                                   "fit, else k_force_lj (4 lanes/atom)",
                          "avg_launch_ms": avg_ms, "launches": nl.value,
                          "bytes_per_launch": bytes_launch, "bytes_basis": "compulsory",
                          "model_bytes_per_launch": model_bytes,
@@ -351,7 +352,7 @@ def bench_eam(args, mod, nx=32, resort=0):
                        "atoms": natoms, "avg_neighbors": sum_nn / nlocal},
             "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": None,
-                         "kernel": "k_eam_density_tab + k_eam_force_tab (4 lanes/atom, spline rows in LDS)",
+                         "kernel": "k_eam_density_tab + k_ghost_rows + k_eam_force_tab (4 lanes/atom, spline rows in LDS)",
                          "avg_launch_ms": avg_ms, "launches": nl.value,
                          "bytes_per_launch": bytes_launch},
         }
