@@ -1125,7 +1125,7 @@ __global__ void __launch_bounds__(BLOCK) k_force_lj(int nlocal, const double* __
 // only hints: a pair uses the staged position only if the staged atom is the one its list entry
 // names, and loads it from memory otherwise (a list written by someone else, a region with more than
 // STAGE_CAP distinct neighbours).  1.05 M atoms: 276 us per call with the positions gathered, 192
-// staged (60 % of the VALU's time and half the LDS's; the list and hints at 2.5 TB/s).  The two blocks
+// staged, bound by HBM (676 MB a call at 3.5 TB/s, 480 of them list and hints; VALU 60 %).  The two blocks
 // that a CU's LDS and waves hold set STAGE_CAP; a 256-atom lattice block names 1300 - 1700.  Blocks
 // of 512 threads and 128 atoms took the same, three or four sets of entries ahead too.
 constexpr int STAGE_T = 1024, STAGE_A = 256, STAGE_CAP = 2000, STAGE_LOG = 10;
