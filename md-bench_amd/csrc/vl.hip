@@ -27,7 +27,7 @@ constexpr int BLOCK     = 256;
 constexpr int MAXTYPES2 = 64;  // ntypes <= 8
 // LJ passes of full lists stage their neighbours' positions in LDS (k_force_lj_staged, k_stage_build)
 // above STAGE_MIN atoms, where the list is kept for STAGE_USES force calls or more: at 1.05 M atoms a
-// call gains 84 us and the tables cost 300 us per list; whole steps with a list per 20 measured 323 us
+// call gains 84 us and the tables cost 250 us per list; whole steps with a list per 20 measured 323 us
 // without and 255 with, at 702 k atoms 218 and 170, at 562 k 148 and 137, at 500 k (the list just fits
 // the last-level cache) 126 and 127.
 constexpr int STAGE_MIN = 520000, STAGE_USES = 8, STAGE_RETRY = 32;
@@ -1133,9 +1133,9 @@ constexpr int STAGE_T = 1024, STAGE_A = 256, STAGE_CAP = 2000, STAGE_LOG = 10;
 // tab: STAGE_CAP atoms per block, tab_n: how many (0: too many), hint[k * nlocal + i]: the place.
 // Atoms are taken by pages of 64: a block's neighbours lie in a hundred or two of them, found in a
 // small hash table; a page's members are bits of a word, so that a list entry is entered with an OR
-// and an atom's place is its page's first plus the members below it (pages in table order).  LDS
-// atomics bound it: 285 - 305 us at 1.05 M atoms (800 us for the list itself), 322 where every entry
-// is an OR without the read before it.
+// and an atom's place is its page's first plus the members below it (pages in table order).  LDS and
+// the lists' two readings bound it: 252 us at 1.05 M atoms (800 us for the list itself), 17 more where
+// every entry is an OR without the read before it.
 __global__ void __launch_bounds__(STAGE_T) k_stage_build(int nlocal,
     const int* __restrict__ neighbors, const int* __restrict__ numneigh, int maxneighs,
     int* __restrict__ tab, int* __restrict__ tab_n, unsigned short* __restrict__ hint,
@@ -1172,8 +1172,20 @@ __global__ void __launch_bounds__(STAGE_T) k_stage_build(int nlocal,
         else if (!(__hip_atomic_load(&s_bits[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & bit))
             atomicOr(&s_bits[h], bit);
     };
-    for (int k = lane; k < nn; k += LPA)
-        enter(neighbors[(size_t)k * nlocal + i]);
+    // (list entries two ahead in two registers: 305 -> 252 us; four: 255)
+    auto walk = [&](auto use) {
+        ListWalk<LPA> list(neighbors, nlocal, i < nlocal ? i : 0, lane, nn);
+        int ja = list.next(lane), jb = list.next(lane + LPA);
+        for (int k = lane; k < nn; k += 2 * LPA) {
+            const int j0 = ja;
+            ja           = list.next(k + 2 * LPA);
+            use(k, j0);
+            const int j1 = jb;
+            jb           = list.next(k + 3 * LPA);
+            if (k + LPA < nn) use(k + LPA, j1);
+        }
+    };
+    walk([&](int, int j) { enter(j); });
     __syncthreads();
     unsigned long long bits = s_bits[threadIdx.x];
     int n;
@@ -1196,8 +1208,7 @@ __global__ void __launch_bounds__(STAGE_T) k_stage_build(int nlocal,
             h = (h + 1) & (SLOTS - 1);
         return (unsigned short)(s_first[h] + __popcll(s_bits[h] & ((1ull << (j & 63)) - 1)));
     };
-    for (int k = lane; k < nn; k += LPA)
-        hint[(size_t)k * nlocal + i] = place(neighbors[(size_t)k * nlocal + i]);
+    walk([&](int k, int j) { hint[(size_t)k * nlocal + i] = place(j); });
 }
 
 // LJ, full lists, fast, without energies: the pairs, their order and arithmetic are those of
