@@ -11,13 +11,15 @@
 //                           16 list entries side by side, the reference kernel's arithmetic and
 //                           order of sums (computeForceLJRef, src/clusterpair/force_lj.c:22-189),
 //                           bit-identical to it; the run loop's kicks and drift fused in.
-//   k_cp_force_f64          the same arithmetic, one thread per i-slot: half lists and 1x2
-//                           clusters.
+//   k_cp_force_f64_half     FP64, half lists of i-clusters of four: the same lanes, a j-atom's forces
+//                           summed over them before its atomics.
+//   k_cp_force_f64          the same arithmetic, one thread per i-slot: 1x2 clusters.
 //   k_cp_force_f32_full     FP32-mixed, full lists: one wavefront per four i-clusters, one
 //                           j-atom per lane against the group's four i-atoms, j-atoms read as
 //                           16-byte FP32 records (offset in a power-of-two grid cell, cell bytes
 //                           and type), the cutoff decided as in FP64 (a band re-check); with the
-//                           run loop's final kick, next half kick and drift fused in.
+//                           run loop's final kick, next half kick and drift fused in; small
+//                           systems: one wavefront per i-cluster, the ghosts moved too.
 //   k_cp_force_half_tiled   FP32-mixed, half lists: one block per tile of 16 i-clusters, the
 //   + k_cp_gather_half      tile's j-forces summed in LDS as 64-bit fixed point and written once
 //                           per tile, then added per atom in record order (no atomics).

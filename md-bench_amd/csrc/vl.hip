@@ -2324,15 +2324,13 @@ static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
     K<<<G, T, 0, stream()>>>(nlocal, S.xs_ld, S.d_xs, atom->d_atom.type, S.ntypes, S.tab,        \
         S.uniform ? 1 : 0, cnmax, S.g.mbins, S.d_binstart, S.d_binatoms, S.d_stencil,            \
         S.nstencil, neighbor->half_neigh, neighbor->maxneighs, neighbor->d_neighbor.neighbors,   \
-        neighbor->d_neighbor.numneigh, S.d_status __VA_ARGS__)
-#define MDG_COMMA ,
+        neighbor->d_neighbor.numneigh, __VA_ARGS__)
     if (nlocal <= NB_SMALL) {
         S.h_flag[HF_OVERFLOW] = S.h_flag[HF_RANGE] = 0;  // (no earlier list build is running)
-        MDG_NB(k_build_neighbor, S.g.mbins, NB_T, MDG_COMMA S.h_flag MDG_COMMA go);
+        MDG_NB(k_build_neighbor, S.g.mbins, NB_T, S.d_status, S.h_flag, go);
     } else {
-        MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK);
+        MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK, S.d_status);
     }
-#undef MDG_COMMA
 #undef MDG_NB
     MDG_LAUNCH_CHECK("build_neighbor");
 }
