@@ -231,20 +231,28 @@ struct Prd {
     double p[3];
 };
 
-__global__ void k_ghost_count(int nlocal, const double* __restrict__ x, Prd prd, double cut,
-    int* __restrict__ cnt)
+// (wrap: the atom back into the box first, as k_wrap does)
+__global__ void k_ghost_count(int nlocal, double* __restrict__ x, Prd prd, double cut,
+    int* __restrict__ cnt, int wrap)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nlocal) return;
     double xi[3] = { x[3 * i], x[3 * i + 1], x[3 * i + 2] };
-    cnt[i]       = __popc(ghost_mask(xi, prd.p, cut));
+    if (wrap)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            if (xi[d] < 0.0) x[3 * i + d] = xi[d] += prd.p[d];
+            else if (xi[d] >= prd.p[d]) x[3 * i + d] = xi[d] -= prd.p[d];
+        }
+    cnt[i] = __popc(ghost_mask(xi, prd.p, cut));
 }
 
 // (the ghosts' positions too, as k_update_pbc writes them)
 __global__ void k_ghost_fill(int nlocal, double* x, Prd prd, double cut,
     const int* __restrict__ off, int* __restrict__ border_map, int* __restrict__ pbc,
-    int* __restrict__ type)
+    int* __restrict__ type, const int* __restrict__ go = nullptr)
 {
+    if (go && !*go) return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nlocal) return;
     double xi[3] = { x[3 * i], x[3 * i + 1], x[3 * i + 2] };
@@ -264,6 +272,13 @@ __global__ void k_ghost_fill(int nlocal, double* x, Prd prd, double cut,
         type[nlocal + g] = ti;
         g++;
     }
+}
+
+// After a ghost count: whether room suffices (see k_ghost_setup), and clean words for the list build
+__global__ void k_ghost_go(int room, int* __restrict__ status, int* __restrict__ go)
+{
+    status[0] = status[1] = 0;
+    *go       = status[2] <= room;
 }
 
 // The ghosts' counts and offsets of a small system in one block (and, with wrap, the atoms' return
@@ -362,11 +377,13 @@ __global__ void k_update_pbc(int nlocal, int nghost, double* __restrict__ x,
 // ---------------------------------------------------------------- binning (neighbor.c:386-464)
 // Each atom's bin and its place among the bin's atoms as they arrive (one atomic per atom: with a
 // second one in the scatter the two took 29 us each at 1M atoms).
-__global__ void k_bin_count(int nall, const double* __restrict__ x, Grid g, int* __restrict__ bin_of,
-    int* __restrict__ place, int* __restrict__ count, int* __restrict__ status)
+__global__ void k_bin_count(int nlocal, const int* __restrict__ nghost, const double* __restrict__ x, Grid g, int* __restrict__ bin_of,
+    int* __restrict__ place, int* __restrict__ count, int* __restrict__ status,
+    const int* __restrict__ go)
 {
+    if (go && !*go) return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nall) return;
+    if (i >= nlocal + (nghost ? *nghost : 0)) return;
     int b = coord2bin(g, x[3 * i], x[3 * i + 1], x[3 * i + 2]);
     if (b < 0 || b >= g.mbins) {
         atomicOr(&status[0], ST_BIN_RANGE);
@@ -377,11 +394,13 @@ __global__ void k_bin_count(int nall, const double* __restrict__ x, Grid g, int*
     place[i]  = atomicAdd(&count[b], 1);
 }
 
-__global__ void k_bin_scatter(int nall, const int* __restrict__ bin_of,
-    const int* __restrict__ place, const int* __restrict__ binstart, int* __restrict__ slots)
+__global__ void k_bin_scatter(int nlocal, const int* __restrict__ nghost, const int* __restrict__ bin_of,
+    const int* __restrict__ place, const int* __restrict__ binstart, int* __restrict__ slots,
+    const int* __restrict__ go)
 {
+    if (go && !*go) return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nall) return;
+    if (i >= nlocal + (nghost ? *nghost : 0)) return;
     int b = bin_of[i];
     if (b < 0) return;
     slots[binstart[b] + place[i]] = i;
@@ -741,13 +760,14 @@ __global__ void __launch_bounds__(BLOCK) k_build_neighbor_wave(int nlocal, int l
     const double* __restrict__ xs, const int* __restrict__ type, int ntypes, Tables tab, int uniform,
     double cnmax, int mbins, const int* __restrict__ binstart, const int* __restrict__ binatoms,
     const int* __restrict__ stencil, int nstencil, int half, int maxneighs,
-    int* __restrict__ neighbors, int* __restrict__ numneigh, int* __restrict__ status)
+    int* __restrict__ neighbors, int* __restrict__ numneigh, int* __restrict__ status,
+    const int* __restrict__ go)
 {
     __shared__ int s_c[BLOCK / 64][NBW_SEG];
     __shared__ __align__(16) NbLocal s_l[BLOCK / 64][NB_Q];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64) + w);
-    if (b >= mbins) return;
+    if (b >= mbins || (go && !*go)) return;
     const int beg = binstart[b], end = binstart[b + 1];
     if (beg >= end || binatoms[beg] >= nlocal) return;
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -2194,6 +2214,43 @@ void setupNeighborGFX950(Parameter* param)
 }
 
 // clear_status: the two words of the list build's status zeroed on the way
+// Room for the bins of n atoms
+static void grow_bins(size_t n)
+{
+    const size_t mb = (size_t)S.g.mbins, cap0 = S.cap_bins;
+    grow_n(&S.d_binplace, &S.cap_binplace, n, 0);
+    grow_n(&S.d_xs, &S.cap_xs, 3 * n, 0);
+    grow_n(&S.d_bin_of, &S.cap_bin_of, n, 0);
+    grow_n(&S.d_bincount, &S.cap_bins, mb + 1, 0);
+    grow_n(&S.d_binstart, &S.cap_binstart, mb + 1, 0);
+    grow_n(&S.d_binatoms, &S.cap_binatoms, n + 1, 0);
+    grow_n(&S.d_binslots, &S.cap_binslots, n + 1, 0);
+    if (failed()) return;
+    // (all zero between binnings: the scan clears them)
+    if (S.cap_bins != cap0) fill_i32(S.d_bincount, 0, S.cap_bins);
+}
+
+// Launches the binning of nlocal and *nghost atoms (null: none), max_n at most.
+static void launch_bins(int nlocal, const int* nghost, int max_n, const double* x, bool clear,
+    const int* go)
+{
+    const int mb = S.g.mbins;
+    if (max_n <= BIN1_N && mb <= BIN1_BINS) {
+        launch_bins_small(nlocal, nghost, max_n, x, clear, go);
+        return;
+    }
+    hipStream_t s       = stream();
+    const unsigned grid = blocks_for(max_n, BLOCK);
+    k_bin_count<<<grid, BLOCK, 0, s>>>(nlocal, nghost, x, S.g, S.d_bin_of, S.d_binplace,
+        S.d_bincount, S.d_status, go);
+    exclusive_scan_take(S.d_bincount, S.d_binstart, mb, S.d_binstart + mb);
+    k_bin_scatter<<<grid, BLOCK, 0, s>>>(nlocal, nghost, S.d_bin_of, S.d_binplace, S.d_binstart,
+        S.d_binslots, go);
+    k_bin_rank<<<grid, BLOCK, 0, s>>>(S.xs_ld, S.d_bin_of, S.d_binstart, S.d_binslots, x,
+        S.d_binatoms, S.d_xs, S.d_binstart + mb, clear ? S.d_status : nullptr, go);
+    MDG_LAUNCH_CHECK("binatoms");
+}
+
 static void bin_atoms(Atom* atom, bool clear_status)
 {
     if (failed() || !S.ready || S.g.mbins == 0) {
@@ -2201,35 +2258,12 @@ static void bin_atoms(Atom* atom, bool clear_status)
         return;
     }
     TimedRegion tr(F_BINNING);
-    int nall = atom->Nlocal + atom->Nghost;
-    int mb   = S.g.mbins;
-    const size_t cap0 = S.cap_bins;
-    grow_n(&S.d_binplace, &S.cap_binplace, (size_t)nall, 0);
-    grow_n(&S.d_xs, &S.cap_xs, 3 * (size_t)nall, 0);
-    grow_n(&S.d_bin_of, &S.cap_bin_of, (size_t)nall, 0);
-    grow_n(&S.d_bincount, &S.cap_bins, (size_t)mb + 1, 0);
-    grow_n(&S.d_binstart, &S.cap_binstart, (size_t)mb + 1, 0);
-    grow_n(&S.d_binatoms, &S.cap_binatoms, (size_t)nall + 1, 0);
-    grow_n(&S.d_binslots, &S.cap_binslots, (size_t)nall + 1, 0);
+    const int nall = atom->Nlocal + atom->Nghost;
+    grow_bins((size_t)nall);
     if (failed()) return;
-    hipStream_t s = stream();
-    S.xs_ld       = nall;
-    S.binned      = true;
-    if (nall <= BIN1_N && mb <= BIN1_BINS) {
-        launch_bins_small(nall, nullptr, nall, atom->d_atom.x, clear_status, nullptr);
-        return;
-    }
-    // (all zero between binnings: the scan clears them)
-    if (S.cap_bins != cap0) fill_i32(S.d_bincount, 0, S.cap_bins);
-    k_bin_count<<<blocks_for(nall, BLOCK), BLOCK, 0, s>>>(nall, atom->d_atom.x, S.g, S.d_bin_of,
-        S.d_binplace, S.d_bincount, S.d_status);
-    exclusive_scan_take(S.d_bincount, S.d_binstart, mb, S.d_binstart + mb);
-    k_bin_scatter<<<blocks_for(nall, BLOCK), BLOCK, 0, s>>>(nall, S.d_bin_of, S.d_binplace,
-        S.d_binstart, S.d_binslots);
-    k_bin_rank<<<blocks_for(nall, BLOCK), BLOCK, 0, s>>>(nall, S.d_bin_of, S.d_binstart,
-        S.d_binslots, atom->d_atom.x, S.d_binatoms, S.d_xs, S.d_binstart + mb,
-        clear_status ? S.d_status : nullptr);
-    MDG_LAUNCH_CHECK("binatoms");
+    S.xs_ld  = nall;
+    S.binned = true;
+    launch_bins(nall, nullptr, nall, atom->d_atom.x, clear_status, nullptr);
 }
 
 void binatomsGFX950(Atom* atom) { bin_atoms(atom, false); }
@@ -2329,24 +2363,24 @@ static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
         S.h_flag[HF_OVERFLOW] = S.h_flag[HF_RANGE] = 0;  // (no earlier list build is running)
         MDG_NB(k_build_neighbor, S.g.mbins, NB_T, S.d_status, S.h_flag, go);
     } else {
-        MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK, S.d_status);
+        MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK, S.d_status, go);
     }
 #undef MDG_NB
     MDG_LAUNCH_CHECK("build_neighbor");
 }
 
 // Waits for the list build; false: the lists were too short and have been given more room.
-static bool lists_done(int nlocal, Neighbor* neighbor)
+static bool lists_done(int nlocal, Neighbor* neighbor, bool waited = false)
 {
     bool range, overflow;
     if (nlocal <= NB_SMALL) {
-        MDG_HIP(hipStreamSynchronize(stream()));
+        if (!waited) MDG_HIP(hipStreamSynchronize(stream()));
         if (failed()) return true;
         range    = S.h_flag[HF_RANGE] != 0;
         overflow = S.h_flag[HF_OVERFLOW] != 0;
         if (overflow) read_status();  // the longest list
     } else {
-        read_status();
+        if (!waited) read_status();
         range    = (S.h_status[0] & ST_BIN_RANGE) != 0;
         overflow = (S.h_status[0] & ST_NB_OVERFLOW) != 0;
     }
@@ -2401,7 +2435,7 @@ void setupPbcGFX950(Atom* atom, Parameter* param)
         nghost = S.h_flag[HF_TOTAL];
     } else {
         k_ghost_count<<<blocks_for(nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x, prd,
-            param->cutneigh, S.d_gcnt);
+            param->cutneigh, S.d_gcnt, 0);
         exclusive_scan(S.d_gcnt, S.d_goff, nlocal, S.d_status + 2);
         read_status();
         if (failed()) return;
@@ -2440,18 +2474,20 @@ void setupPbcGFX950(Atom* atom, Parameter* param)
     S.ghosts_current = true;
 }
 
-// A run's rebuild: updateAtomsPbcGFX950, setupPbcGFX950, updatePbcGFX950 and buildNeighborGFX950.  Of a
-// small system whose buffers have room for its ghosts, everything is launched before the host waits
-// (once, for the lists): the launches behind the ghosts' count take it from device memory.  With the
-// kernels of few launches a rebuild takes 16 us less for 256 atoms (of about 75) and 25 for 4000.
+// A run's rebuild: updateAtomsPbcGFX950, setupPbcGFX950, updatePbcGFX950 and buildNeighborGFX950.  Where
+// the buffers have room for the ghosts, everything is launched before the host waits (once, for the
+// lists): the launches behind the ghosts' count take it from device memory, and do nothing if the
+// room turns out too small.  With the small systems' kernels of few launches a rebuild takes 16 us
+// less for 256 atoms (of about 75) and 25 for 4000; larger ones 8 less at 11,000 atoms, 14 at 62,000 and
+// 131,000, 27 (of 1200, a force call included) at 1.05 M.
 void mdg_vl_reneighbour(Parameter* param, Atom* atom, Neighbor* neighbor)
 {
     if (failed() || !S.ready) return;
-    const int nlocal = atom->Nlocal;
-    const size_t ld  = std::min(S.cap_all, (size_t)BIN1_N);
+    const int nlocal = atom->Nlocal, mb = S.g.mbins;
+    const bool small = nlocal <= SETUP_SMALL && mb <= BIN1_BINS;
+    const size_t ld  = std::min(S.cap_all, (size_t)(small ? BIN1_N : INT_MAX / 3));
     const size_t room = std::min({ ld - std::min(ld, (size_t)nlocal), S.cap_ghost, S.cap_pbc / 3 });
-    const int mb = S.g.mbins;
-    if (nlocal <= 0 || nlocal > SETUP_SMALL || mb <= 0 || mb > BIN1_BINS || room == 0) {
+    if (nlocal <= 0 || mb <= 0 || room == 0) {
         updateAtomsPbcGFX950(atom, param, true);
         setupPbcGFX950(atom, param);
         if (!S.ghosts_current) updatePbcGFX950(atom, param, true);
@@ -2465,32 +2501,40 @@ void mdg_vl_reneighbour(Parameter* param, Atom* atom, Neighbor* neighbor)
     const Prd prd{ { param->xprd, param->yprd, param->zprd } };
     grow_n(&S.d_gcnt, &S.cap_gcnt, (size_t)nlocal + 1, 0);
     grow_n(&S.d_goff, &S.cap_goff, (size_t)nlocal + 1, 0);
-    grow_n(&S.d_xs, &S.cap_xs, 3 * ld, 0);
-    grow_n(&S.d_bin_of, &S.cap_bin_of, ld, 0);
-    grow_n(&S.d_binslots, &S.cap_binslots, ld + 1, 0);
-    grow_n(&S.d_binstart, &S.cap_binstart, (size_t)mb + 1, 0);
-    grow_n(&S.d_binatoms, &S.cap_binatoms, ld + 1, 0);
+    grow_bins(ld);
     if (failed()) return;
     hipStream_t s = stream();
     int* go       = S.d_status + 4;
-    {
+    DeviceAtom* d = &atom->d_atom;
+    if (small) {
         TimedRegion tr(F_PBC);
-        k_ghost_setup<<<1, SETUP_T, 0, s>>>(nlocal, atom->d_atom.x, 1, prd, param->cutneigh, S.d_gcnt,
-            S.d_goff, S.d_status, (int)room, go, S.h_flag);
-        k_ghost_fill_small<<<blocks_for(32LL * nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, atom->d_atom.x,
-            prd, param->cutneigh, S.d_goff, atom->d_atom.border_map, S.d_pbc, atom->d_atom.type, go);
+        k_ghost_setup<<<1, SETUP_T, 0, s>>>(nlocal, d->x, 1, prd, param->cutneigh, S.d_gcnt, S.d_goff,
+            S.d_status, (int)room, go, S.h_flag);
+        k_ghost_fill_small<<<blocks_for(32LL * nlocal, BLOCK), BLOCK, 0, s>>>(nlocal, d->x, prd,
+            param->cutneigh, S.d_goff, d->border_map, S.d_pbc, d->type, go);
+        MDG_LAUNCH_CHECK("ghost_setup");
+    } else {
+        TimedRegion tr(F_PBC);
+        const unsigned grid = blocks_for(nlocal, BLOCK);
+        k_ghost_count<<<grid, BLOCK, 0, s>>>(nlocal, d->x, prd, param->cutneigh, S.d_gcnt, 1);
+        exclusive_scan(S.d_gcnt, S.d_goff, nlocal, S.d_status + 2);
+        k_ghost_go<<<1, 1, 0, s>>>((int)room, S.d_status, go);
+        k_ghost_fill<<<grid, BLOCK, 0, s>>>(nlocal, d->x, prd, param->cutneigh, S.d_goff,
+            d->border_map, S.d_pbc, d->type, go);
         MDG_LAUNCH_CHECK("ghost_setup");
     }
     {
         TimedRegion tr(F_BINNING);
-        launch_bins_small(nlocal, S.d_status + 2, (int)ld, atom->d_atom.x, true, go);
+        launch_bins(nlocal, S.d_status + 2, (int)ld, d->x, true, go);
     }
     if (failed()) return;
     launch_lists(atom, neighbor, go);
     if (failed()) return;
-    MDG_HIP(hipStreamSynchronize(s));
+    const bool flags = nlocal <= NB_SMALL;  // (lists_done's two ways)
+    if (small && flags) MDG_HIP(hipStreamSynchronize(s));
+    else read_status();
     if (failed()) return;
-    const int nghost = S.h_flag[HF_TOTAL];
+    const int nghost = small ? S.h_flag[HF_TOTAL] : S.h_status[2];
     if ((size_t)nghost > room) {  // nothing was built (the atoms are in the box)
         setupPbcGFX950(atom, param);
         buildNeighborGFX950(atom, neighbor);
@@ -2501,7 +2545,7 @@ void mdg_vl_reneighbour(Parameter* param, Atom* atom, Neighbor* neighbor)
     S.gmap_nghost    = nghost;
     S.ghosts_current = true;
     S.binned         = true;
-    for (int attempt = 1; !lists_done(nlocal, neighbor); attempt++) {
+    for (int attempt = 1; !lists_done(nlocal, neighbor, attempt == 1); attempt++) {
         if (attempt == 8) {
             set_error(MDG_ERR_CAPACITY, "neighbour list did not converge");
             return;
