@@ -84,7 +84,8 @@ void binatomsGFX950(Atom* atom);
    that follows uses the atom's own force. */
 void sortAtomGFX950(Atom* atom);
 /* replaces buildNeighborCUDA (src/verletlist/neighborCuda.cu:259-366) / buildNeighborCPU
-   (src/verletlist/neighbor.c:260-352); grows neighbor->maxneighs on overflow */
+   (src/verletlist/neighbor.c:260-352); grows neighbor->maxneighs on overflow.  An atom outside the
+   bin grid is MDG_ERR_BIN: its list has not been built. */
 void buildNeighborGFX950(Atom* atom, Neighbor* neighbor);
 /* replaces setupPbc (src/verletlist/pbc.c:103-232), on the device: same ghost order */
 void setupPbcGFX950(Atom* atom, Parameter* param);

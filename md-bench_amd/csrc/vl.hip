@@ -376,10 +376,12 @@ __global__ void k_update_pbc(int nlocal, int nghost, double* __restrict__ x,
 
 // ---------------------------------------------------------------- binning (neighbor.c:386-464)
 // Each atom's bin and its place among the bin's atoms as they arrive (one atomic per atom: with a
-// second one in the scatter the two took 29 us each at 1M atoms).
+// second one in the scatter the two took 29 us each at 1M atoms).  An atom outside the grid is in no
+// bin; it sets the status flag, and for a list build (host set) the host's word, which outlasts the
+// clearing of the status words on the way to the lists.
 __global__ void k_bin_count(int nlocal, const int* __restrict__ nghost, const double* __restrict__ x, Grid g, int* __restrict__ bin_of,
     int* __restrict__ place, int* __restrict__ count, int* __restrict__ status,
-    const int* __restrict__ go)
+    int* __restrict__ host, const int* __restrict__ go)
 {
     if (go && !*go) return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -387,6 +389,7 @@ __global__ void k_bin_count(int nlocal, const int* __restrict__ nghost, const do
     int b = coord2bin(g, x[3 * i], x[3 * i + 1], x[3 * i + 2]);
     if (b < 0 || b >= g.mbins) {
         atomicOr(&status[0], ST_BIN_RANGE);
+        if (host) host[HF_RANGE] = 1;
         bin_of[i] = -1;
         return;
     }
@@ -436,7 +439,7 @@ __global__ void k_bin_rank(int n, const int* __restrict__ bin_of, const int* __r
 // k_bin_rank's work.  n: nlocal plus the ghosts counted by k_ghost_setup where nghost is not null.
 // 256 atoms and 1500 ghosts: 15 us in four launches, 7.7 in one.  4000 atoms and 5500 ghosts: 25 us in
 // four launches, 17.5 in two, 24 in one (6 for the ranks and 9 for the writes, which many blocks share
-// better).
+// better).  host: set for a list build (see k_bin_count), which also has its status words cleared.
 constexpr int BIN1_T = 1024, BIN1_I = 16, BIN1_N = BIN1_T * BIN1_I, BIN1_BINS = 16384;
 constexpr int BIN1_ORDER = 4 * BIN1_T;
 
@@ -444,7 +447,8 @@ template <bool ORDER>
 __global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __restrict__ nghost,
     int ld, const double* __restrict__ x, Grid g, int* __restrict__ binstart,
     int* __restrict__ bin_of, int* __restrict__ slots, int* __restrict__ binatoms,
-    double* __restrict__ xs, int* __restrict__ status, int clear, const int* __restrict__ go)
+    double* __restrict__ xs, int* __restrict__ status, int* __restrict__ host,
+    const int* __restrict__ go)
 {
     constexpr int NI = ORDER ? BIN1_ORDER / BIN1_T : BIN1_I;
     __shared__ int s_bin[BIN1_BINS];  // atoms per bin, then the bins' starts
@@ -472,7 +476,8 @@ __global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __
         if (i >= n) continue;
         const int b = coord2bin(g, r[k & 3][0], r[k & 3][1], r[k & 3][2]);
         if (b < 0 || b >= g.mbins) {
-            if (!clear) atomicOr(&status[0], ST_BIN_RANGE);
+            if (host) host[HF_RANGE] = 1;
+            else atomicOr(&status[0], ST_BIN_RANGE);
             continue;
         }
         bin[k]   = b;
@@ -496,7 +501,7 @@ __global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __
         binstart[b] = s_bin[b];
     if (tid == 0) {
         binstart[g.mbins] = total;
-        if (clear) status[0] = status[1] = 0;
+        if (host) status[0] = status[1] = 0;
     }
 #pragma unroll
     for (int k = 0; k < NI; k++) {
@@ -522,16 +527,16 @@ __global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __
 }
 
 // Launches the binning of up to BIN1_N atoms (nlocal and *nghost), max_n at most, in few launches.
-void launch_bins_small(int nlocal, const int* nghost, int max_n, const double* x, bool clear,
+void launch_bins_small(int nlocal, const int* nghost, int max_n, const double* x, int* host,
     const int* go)
 {
     hipStream_t s = stream();
     if (max_n <= BIN1_ORDER) {
         k_bin_single<true><<<1, BIN1_T, 0, s>>>(nlocal, nghost, S.xs_ld, x, S.g, S.d_binstart,
-            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, S.d_status, clear, go);
+            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, S.d_status, host, go);
     } else {
         k_bin_single<false><<<1, BIN1_T, 0, s>>>(nlocal, nghost, S.xs_ld, x, S.g, S.d_binstart,
-            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, S.d_status, clear, go);
+            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, S.d_status, host, go);
         k_bin_rank<<<blocks_for(max_n, BLOCK), BLOCK, 0, s>>>(S.xs_ld, S.d_bin_of, S.d_binstart,
             S.d_binslots, x, S.d_binatoms, S.d_xs, S.d_binstart + S.g.mbins, nullptr, go);
     }
@@ -2213,7 +2218,6 @@ void setupNeighborGFX950(Parameter* param)
     S.binned = false;
 }
 
-// clear_status: the two words of the list build's status zeroed on the way
 // Room for the bins of n atoms
 static void grow_bins(size_t n)
 {
@@ -2230,28 +2234,32 @@ static void grow_bins(size_t n)
     if (S.cap_bins != cap0) fill_i32(S.d_bincount, 0, S.cap_bins);
 }
 
-// Launches the binning of nlocal and *nghost atoms (null: none), max_n at most.
-static void launch_bins(int nlocal, const int* nghost, int max_n, const double* x, bool clear,
+// Launches the binning of nlocal and *nghost atoms (null: none), max_n at most.  for_lists: the list
+// build follows; its status words are cleared on the way, and an atom outside the grid is reported by
+// lists_done (without it, by status word 0).
+static void launch_bins(int nlocal, const int* nghost, int max_n, const double* x, bool for_lists,
     const int* go)
 {
     const int mb = S.g.mbins;
+    int* host    = for_lists ? S.h_flag : nullptr;
+    if (for_lists) S.h_flag[HF_RANGE] = 0;  // (the host has waited for the last build that writes it)
     if (max_n <= BIN1_N && mb <= BIN1_BINS) {
-        launch_bins_small(nlocal, nghost, max_n, x, clear, go);
+        launch_bins_small(nlocal, nghost, max_n, x, host, go);
         return;
     }
     hipStream_t s       = stream();
     const unsigned grid = blocks_for(max_n, BLOCK);
     k_bin_count<<<grid, BLOCK, 0, s>>>(nlocal, nghost, x, S.g, S.d_bin_of, S.d_binplace,
-        S.d_bincount, S.d_status, go);
+        S.d_bincount, S.d_status, host, go);
     exclusive_scan_take(S.d_bincount, S.d_binstart, mb, S.d_binstart + mb);
     k_bin_scatter<<<grid, BLOCK, 0, s>>>(nlocal, nghost, S.d_bin_of, S.d_binplace, S.d_binstart,
         S.d_binslots, go);
     k_bin_rank<<<grid, BLOCK, 0, s>>>(S.xs_ld, S.d_bin_of, S.d_binstart, S.d_binslots, x,
-        S.d_binatoms, S.d_xs, S.d_binstart + mb, clear ? S.d_status : nullptr, go);
+        S.d_binatoms, S.d_xs, S.d_binstart + mb, for_lists ? S.d_status : nullptr, go);
     MDG_LAUNCH_CHECK("binatoms");
 }
 
-static void bin_atoms(Atom* atom, bool clear_status)
+static void bin_atoms(Atom* atom, bool for_lists)
 {
     if (failed() || !S.ready || S.g.mbins == 0) {
         if (!failed()) set_error(MDG_ERR_ARG, "binatomsGFX950 before setupNeighborGFX950");
@@ -2263,7 +2271,7 @@ static void bin_atoms(Atom* atom, bool clear_status)
     if (failed()) return;
     S.xs_ld  = nall;
     S.binned = true;
-    launch_bins(nall, nullptr, nall, atom->d_atom.x, clear_status, nullptr);
+    launch_bins(nall, nullptr, nall, atom->d_atom.x, for_lists, nullptr);
 }
 
 void binatomsGFX950(Atom* atom) { bin_atoms(atom, false); }
@@ -2360,7 +2368,7 @@ static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
         S.nstencil, neighbor->half_neigh, neighbor->maxneighs, neighbor->d_neighbor.neighbors,   \
         neighbor->d_neighbor.numneigh, __VA_ARGS__)
     if (nlocal <= NB_SMALL) {
-        S.h_flag[HF_OVERFLOW] = S.h_flag[HF_RANGE] = 0;  // (no earlier list build is running)
+        S.h_flag[HF_OVERFLOW] = 0;  // (no earlier list build is running)
         MDG_NB(k_build_neighbor, S.g.mbins, NB_T, S.d_status, S.h_flag, go);
     } else {
         MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK, S.d_status, go);
@@ -2369,14 +2377,15 @@ static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
     MDG_LAUNCH_CHECK("build_neighbor");
 }
 
-// Waits for the list build; false: the lists were too short and have been given more room.
+// Waits for the list build; false: the lists were too short and have been given more room.  An atom
+// outside the grid is an error: it is in no bin, and its own list has not been written.
 static bool lists_done(int nlocal, Neighbor* neighbor, bool waited = false)
 {
     bool range, overflow;
     if (nlocal <= NB_SMALL) {
         if (!waited) MDG_HIP(hipStreamSynchronize(stream()));
         if (failed()) return true;
-        range    = S.h_flag[HF_RANGE] != 0;
+        range    = false;
         overflow = S.h_flag[HF_OVERFLOW] != 0;
         if (overflow) read_status();  // the longest list
     } else {
@@ -2385,7 +2394,7 @@ static bool lists_done(int nlocal, Neighbor* neighbor, bool waited = false)
         overflow = (S.h_status[0] & ST_NB_OVERFLOW) != 0;
     }
     if (failed()) return true;
-    if (range) {
+    if (range || S.h_flag[HF_RANGE]) {
         set_error(MDG_ERR_BIN, "an atom lies outside the bin grid (coord2bin out of range)");
         return true;
     }

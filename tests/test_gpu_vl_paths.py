@@ -341,3 +341,54 @@ def test_eam_tables_too_long_for_lds(dims, tmp_path):
         _ghosts_follow_owners(sim, st)
     finally:
         sim.close()
+
+
+def _put(sim, x):
+    """The sim's local atoms to x, without ghosts."""
+    nl = sim.atom.Nlocal
+    np.ctypeslib.as_array(sim.atom.x, (3 * nl,))[:] = x
+    sim.atom.Nghost = 0  # the host copies hold the local atoms only
+    product().lib().copyDataToGFX950Device(sim.param_p, sim.atom_p)
+
+
+@pytest.mark.parametrize("call", ["calls", "run"])
+@pytest.mark.parametrize("dims", [(4, 4, 4), (10, 10, 10), (16, 16, 16), (19, 18, 19)], ids=str)
+def test_atom_outside_the_grid_is_an_error(dims, call):
+    """An atom many boxes away is in no bin, so its list would stay the last one: the rebuild says so,
+    by the separate calls and inside a run, at each of the binnings and list builds; no force call
+    follows it.  With the atom back the next rebuild gives the oracle's lists."""
+    P = product()
+    L = P.lib()
+    print(dims, call, flush=True)
+    sim = P.VLSim(nx=dims[0], ny=dims[1], nz=dims[2], reneigh_every=1)
+    try:
+        p = sim.param
+        nl = sim.atom.Nlocal
+        good = sim.state(lists=False)["x"][:3 * nl].copy()
+        far = good.copy()
+        far[3 * 7 + 2] += 50 * p.zprd
+
+        def rebuild():
+            if call == "run":
+                return L.mdbVLRun(sim.h, 1, None)
+            L.updateAtomsPbcGFX950(sim.atom_p, sim.param_p, True)
+            L.setupPbcGFX950(sim.atom_p, sim.param_p)
+            L.updatePbcGFX950(sim.atom_p, sim.param_p, True)
+            L.buildNeighborGFX950(sim.atom_p, sim.neighbor_p)
+            return P.status()[0]
+
+        _put(sim, far)
+        assert rebuild() == 2  # MDG_ERR_BIN
+        assert "outside the bin grid" in P.status()[1]
+        L.mdgfx950ClearStatus()
+        _put(sim, good)
+        assert rebuild() == 0, P.status()
+        st = sim.state()
+        nn, nb = ob.build_neighbor(ob.vl_grid(*dims, p.lattice, p.cutneigh), nl, st["x"],
+                                   np.zeros(nl + st["nghost"], np.int32), 4,
+                                   np.full(16, p.cutneigh ** 2), 0, cap_per_atom=2000)
+        np.testing.assert_array_equal(st["numneigh"], nn)
+        np.testing.assert_array_equal(st["neighbors"], nb)
+    finally:
+        L.mdgfx950ClearStatus()
+        sim.close()
