@@ -1459,7 +1459,7 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64_half(int nci, int ncj, i
                 if ((cj != own || si < cj * N + b) && rsq < cut) {
                     const double eps   = UNIFORM ? tab.eps[0] : s_tab[0][tij];
                     const double sig6  = UNIFORM ? tab.sig6[0] : s_tab[1][tij];
-                    const double sr2   = EV ? 1.0 / rsq : recip_normal(rsq);
+                    const double sr2   = 1.0 / rsq;
                     const double sr6   = sr2 * sr2 * sr2 * sig6;
                     const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
 #pragma unroll
@@ -1517,8 +1517,8 @@ struct GhostOut {
 // One thread per i-slot walking its whole list (k_cp_force_f64, still the half lists' and the
 // 1x2 clusters' kernel) took 148 us for 34,960 atoms of the Kob-Andersen mixture, 547 wavefronts
 // waiting on their lists; this takes 24.6 us, kicks and drift included (9.9 us in launches of
-// their own before).  Bound now: FP64 instructions (the exact division of the pairs inside the
-// cutoff above all).
+// their own before).  Bound: FP64 instructions.  With energies the pairs divide, without them they take
+// the correctly rounded reciprocal (recip_rounded), the same value.
 template <int N, bool EV, bool UNIFORM>
 __global__ void __launch_bounds__(BLOCK) k_cp_force_f64_full(int nci, int ntypes, Tab64 tab,
     const double* __restrict__ sx, const int* __restrict__ st, const int* __restrict__ nb,
@@ -1587,7 +1587,7 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64_full(int nci, int ntypes
                 if (cj * N + b != si && rsq < cut) {
                     const double eps   = UNIFORM ? tab.eps[0] : s_tab[0][tij];
                     const double sig6  = UNIFORM ? tab.sig6[0] : s_tab[1][tij];
-                    const double sr2   = EV ? 1.0 / rsq : recip_normal(rsq);
+                    const double sr2   = EV ? 1.0 / rsq : recip_rounded(rsq);
                     const double sr6   = sr2 * sr2 * sr2 * sig6;
                     const double force = 48.0 * sr6 * (sr6 - 0.5) * sr2 * eps;
                     fix += dx * force;

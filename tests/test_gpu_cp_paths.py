@@ -179,3 +179,51 @@ def test_atoms_to_and_from_the_device(nx):
             np.testing.assert_array_equal(a, b)
     finally:
         sim.close()
+
+
+def _pair_at(rsq, rng):
+    """A separation whose squared length, as the kernels and the oracle add it up, is rsq exactly."""
+    r = np.sqrt(rsq)
+    while True:
+        d = rng.standard_normal(3)
+        d[2] *= 1e-3
+        d = np.round(d * r / np.linalg.norm(d) * 2.0 ** 49) * 2.0 ** -49
+        d[1] = np.round(np.sqrt(max(rsq - d[0] ** 2 - 1e-5, 0.0)) * 2.0 ** 49) * 2.0 ** -49
+        rest = rsq - (d[0] * d[0] + d[1] * d[1])
+        if not 1e-6 < rest < 1e-4:
+            continue
+        z = np.round(np.sqrt(rest) * 2.0 ** 49)
+        for k in range(-64, 65):
+            d[2] = (z + k) * 2.0 ** -49
+            if d[0] * d[0] + d[1] * d[1] + d[2] * d[2] == rsq:
+                return d
+
+
+@pytest.mark.parametrize("N", [4, 8])
+def test_fp64_forces_equal_oracle_where_reciprocals_round_hardest(N):
+    """Squared distances a few units in the last place below a power of two, whose reciprocals lie next
+    to the middle of two doubles: two Newton steps from an estimate give the wrong one."""
+    nx, rho = 6, 0.1
+    x, v, t = product().create_lattice(nx=nx, ny=nx, nz=nx, rho=rho)
+    x = np.round(x.reshape(-1, 3) * 2.0 ** 10) * 2.0 ** -10
+    rng = np.random.default_rng(4)
+    lat = (4 / rho) ** (1 / 3)
+    inner = np.flatnonzero(((x > 2 * lat) & (x < 4 * lat)).all(axis=1))
+    outer = np.flatnonzero(~((x > lat) & (x < 5 * lat)).all(axis=1))
+    targets = [p * (1.0 - m * 2.0 ** -53) for p in (1.0, 2.0) for m in (1, 3, 5, 7, 9, 11, 13)]
+    assert inner.size >= len(targets)
+    for a, b, rsq in zip(inner, outer, targets):
+        d = _pair_at(rsq, rng)
+        x[b] = x[a] + d
+        got = x[a] - x[b]
+        assert got[0] * got[0] + got[1] * got[1] + got[2] * got[2] == rsq
+    sim = product().CPSim(nx=nx, ny=nx, nz=nx, rho=rho, cluster_m=4, cluster_n=N, precision=1, ntimes=0)
+    try:
+        sim.set_atoms(x.reshape(-1), v, t)
+        _, f64, _, _ = _oracle_forces(sim, 4, N, 0, lat, nx)
+        live = _live_slots(sim.get("ci_natoms"), 4)
+        assert np.abs(f64.reshape(-1, 3)[live]).max() > 10.0
+        np.testing.assert_array_equal(sim.get("slot_f").reshape(-1, 3)[live],
+                                      f64.reshape(-1, 3)[live])
+    finally:
+        sim.close()
