@@ -1359,13 +1359,15 @@ __global__ void __launch_bounds__(STAGE_T) k_force_lj_staged(int nlocal, int nal
 // 121 us a call for 35,700 atoms (1.4M pairs), nearly all of it the atomics; this takes
 // 18.5 us and 5.3 for the gather of the accumulators (with the integration).
 // LDS atomics and the latency of the list's loads bound it.  A pair that finds no slot within HALF_PROBE tries adds to memory directly.  acc: zero on entry.
+// fghost: the ghosts' rows of the forces, which are zero (cleared here, beside the lists' loads; as more
+// blocks of k_take_half it cost 0.8 us more at 6912 atoms).
 constexpr int HALF_T = 1024, HALF_PROBE = 8;
 
 template <int LPA, bool EV>
 __global__ void __launch_bounds__(HALF_T) k_force_lj_half(int nlocal, const double* __restrict__ x,
     const int* __restrict__ type, int ntypes, Tables tab, int uniform,
     const int* __restrict__ neighbors, const int* __restrict__ numneigh, double* __restrict__ acc,
-    double* __restrict__ ev)
+    double* __restrict__ ev, int nghost, double* __restrict__ fghost)
 {
     constexpr int A = HALF_T / LPA, LOG = LPA <= 8 ? 11 : 10, SLOTS = 1 << LOG;
     __shared__ double s_tab[3][MAXTYPES2];
@@ -1385,6 +1387,8 @@ __global__ void __launch_bounds__(HALF_T) k_force_lj_half(int nlocal, const doub
         s_f[k] = 0.0;
     for (int k = threadIdx.x; k < 3 * A; k += HALF_T)
         s_own[k] = 0.0;
+    for (int k = blockIdx.x * HALF_T + threadIdx.x; k < 3 * nghost; k += gridDim.x * HALF_T)
+        fghost[k] = 0.0;
     __syncthreads();
     const int i0   = blockIdx.x * A;
     const int i    = i0 + threadIdx.x / LPA;
@@ -2650,7 +2654,8 @@ static double force_lj(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu
 #define MDG_LJH(L, E)                                                                            \
     k_force_lj_half<L, E><<<blocks_for(nlocal, HALF_T / L), HALF_T, 0, s>>>(nlocal,              \
         atom->d_atom.x, atom->d_atom.type, S.ntypes, S.tab, S.uniform ? 1 : 0,                   \
-        neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, S.d_acc, S.d_ev)
+        neighbor->d_neighbor.neighbors, neighbor->d_neighbor.numneigh, S.d_acc, S.d_ev,           \
+        atom->Nghost, atom->d_atom.fx + 3 * (size_t)nlocal)
         if (strict) {
             if (half) {
                 if (S.ev_on) MDG_LJ(1, true, true, true);

@@ -1,5 +1,7 @@
 """GPU paths of the Verlet-list kernels that are chosen by the system's size, against the CPU
 oracle: at the sizes where the choice changes and with remainders."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -391,4 +393,38 @@ def test_atom_outside_the_grid_is_an_error(dims, call):
         np.testing.assert_array_equal(st["neighbors"], nb)
     finally:
         L.mdgfx950ClearStatus()
+        sim.close()
+
+
+def _hip():
+    hip = C.CDLL("libamdhip64.so.7")  # the runtime libmdgfx950.so is linked against
+    hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    return hip
+
+
+@pytest.mark.parametrize("fused", [0, 1])
+@pytest.mark.parametrize("dims", [(4, 4, 4), (15, 14, 16), (29, 27, 27)], ids=str)
+def test_half_list_call_leaves_zero_forces_on_ghosts(dims, fused):
+    """A half-list call gives every atom's row of the device's forces: a ghost's is zero, whatever the
+    buffer held."""
+    P = product()
+    L = P.lib()
+    hip = _hip()
+    print(dims, fused, flush=True)
+    sim = P.VLSim(nx=dims[0], ny=dims[1], nz=dims[2], half_neigh=1, reneigh_every=5)
+    try:
+        nl, ng = sim.atom.Nlocal, sim.atom.Nghost
+        f = np.full(3 * (nl + ng), np.nan)
+        L.mdgfx950Synchronize()
+        fx = C.cast(sim.atom.d_atom.fx, C.c_void_p)
+        assert hip.hipMemcpy(fx, f.ctypes.data, f.nbytes, 1) == 0
+        if fused:
+            L.computeForceFinalInitialGFX950(sim.param_p, sim.atom_p, sim.neighbor_p, sim.stats_p)
+        else:
+            sim.compute_force()
+        L.mdgfx950Synchronize()
+        assert hip.hipMemcpy(f.ctypes.data, fx, f.nbytes, 2) == 0
+        assert ng > 0 and np.isfinite(f[:3 * nl]).all()
+        np.testing.assert_array_equal(f[3 * nl:], 0.0)
+    finally:
         sim.close()
