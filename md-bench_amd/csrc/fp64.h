@@ -19,8 +19,9 @@
  * million differed from the division).  37,044 atoms of a mixture, us a call: division 30.1, this 29.0,
  * recip_normal 28.3; 256,000 atoms of 4x8 clusters 169, 152, 147.
  *
- * A zero argument gives NaN (a pair at distance zero: its force is 0 times infinity, NaN, either way),
- * and so does one whose reciprocal overflows (a distance below 1e-154); callers that need the special
+ * A zero argument's reciprocal is NaN (a pair at distance zero: its force is 0 times infinity, NaN,
+ * either way), its root zero, and an argument whose reciprocal overflows (a distance below 1e-154)
+ * gives NaN too; callers that need the special
  * cases divide, and so do the passes that instructions do not bound: the EAM density pass (264 us with
  * a root from here, 261 without, 1.05 M atoms) and the FP64 cluster pairs' half lists.
  */
@@ -52,7 +53,7 @@ __device__ inline double root_recip_normal(double d, double* r)
     h              = fma(h, e, h);
     g              = fma(fma(-g, g, d), h, g);
     h              = h + h;
-    *r             = g;
+    *r             = fmax(g, 0.0);  // (g is NaN for zero)
     return fma(h, fma(-g, h, 1.0), h);
 }
 
