@@ -50,7 +50,10 @@ struct TimedRegion {
 };
 
 // ---------------------------------------------------------------- buffers
-// Grows a device buffer to at least `bytes` (1.25x headroom); preserves `keep` leading bytes.
+// Grows a device buffer to at least `bytes` (1.25x headroom); preserves `keep` leading bytes.  Where
+// the device has no room, grow first asks for memory that only saves time (the function of
+// set_give_back, which returns whether it freed any).
+void set_give_back(bool (*give_back)());
 bool grow(void** ptr, size_t* cap, size_t bytes, size_t keep);
 template <class T>
 bool grow_n(T** ptr, size_t* cap_elems, size_t n, size_t keep_n)

@@ -124,13 +124,22 @@ TimedRegion::~TimedRegion()
 }
 
 // ---------------------------------------------------------------- buffers
+static bool (*g_give_back)() = nullptr;
+void set_give_back(bool (*give_back)()) { g_give_back = give_back; }
+
 bool grow(void** ptr, size_t* cap, size_t bytes, size_t keep)
 {
     if (failed()) return false;
     if (bytes <= *cap && *ptr) return true;
     size_t nb = bytes + bytes / 4 + 256;
     void* np  = nullptr;
-    if (hipMalloc(&np, nb) != hipSuccess) {
+    hipError_t e = hipMalloc(&np, nb);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // (else the next launch's check would find it)
+        if (g_give_back && g_give_back()) e = hipMalloc(&np, nb);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         set_error(MDG_ERR_CAPACITY, "hipMalloc of %zu bytes failed", nb);
         return false;
     }

@@ -1919,7 +1919,16 @@ void stage_release()
     S.stage_nlocal = -1;
 }
 
-// Room for n elements, or false: a system that fits the device without the tables runs without them.
+// For grow, which has no room left: a system that fits the device without the tables runs without them.
+bool stage_give_back()
+{
+    if (!S.d_stage && !S.d_stage_n && !S.d_hint) return false;
+    MDG_HIP(hipStreamSynchronize(stream()));
+    stage_release();
+    return !failed();
+}
+
+// Room for n elements, or false (no error: see stage_give_back).
 template <typename T>
 bool stage_room(T** p, size_t* cap, size_t n)
 {
@@ -1966,6 +1975,7 @@ void initDeviceGFX950(Parameter* param, Atom* atom, Neighbor* neighbor)
         if (failed()) return;
         S.ncu = (cu + 7) / 8 * 8;
     }
+    set_give_back(stage_give_back);
     DeviceAtom* d   = &atom->d_atom;
     memset(d, 0, sizeof(*d));
     S.cap_all = S.cap_v = 0;
