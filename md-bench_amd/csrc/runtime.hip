@@ -6,8 +6,8 @@
 #include <cstring>
 #include <ctime>
 #include <algorithm>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -223,8 +223,8 @@ static hipError_t bounce(size_t bytes, F fn)
     try {
         for (; started < BOUNCE_T; started++)
             threads[started] = std::thread(work, started);
-    } catch (const std::system_error&) {
-        // no more threads: this one takes the rest's chunks as well
+    } catch (const std::exception&) {
+        // no more threads, or no memory for one: this one takes the rest's chunks as well
     }
     work(0);
     for (int t = started; t < BOUNCE_T; t++)

@@ -37,6 +37,44 @@ int main()
 }
 """
 
+THREADS = """
+#include <cstdio>
+#include <cstdlib>
+#include <new>
+#include <vector>
+namespace mdg {
+void copy_to_device(void*, const void*, size_t);
+void copy_from_device(void*, const void*, size_t);
+}
+static thread_local int g_news = -1;  // allocations of this thread left before one fails (-1: no limit)
+void* operator new(size_t n)
+{
+    if (g_news == 0) throw std::bad_alloc();
+    if (g_news > 0) g_news--;
+    if (void* p = malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
+int main()
+{
+    const size_t n = 17 << 20;  // nine chunks
+    std::vector<unsigned char> a(n), b(n), c(n);
+    for (size_t i = 0; i < n; i++)
+        a[i] = (unsigned char)(i * 2654435761u >> 13);
+    for (int news = 0; news < 4; news++) {
+        g_news = news;
+        mdg::copy_to_device(b.data(), a.data(), n);
+        g_news = news;
+        mdg::copy_from_device(c.data(), b.data(), n);
+        g_news = -1;
+        std::printf("%d\\n", a == b && a == c);
+        b.assign(n, 0);
+        c.assign(n, 0);
+    }
+}
+"""
+
 
 def _run(tmp_path, source):
     (tmp_path / "main.cpp").write_text(source)
@@ -61,3 +99,8 @@ def test_staging_tables_make_room_for_what_a_run_needs(tmp_path):
     assert status == 0  # MDG_ERR_CAPACITY (3) where the tables stay
     assert change < -100e6  # 123 MB of tables for 16 MB of positions
     assert [int(v) for v in second] == [3, 2]
+
+
+def test_host_copies_without_memory_for_threads(tmp_path):
+    """A copy whose threads cannot be started for want of memory is made by the calling thread."""
+    assert _run(tmp_path, THREADS) == [["1"]] * 4
