@@ -118,7 +118,9 @@ struct State {
     double* d_red = nullptr;
     size_t cap_red = 0;
     double* d_ev = nullptr;
-    int* d_status = nullptr;  // [0] flags, [1] max numneigh, [2] scan total, [3] staging overflows
+    // [0] flags, [1] max numneigh, [2] scan total, [3] staging overflows, [4] go (k_ghost_setup),
+    // [ST_OUTSIDE]
+    int* d_status = nullptr;
     int* h_status = nullptr;  // pinned
     int* h_flag   = nullptr;  // pinned, written by kernels (HF_*)
     int xs_ld = 0;            // length of d_xs's three runs
@@ -130,6 +132,10 @@ struct State {
 State S;
 
 enum { ST_BIN_RANGE = 1, ST_NB_OVERFLOW = 2 };
+// Status word set by a binning with an atom outside the grid, zero between calls: whoever reads it set
+// clears it.  (The other flags are cleared between the binning and the list build; with a host word
+// for the binning kernels to set, a list of 32,000 atoms took about 2 us more.)
+constexpr int ST_OUTSIDE = 5;
 
 // ---------------------------------------------------------------- helpers
 __device__ inline int coord2bin(const Grid& g, double x, double y, double z)
@@ -377,19 +383,17 @@ __global__ void k_update_pbc(int nlocal, int nghost, double* __restrict__ x,
 // ---------------------------------------------------------------- binning (neighbor.c:386-464)
 // Each atom's bin and its place among the bin's atoms as they arrive (one atomic per atom: with a
 // second one in the scatter the two took 29 us each at 1M atoms).  An atom outside the grid is in no
-// bin; it sets the status flag, and for a list build (host set) the host's word, which outlasts the
-// clearing of the status words on the way to the lists.
+// bin, and sets *outside where the caller asks for it.
 __global__ void k_bin_count(int nlocal, const int* __restrict__ nghost, const double* __restrict__ x, Grid g, int* __restrict__ bin_of,
-    int* __restrict__ place, int* __restrict__ count, int* __restrict__ status,
-    int* __restrict__ host, const int* __restrict__ go)
+    int* __restrict__ place, int* __restrict__ count, int* __restrict__ outside,
+    const int* __restrict__ go)
 {
     if (go && !*go) return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nlocal + (nghost ? *nghost : 0)) return;
     int b = coord2bin(g, x[3 * i], x[3 * i + 1], x[3 * i + 2]);
     if (b < 0 || b >= g.mbins) {
-        atomicOr(&status[0], ST_BIN_RANGE);
-        if (host) host[HF_RANGE] = 1;
+        if (outside) *outside = 1;
         bin_of[i] = -1;
         return;
     }
@@ -439,7 +443,7 @@ __global__ void k_bin_rank(int n, const int* __restrict__ bin_of, const int* __r
 // k_bin_rank's work.  n: nlocal plus the ghosts counted by k_ghost_setup where nghost is not null.
 // 256 atoms and 1500 ghosts: 15 us in four launches, 7.7 in one.  4000 atoms and 5500 ghosts: 25 us in
 // four launches, 17.5 in two, 24 in one (6 for the ranks and 9 for the writes, which many blocks share
-// better).  host: set for a list build (see k_bin_count), which also has its status words cleared.
+// better).  outside: as for k_bin_count; clear: two status words zeroed for the list build that follows.
 constexpr int BIN1_T = 1024, BIN1_I = 16, BIN1_N = BIN1_T * BIN1_I, BIN1_BINS = 16384;
 constexpr int BIN1_ORDER = 4 * BIN1_T;
 
@@ -447,7 +451,7 @@ template <bool ORDER>
 __global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __restrict__ nghost,
     int ld, const double* __restrict__ x, Grid g, int* __restrict__ binstart,
     int* __restrict__ bin_of, int* __restrict__ slots, int* __restrict__ binatoms,
-    double* __restrict__ xs, int* __restrict__ status, int* __restrict__ host,
+    double* __restrict__ xs, int* __restrict__ outside, int* __restrict__ clear,
     const int* __restrict__ go)
 {
     constexpr int NI = ORDER ? BIN1_ORDER / BIN1_T : BIN1_I;
@@ -476,8 +480,7 @@ __global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __
         if (i >= n) continue;
         const int b = coord2bin(g, r[k & 3][0], r[k & 3][1], r[k & 3][2]);
         if (b < 0 || b >= g.mbins) {
-            if (host) host[HF_RANGE] = 1;
-            else atomicOr(&status[0], ST_BIN_RANGE);
+            if (outside) *outside = 1;
             continue;
         }
         bin[k]   = b;
@@ -501,7 +504,7 @@ __global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __
         binstart[b] = s_bin[b];
     if (tid == 0) {
         binstart[g.mbins] = total;
-        if (host) status[0] = status[1] = 0;
+        if (clear) clear[0] = clear[1] = 0;
     }
 #pragma unroll
     for (int k = 0; k < NI; k++) {
@@ -527,16 +530,16 @@ __global__ void __launch_bounds__(BIN1_T) k_bin_single(int nlocal, const int* __
 }
 
 // Launches the binning of up to BIN1_N atoms (nlocal and *nghost), max_n at most, in few launches.
-void launch_bins_small(int nlocal, const int* nghost, int max_n, const double* x, int* host,
-    const int* go)
+void launch_bins_small(int nlocal, const int* nghost, int max_n, const double* x, int* outside,
+    int* clear, const int* go)
 {
     hipStream_t s = stream();
     if (max_n <= BIN1_ORDER) {
         k_bin_single<true><<<1, BIN1_T, 0, s>>>(nlocal, nghost, S.xs_ld, x, S.g, S.d_binstart,
-            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, S.d_status, host, go);
+            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, outside, clear, go);
     } else {
         k_bin_single<false><<<1, BIN1_T, 0, s>>>(nlocal, nghost, S.xs_ld, x, S.g, S.d_binstart,
-            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, S.d_status, host, go);
+            S.d_bin_of, S.d_binslots, S.d_binatoms, S.d_xs, outside, clear, go);
         k_bin_rank<<<blocks_for(max_n, BLOCK), BLOCK, 0, s>>>(S.xs_ld, S.d_bin_of, S.d_binstart,
             S.d_binslots, x, S.d_binatoms, S.d_xs, S.d_binstart + S.g.mbins, nullptr, go);
     }
@@ -596,6 +599,7 @@ __global__ void __launch_bounds__(NB_T) k_build_neighbor(int nlocal, int ld, con
     const double* zs = ys + ld;
     const int b      = blockIdx.x;
     if (b >= mbins || (go && !*go)) return;
+    if (b == 0 && threadIdx.x == 0 && status[ST_OUTSIDE]) host[HF_RANGE] = 1;
     const int beg = binstart[b], end = binstart[b + 1];
     // index order inside a bin: its local atoms come first
     if (beg >= end || binatoms[beg] >= nlocal) return;
@@ -2248,32 +2252,34 @@ static void grow_bins(size_t n)
     if (S.cap_bins != cap0) fill_i32(S.d_bincount, 0, S.cap_bins);
 }
 
-// Launches the binning of nlocal and *nghost atoms (null: none), max_n at most.  for_lists: the list
-// build follows; its status words are cleared on the way, and an atom outside the grid is reported by
-// lists_done (without it, by status word 0).
-static void launch_bins(int nlocal, const int* nghost, int max_n, const double* x, bool for_lists,
+// What a binning is for: lists (their status words are cleared on the way, and lists_done reports an
+// atom outside the grid), the sort (which reports one), or the caller's own use.
+enum BinFor { BIN_CALLER, BIN_SORT, BIN_LISTS };
+
+// Launches the binning of nlocal and *nghost atoms (null: none), max_n at most.
+static void launch_bins(int nlocal, const int* nghost, int max_n, const double* x, BinFor use,
     const int* go)
 {
     const int mb = S.g.mbins;
-    int* host    = for_lists ? S.h_flag : nullptr;
-    if (for_lists) S.h_flag[HF_RANGE] = 0;  // (the host has waited for the last build that writes it)
+    int* outside = use == BIN_CALLER ? nullptr : S.d_status + ST_OUTSIDE;
+    int* clear   = use == BIN_LISTS ? S.d_status : nullptr;
     if (max_n <= BIN1_N && mb <= BIN1_BINS) {
-        launch_bins_small(nlocal, nghost, max_n, x, host, go);
+        launch_bins_small(nlocal, nghost, max_n, x, outside, clear, go);
         return;
     }
     hipStream_t s       = stream();
     const unsigned grid = blocks_for(max_n, BLOCK);
     k_bin_count<<<grid, BLOCK, 0, s>>>(nlocal, nghost, x, S.g, S.d_bin_of, S.d_binplace,
-        S.d_bincount, S.d_status, host, go);
+        S.d_bincount, outside, go);
     exclusive_scan_take(S.d_bincount, S.d_binstart, mb, S.d_binstart + mb);
     k_bin_scatter<<<grid, BLOCK, 0, s>>>(nlocal, nghost, S.d_bin_of, S.d_binplace, S.d_binstart,
         S.d_binslots, go);
     k_bin_rank<<<grid, BLOCK, 0, s>>>(S.xs_ld, S.d_bin_of, S.d_binstart, S.d_binslots, x,
-        S.d_binatoms, S.d_xs, S.d_binstart + mb, for_lists ? S.d_status : nullptr, go);
+        S.d_binatoms, S.d_xs, S.d_binstart + mb, clear, go);
     MDG_LAUNCH_CHECK("binatoms");
 }
 
-static void bin_atoms(Atom* atom, bool for_lists)
+static void bin_atoms(Atom* atom, BinFor use)
 {
     if (failed() || !S.ready || S.g.mbins == 0) {
         if (!failed()) set_error(MDG_ERR_ARG, "binatomsGFX950 before setupNeighborGFX950");
@@ -2285,10 +2291,10 @@ static void bin_atoms(Atom* atom, bool for_lists)
     if (failed()) return;
     S.xs_ld  = nall;
     S.binned = true;
-    launch_bins(nall, nullptr, nall, atom->d_atom.x, for_lists, nullptr);
+    launch_bins(nall, nullptr, nall, atom->d_atom.x, use, nullptr);
 }
 
-void binatomsGFX950(Atom* atom) { bin_atoms(atom, false); }
+void binatomsGFX950(Atom* atom) { bin_atoms(atom, BIN_CALLER); }
 
 void sortAtomGFX950(Atom* atom)
 {
@@ -2300,12 +2306,12 @@ void sortAtomGFX950(Atom* atom)
     S.gmap_nlocal    = -1;
     S.ghosts_current = false;
     if (n <= 0) return;
-    fill_i32(S.d_status, 0, 2);
-    binatomsGFX950(atom);
+    bin_atoms(atom, BIN_SORT);
     if (failed()) return;
     read_status();
     if (failed()) return;
-    if (S.h_status[0] & ST_BIN_RANGE) {
+    if (S.h_status[ST_OUTSIDE]) {
+        fill_i32(S.d_status + ST_OUTSIDE, 0, 1);
         set_error(MDG_ERR_BIN, "sortAtomGFX950: an atom lies outside the bin grid");
         return;
     }
@@ -2382,7 +2388,7 @@ static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
         S.nstencil, neighbor->half_neigh, neighbor->maxneighs, neighbor->d_neighbor.neighbors,   \
         neighbor->d_neighbor.numneigh, __VA_ARGS__)
     if (nlocal <= NB_SMALL) {
-        S.h_flag[HF_OVERFLOW] = 0;  // (no earlier list build is running)
+        S.h_flag[HF_OVERFLOW] = S.h_flag[HF_RANGE] = 0;  // (no earlier list build is running)
         MDG_NB(k_build_neighbor, S.g.mbins, NB_T, S.d_status, S.h_flag, go);
     } else {
         MDG_NB(k_build_neighbor_wave, blocks_for(S.g.mbins, BLOCK / 64), BLOCK, S.d_status, go);
@@ -2399,16 +2405,17 @@ static bool lists_done(int nlocal, Neighbor* neighbor, bool waited = false)
     if (nlocal <= NB_SMALL) {
         if (!waited) MDG_HIP(hipStreamSynchronize(stream()));
         if (failed()) return true;
-        range    = false;
+        range    = S.h_flag[HF_RANGE] != 0;
         overflow = S.h_flag[HF_OVERFLOW] != 0;
         if (overflow) read_status();  // the longest list
     } else {
         if (!waited) read_status();
-        range    = (S.h_status[0] & ST_BIN_RANGE) != 0;
+        range    = (S.h_status[0] & ST_BIN_RANGE) != 0 || S.h_status[ST_OUTSIDE] != 0;
         overflow = (S.h_status[0] & ST_NB_OVERFLOW) != 0;
     }
     if (failed()) return true;
-    if (range || S.h_flag[HF_RANGE]) {
+    if (range) {
+        fill_i32(S.d_status + ST_OUTSIDE, 0, 1);
         set_error(MDG_ERR_BIN, "an atom lies outside the bin grid (coord2bin out of range)");
         return true;
     }
@@ -2426,7 +2433,7 @@ static bool lists_done(int nlocal, Neighbor* neighbor, bool waited = false)
 void buildNeighborGFX950(Atom* atom, Neighbor* neighbor)
 {
     if (failed() || !S.ready) return;
-    bin_atoms(atom, true);
+    bin_atoms(atom, BIN_LISTS);
     for (int attempt = 0; attempt < 8; attempt++) {
         if (failed()) return;
         launch_lists(atom, neighbor, nullptr);
@@ -2548,7 +2555,7 @@ void mdg_vl_reneighbour(Parameter* param, Atom* atom, Neighbor* neighbor)
     }
     {
         TimedRegion tr(F_BINNING);
-        launch_bins(nlocal, S.d_status + 2, (int)ld, d->x, true, go);
+        launch_bins(nlocal, S.d_status + 2, (int)ld, d->x, BIN_LISTS, go);
     }
     if (failed()) return;
     launch_lists(atom, neighbor, go);
