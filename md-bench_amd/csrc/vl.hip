@@ -582,6 +582,7 @@ __global__ void k_sort_gather(int n, const int* __restrict__ order, const double
 // 32000 atoms on 50 us against 56, and 794 against 1650 us at 1M).
 constexpr int NB_T = 256, NB_SEG = 1024, NB_Q = 32;
 constexpr int NB_SMALL = 24000;  // atoms up to which the block kernel builds the lists
+constexpr int NB_BINS  = 16384;  // and bins (see small_lists)
 
 __global__ void __launch_bounds__(NB_T) k_build_neighbor(int nlocal, int ld, const double* __restrict__ xs,
     const int* __restrict__ type, int ntypes, Tables tab, int uniform, double cnmax, int mbins,
@@ -2369,6 +2370,21 @@ static void stage_build(int nlocal, Neighbor* neighbor)
     S.stage_max    = mn;
 }
 
+// Whether the block kernel builds the lists: for few atoms, and few bins, since it spends a block on
+// each bin, empty ones too.  Boxes read from a file have bins of half the list cutoff, and may be mostly
+// empty.  us per list (kernel), a block and a wavefront per bin:
+//     atoms    bins
+//       256   17576   11.7   14.4
+//       256   64000   22.4   14.9
+//      2048   17576   14.9   16.2
+//      2048   29791   21.4   19.8
+//      6912   10648   21.6   31.2
+//      6912   17576   28.1   22.5
+//     16384   15625   33.9   41.7
+//     16384   29791   63.5   33.1
+//     16384  328509   125    37
+static bool small_lists(int nlocal) { return nlocal <= NB_SMALL && S.g.mbins <= NB_BINS; }
+
 // Launches the list build over the bins; go: see k_ghost_setup.
 static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
 {
@@ -2387,7 +2403,7 @@ static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
         S.uniform ? 1 : 0, cnmax, S.g.mbins, S.d_binstart, S.d_binatoms, S.d_stencil,            \
         S.nstencil, neighbor->half_neigh, neighbor->maxneighs, neighbor->d_neighbor.neighbors,   \
         neighbor->d_neighbor.numneigh, __VA_ARGS__)
-    if (nlocal <= NB_SMALL) {
+    if (small_lists(nlocal)) {
         S.h_flag[HF_OVERFLOW] = S.h_flag[HF_RANGE] = 0;  // (no earlier list build is running)
         MDG_NB(k_build_neighbor, S.g.mbins, NB_T, S.d_status, S.h_flag, go);
     } else {
@@ -2402,7 +2418,7 @@ static void launch_lists(Atom* atom, Neighbor* neighbor, const int* go)
 static bool lists_done(int nlocal, Neighbor* neighbor, bool waited = false)
 {
     bool range, overflow;
-    if (nlocal <= NB_SMALL) {
+    if (small_lists(nlocal)) {
         if (!waited) MDG_HIP(hipStreamSynchronize(stream()));
         if (failed()) return true;
         range    = S.h_flag[HF_RANGE] != 0;
@@ -2560,7 +2576,7 @@ void mdg_vl_reneighbour(Parameter* param, Atom* atom, Neighbor* neighbor)
     if (failed()) return;
     launch_lists(atom, neighbor, go);
     if (failed()) return;
-    const bool flags = nlocal <= NB_SMALL;  // (lists_done's two ways)
+    const bool flags = small_lists(nlocal);  // (lists_done's two ways)
     if (small && flags) MDG_HIP(hipStreamSynchronize(s));
     else read_status();
     if (failed()) return;

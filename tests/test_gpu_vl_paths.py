@@ -428,3 +428,43 @@ def test_half_list_call_leaves_zero_forces_on_ghosts(dims, fused):
         np.testing.assert_array_equal(f[3 * nl:], 0.0)
     finally:
         sim.close()
+
+
+@pytest.mark.parametrize("half", [0, 1])
+@pytest.mark.parametrize("nx,wide", [(6, 1.0), (8, 1.5), (8, 4.0), (20, 1.0)])
+def test_lists_in_boxes_of_many_bins(nx, wide, half, tmp_path):
+    """Boxes read from a file (bins of half the list cutoff, none to a few atoms each), and a droplet in
+    a box whose bins are mostly empty, around the number of bins where the list build changes: the
+    lists name the pairs inside the cutoff, at setup and after a run's rebuild."""
+    from scipy.spatial import cKDTree
+    P = product()
+    print(nx, wide, half, flush=True)
+    x, v, t = P.create_lattice(nx=nx, ny=nx, nz=nx)
+    side = nx * (4 / 0.8442) ** (1 / 3) * wide
+    rng = np.random.default_rng(nx)
+    x = np.mod(x + rng.uniform(-0.2, 0.2, x.size) + side / 3, side)
+    path = str(tmp_path / "a.dmp")
+    P.write_dmp(path, x, 0.01 * v, t, [0.0, side] * 3)
+    sim = P.VLSim(input_file=path, half_neigh=half, reneigh_every=2, dt=1e-5)
+    try:
+        bins = sim.bins()[0].size - 1
+        assert (bins > 16384) == ((nx, wide) != (6, 1.0))
+        for steps in (0, 2):
+            if steps:
+                sim.run(steps)
+            st = sim.state()
+            pos = st["x"].reshape(-1, 3)
+            nl = st["nlocal"]
+            _ghosts_follow_owners(sim, st)
+            cn = sim.param.cutneigh ** 2
+            near = cKDTree(pos[:nl]).query_ball_tree(cKDTree(pos), sim.param.cutneigh * (1 + 1e-9))
+            i = np.repeat(np.arange(nl), [len(q) for q in near])
+            j = np.concatenate([np.asarray(q, np.int64) for q in near])
+            d = pos[i] - pos[j]
+            rsq = d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1] + d[:, 2] * d[:, 2]
+            keep = (i != j) & (rsq <= cn) & ((j > i) if half else True)
+            want = np.sort(i[keep] * (1 << 32) + j[keep])
+            got = np.repeat(np.arange(nl), st["numneigh"]) * (1 << 32) + st["neighbors"]
+            np.testing.assert_array_equal(np.sort(got), want)
+    finally:
+        sim.close()
