@@ -753,7 +753,11 @@ __global__ void __launch_bounds__(NB_T) k_build_neighbor(int nlocal, int ld, con
 // 120 us for 131,000.  The tests' vector instructions (1640 per bin, 400 us) and the texture
 // path's work (the scattered list stores and the candidates' loads, 600 us busy) bound it; bins
 // of one XCD adjacent made it slower (895 us: slabs of ghost bins leave an XCD idle).
-constexpr int NBW_SEG = 1024;
+// Up to NB_FEW local atoms (bins of half the list cutoff, in boxes read from a file) are tested against
+// every candidate at once: choosing the near ones costs as much as those tests.  us per list with 2, 3,
+// 4 and 5 (without: 1319; the kernel before: 1205) for 1.05 M atoms in such bins 1255, 1263, 1223, 1216, for
+// 131,000 136, 137, 134, 135 (141; 128); bins of seven atoms unchanged.
+constexpr int NBW_SEG = 1024, NB_FEW = 4;
 struct NbLocal {
     double x, y, z;
     int id, type;
@@ -836,9 +840,9 @@ __global__ void __launch_bounds__(BLOCK) k_build_neighbor_wave(int nlocal, int l
                     s_m[t - g0] = lo + (t - pre);
                 wave_fence();
                 // the candidates near the box stay, in order (a batch is read before its places,
-                // at or below it, are written)
-                int nc = 0;
-                for (int t0 = 0; t0 < segn; t0 += 64) {
+                // at or below it, are written); all of them for few local atoms
+                int nc = nq <= NB_FEW ? segn : 0;
+                for (int t0 = nc; t0 < segn; t0 += 64) {
                     bool near = false;
                     int m     = 0;
                     if (t0 + lane < segn) {
