@@ -2790,6 +2790,21 @@ static int eam_lanes(int nlocal, bool tab)
                                       : FAST_LPA;
 }
 
+// The same for the passes with energies, whose blocks each end with atomics on the same words: fewer
+// lanes are fewer blocks.  us per call (both passes, 75 listed neighbours) with
+//     atoms     4     8    16    32 lanes
+//       256  28.4  19.7  14.9  13.2
+//       864  30.5  20.1  15.5  15.3
+//      2048  29.9  20.1  18.0  20.5
+//      4000  30.8  22.3  22.4  30.3
+//     10976  33.0  30.5  40.4  69.8
+//     19652  39.8  44.3  65.0   108
+//     32000  50.7  63.9   102   169
+static int eam_energy_lanes(int nlocal)
+{
+    return nlocal <= 1000 ? 32 : nlocal <= 3000 ? 16 : nlocal <= 10000 ? 8 : FAST_LPA;
+}
+
 static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse fu)
 {
     if (failed() || !S.ready) return 0.0;
@@ -2855,8 +2870,10 @@ static double force_eam(Parameter* param, Atom* atom, Neighbor* neighbor, Fuse f
         else if (tab) MDG_EAM_TAB(1, true);
         else MDG_EAM(1, true, false);
     } else if (ev) {
-        if (lanes >= 32) MDG_EAM(32, false, true);
-        else if (lanes >= 8) MDG_EAM(16, false, true);
+        const int el = eam_energy_lanes(nlocal);
+        if (el == 32) MDG_EAM(32, false, true);
+        else if (el == 16) MDG_EAM(16, false, true);
+        else if (el == 8) MDG_EAM(8, false, true);
         else MDG_EAM(FAST_LPA, false, true);
     } else if (lanes == 64) {
         MDG_EAM(64, false, false);

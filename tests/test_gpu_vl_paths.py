@@ -468,3 +468,33 @@ def test_lists_in_boxes_of_many_bins(nx, wide, half, tmp_path):
             np.testing.assert_array_equal(np.sort(got), want)
     finally:
         sim.close()
+
+
+@pytest.mark.parametrize("dims", [(6, 6, 6), (7, 6, 6), (9, 9, 9), (13, 13, 14), (14, 14, 14)], ids=str)
+def test_eam_energies_at_each_lane_count(dims, tmp_path):
+    """32, 16, 16, 8 and 4 lanes per atom in the passes with energies."""
+    P = product()
+    L = P.lib()
+    print(dims, flush=True)
+    path = str(tmp_path / "cu.eam")
+    L.mdbWriteFuncflSynthetic(path.encode())
+    tab = ob.EamTables(path)
+    sim = P.VLSim(nx=dims[0], ny=dims[1], nz=dims[2], force_field=1, lattice_a=3.615, temp=1600.0,
+                  maxwell_seed=5, reneigh_every=5, eam_file=path)
+    try:
+        sim.run(13)
+        st = sim.state()
+        want, ea = ob.force_eam_atom(tab, st["nlocal"], st["x"], st["border_map"],
+                                     sim.param.cutforce ** 2, st["numneigh"], st["neighbors"])
+        want = want[:3 * st["nlocal"]]
+        L.requestEnergyVirialGFX950(1)
+        e = sim.eam_atom_energy()
+        total, _ = sim.energy_virial()
+        L.requestEnergyVirialGFX950(0)
+        assert np.linalg.norm(e - ea) < FORCE_RTOL * np.linalg.norm(ea)
+        assert abs(total - ea.sum()) < 1e-11 * abs(ea.sum())
+        assert np.linalg.norm(sim.state(lists=False)["f"] - want) < \
+            FORCE_RTOL * np.linalg.norm(want)
+    finally:
+        L.requestEnergyVirialGFX950(0)
+        sim.close()
