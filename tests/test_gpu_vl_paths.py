@@ -498,3 +498,49 @@ def test_eam_energies_at_each_lane_count(dims, tmp_path):
     finally:
         L.requestEnergyVirialGFX950(0)
         sim.close()
+
+
+def test_foreign_list_under_staging_tables():
+    """A list uploaded over one that was built with staging tables (same size, so the tables stay): its
+    entries in another order, some dropped, some rows emptied or made of far atoms; the forces are
+    that list's."""
+    P = product()
+    L = P.lib()
+    sim = P.VLSim(nx=51, ny=51, nz=51, reneigh_every=1000)
+    nb = sim.neighbor
+    host = (nb.neighbors, nb.numneigh)
+    try:
+        sim.run(2)
+        st = sim.state()
+        nl, mn = st["nlocal"], nb.maxneighs
+        assert nl == 530604  # above the size from which the lists have tables
+        start = np.concatenate([[0], np.cumsum(st["numneigh"], dtype=np.int64)])
+        row = np.repeat(np.arange(nl), st["numneigh"])
+        k = np.arange(row.size) - start[row]
+        keep = (k % 7 != 3) & (row % 1000 != 5)
+        count = np.bincount(row[keep], minlength=nl).astype(np.int32)
+        at = np.arange(keep.sum()) - np.concatenate([[0], np.cumsum(count, dtype=np.int64)])[row[keep]]
+        lists = np.zeros((nl, mn), np.int32)
+        # backwards, so that every entry is in another place
+        lists[row[keep], count[row[keep]] - 1 - at] = st["neighbors"][keep]
+        for i in range(9, nl, 5000):
+            count[i] = min(mn, 40)
+            lists[i, :count[i]] = (i + 7919 * np.arange(1, count[i] + 1)) % nl
+        csr = lists[np.arange(mn) < count[:, None]]
+        nb.neighbors = lists.ctypes.data_as(C.POINTER(C.c_int))
+        nb.numneigh = count.ctypes.data_as(C.POINTER(C.c_int))
+        L.uploadNeighborGFX950.argtypes = [C.c_void_p, C.c_void_p]
+        L.uploadNeighborGFX950(sim.atom_p, sim.neighbor_p)
+        assert nb.maxneighs == mn
+        sim.compute_force()
+        one = np.ones(16)
+        want, _, _ = ob.force_lj(nl, st["x"], np.zeros(nl + st["nghost"], np.int32), 4, one, one,
+                                 one * 6.25, count, csr, 0)
+        want = want[:3 * nl]
+        got = sim.state(lists=False)["f"]
+        assert np.linalg.norm(want) > 10.0
+        assert np.linalg.norm(got - want) < FORCE_RTOL * np.linalg.norm(want)
+        np.testing.assert_array_equal(got.reshape(-1, 3)[5::1000][count[5::1000] == 0], 0.0)
+    finally:
+        nb.neighbors, nb.numneigh = host
+        sim.close()
