@@ -13,7 +13,7 @@
 //                           bit-identical to it; the run loop's kicks and drift fused in.
 //   k_cp_force_f64_half     FP64, half lists of i-clusters of four: the same lanes, a j-atom's forces
 //                           summed over them before its atomics.
-//   k_cp_force_f64          the same arithmetic, one thread per i-slot: 1x2 clusters.
+//   k_cp_force_f64          the same arithmetic, one thread per i-atom: 1x2 clusters.
 //   k_cp_force_f32_full     FP32-mixed, full lists: one wavefront per four i-clusters, one
 //                           j-atom per lane against the group's four i-atoms, j-atoms read as
 //                           16-byte FP32 records (offset in a power-of-two grid cell, cell bytes
@@ -1336,21 +1336,22 @@ __global__ void __launch_bounds__(EVR_T) k_cp_sum_ev(size_t nw, const double* __
 }
 
 // ---------------------------------------------------------------- FP64 force, reference arithmetic
-template <int M, int N, bool HALF, bool EV>
+// 1x2 clusters: a thread per i-atom walks its list.
+template <bool HALF, bool EV>
 __global__ void __launch_bounds__(BLOCK) k_cp_force_f64(int nci, int ncj, int ntypes, int uniform,
     Tab64 tab, const double* __restrict__ sx, const int* __restrict__ st,
     const int* __restrict__ nb, const int* __restrict__ numneigh, int maxneighs,
     double* __restrict__ f, double* __restrict__ ev)
 {
-    const int si = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ci = si / M;
+    constexpr int N = 2;
+    const int si    = blockIdx.x * blockDim.x + threadIdx.x;
     double e = 0.0, w = 0.0;
-    if (ci < nci) {
-        const int ci_cj0 = (M == N) ? ci : ci >> 1;
+    if (si < nci) {
+        const int ci_cj0 = si >> 1;
         const double xt = sx[3 * si], yt = sx[3 * si + 1], zt = sx[3 * si + 2];
         const int ti    = st[si];
-        const int* lst  = nb + (size_t)ci * maxneighs;
-        const int nn    = numneigh[ci];
+        const int* lst  = nb + (size_t)si * maxneighs;
+        const int nn    = numneigh[si];
         double fx = 0.0, fy = 0.0, fz = 0.0;
         for (int k = 0; k < nn; k++) {
             const int cj = lst[k];
@@ -1403,7 +1404,7 @@ __global__ void __launch_bounds__(BLOCK) k_cp_force_f64(int nci, int ncj, int nt
 // Half lists of i-clusters of four: one wavefront per i-cluster, lane (e, a) takes i-atom a and entry e
 // of a round of 16.  A j-atom's four pair forces are added over the lanes of its i-atoms first, so
 // that one atomic per coordinate goes to memory instead of four; the i-forces are summed over the
-// entries.  One thread per i-slot walking its list (k_cp_force_f64, still the 1x2 clusters' kernel)
+// entries.  One thread per i-slot walking its list (as k_cp_force_f64 does for 1x2 clusters)
 // took 438 us a step for 98,000 atoms of 4x4 clusters, this 103 (864 atoms 150 and 17; 4x8 clusters 468
 // and 131).  Bound: FP64 atomics and the registers' 4 - 6 wavefronts per SIMD.
 template <int N, bool EV, bool UNIFORM>
@@ -1514,11 +1515,11 @@ struct GhostOut {
 // of a round run side by side; their sums go to LDS and 12 lanes (atom and axis) add them in list
 // order.  The tail kicks and drifts like k_cp_final and k_cp_initial (v set, xn set), each on the
 // lane that holds the total.
-// One thread per i-slot walking its whole list (k_cp_force_f64, still the half lists' and the
-// 1x2 clusters' kernel) took 148 us for 34,960 atoms of the Kob-Andersen mixture, 547 wavefronts
-// waiting on their lists; this takes 24.6 us, kicks and drift included (9.9 us in launches of
-// their own before).  Bound: FP64 instructions.  With energies the pairs divide, without them they take
-// the correctly rounded reciprocal (recip_rounded), the same value.
+// One thread per i-slot walking its whole list (as k_cp_force_f64 does for 1x2 clusters) took 148 us
+// for 34,960 atoms of the Kob-Andersen mixture, 547 wavefronts waiting on their lists; this takes
+// 24 us, kicks and drift included (9.9 us in launches of their own before).  Bound: FP64
+// instructions.  With energies the pairs divide, without them they take the correctly rounded
+// reciprocal (recip_rounded), the same value.
 template <int N, bool EV, bool UNIFORM>
 __global__ void __launch_bounds__(BLOCK) k_cp_force_f64_full(int nci, int ntypes, Tab64 tab,
     const double* __restrict__ sx, const int* __restrict__ st, const int* __restrict__ nb,
@@ -3870,8 +3871,8 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
             else MDG_F64C(NN, false, false);                                                     \
         }                                                                                        \
     } while (0)
-#define MDG_F64(MM, NN, H, E)                                                                    \
-    k_cp_force_f64<MM, NN, H, E><<<grid, BLOCK, 0, s>>>(nci, C.ncj, C.ntypes, uni, C.t64, C.d_sx, \
+#define MDG_F64(H, E)                                                                            \
+    k_cp_force_f64<H, E><<<grid, BLOCK, 0, s>>>(nci, C.ncj, C.ntypes, uni, C.t64, C.d_sx, \
         C.d_st, C.d_nb, C.d_numneigh, C.maxneighs, C.d_sf64, evp)
 #define MDG_F64H(NN, E, U)                                                                       \
     k_cp_force_f64_half<NN, E, U><<<grid, BLOCK, 0, s>>>(nci, C.ncj, C.ntypes, C.t64, C.d_sx,      \
@@ -3891,10 +3892,10 @@ static int force_cluster(Parameter* param, Neighbor* neighbor, bool fuse_final,
             else MDG_F64C_N(8);
         } else if (C.M == 4 && C.N == 4) MDG_F64H_N(4);
         else if (C.M == 4) MDG_F64H_N(8);
-        else if (half && C.ev_on) MDG_F64(1, 2, true, true);
-        else if (half) MDG_F64(1, 2, true, false);
-        else if (C.ev_on) MDG_F64(1, 2, false, true);
-        else MDG_F64(1, 2, false, false);
+        else if (half && C.ev_on) MDG_F64(true, true);
+        else if (half) MDG_F64(true, false);
+        else if (C.ev_on) MDG_F64(false, true);
+        else MDG_F64(false, false);
 #undef MDG_F64C_N
 #undef MDG_F64C
 #undef MDG_F64H_N

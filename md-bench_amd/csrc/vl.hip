@@ -1047,13 +1047,16 @@ struct GatherRow {  // row j of four doubles
 };
 
 // ---------------------------------------------------------------- LJ (force_lj.c:17-206)
-// One atom per LPA lanes.  STRICT: LPA == 1, reference order, no fma.
+// One atom per LPA lanes.  STRICT: LPA == 1, reference order, no fma; HALF: strict half lists (the
+// fast ones are k_force_lj_half's).
 template <int LPA, bool STRICT, bool HALF, bool EV>
 __global__ void __launch_bounds__(BLOCK) k_force_lj(int nlocal, const double* __restrict__ x,
     const int* __restrict__ type, int ntypes, Tables tab, int uniform,
     const int* __restrict__ neighbors, const int* __restrict__ numneigh, double* __restrict__ f,
     double* __restrict__ ev, Fuse fu)
 {
+    static_assert(!STRICT || LPA == 1, "the strict kernels sum in list order");
+    static_assert(!HALF || STRICT, "fast half lists have a kernel of their own");
     __shared__ double s_tab[3][MAXTYPES2];
     __shared__ double s_red[16];
     if (!uniform) {
