@@ -78,9 +78,10 @@ void updateSingleAtomsGFX950(Parameter* param, Atom* atom);
    neighbor->half_neigh, precision by setClusterPrecisionGFX950 */
 double computeForceLJClusterGFX950(Parameter* param, Atom* atom, Neighbor* neighbor, Stats* stats);
 /* computeForce then finalIntegrate (main.c:349-350) in one call: the full-list kernels (FP32, and
-   FP64 with i-clusters of four) and the FP32 tiled half-list one apply the final velocity kick to each atom whose total force it has just written (one pass
-   fewer over v and f); other configurations run the two calls in order (no reference
-   counterpart: a fused form of the two reference calls) */
+   FP64 with i-clusters of four) and the FP32 tiled half-list one apply the final velocity kick to
+   each atom whose total force they have just written (one pass fewer over v and f); other
+   configurations run the two calls in order (no reference counterpart: a fused form of the two
+   reference calls) */
 double computeForceFinalClusterGFX950(Parameter* param, Atom* atom, Neighbor* neighbor,
     Stats* stats);
 /* computeForce, finalIntegrate and the NEXT step's initialIntegrate (main.c:349-350, 326) in one
@@ -89,10 +90,10 @@ double computeForceFinalClusterGFX950(Parameter* param, Atom* atom, Neighbor* ne
    operations in the same order as the three calls, so the trajectory is bit-identical.  The
    velocities it leaves are the next half step's: callers that read full-step velocities after a
    step (thermo, the last step) use computeForceFinalClusterGFX950 there.  Ghost slots keep
-   positions one step older than after the separate calls until updatePbcClusterGFX950, so a
-   pruneNeighborClusterGFX950 between the two differs; callers that prune there use the separate
-   calls for the step before.  Other configurations
-   run the calls in order (no reference counterpart: a fused form of three reference calls) */
+   positions one step older than after the separate calls until updatePbcClusterGFX950, or already
+   follow their owners (full lists of up to 12,000 i-clusters, whose kernels write the ghosts too),
+   so a pruneNeighborClusterGFX950 between the two differs; callers that prune there use the
+   separate calls for the step before.  Other configurations run the calls in order (no reference counterpart: a fused form of three reference calls) */
 double computeForceFinalInitialClusterGFX950(Parameter* param, Atom* atom, Neighbor* neighbor,
     Stats* stats);
 /* replace cudaInitialIntegrate / cudaFinalIntegrate (force_lj_cuda.cu:456-542; this one uses

@@ -1370,7 +1370,8 @@ __global__ void __launch_bounds__(STAGE_T) k_force_lj_staged(int nlocal, int nal
 // adds each touched atom to memory once.  One FP64 atomic per pair and axis to memory instead took
 // 121 us a call for 35,700 atoms (1.4M pairs), nearly all of it the atomics; this takes
 // 18.5 us and 5.3 for the gather of the accumulators (with the integration).
-// LDS atomics and the latency of the list's loads bound it.  A pair that finds no slot within HALF_PROBE tries adds to memory directly.  acc: zero on entry.
+// LDS atomics and the latency of the list's loads bound it.  A pair that finds no slot within
+// HALF_PROBE tries adds to memory directly.  acc: zero on entry.
 // fghost: the ghosts' rows of the forces, which are zero (cleared here, beside the lists' loads; as more
 // blocks of k_take_half it cost 0.8 us more at 6912 atoms).
 constexpr int HALF_T = 1024, HALF_PROBE = 8;
